@@ -301,9 +301,11 @@ __device__ inline chunk_fold fold_chunk(const double* nrm, uint32_t chunk, uint3
   return f;
 }
 
+// wave_out (may be null): the 16 wave sums of every chunk as well, for k_find_events.
 template <typename R>
 __global__ __launch_bounds__(SAMPLE_THREADS) void k_chunk_sums(const cpx<R>* __restrict__ a, uint32_t chunk,
-                                                              double* __restrict__ sums) {
+                                                              double* __restrict__ sums,
+                                                              double* __restrict__ wave_out) {
   __shared__ double nrm[SAMPLE_CHUNK];
   __shared__ double wave_sums[SAMPLE_WAVES];
   const uint32_t per = chunk >= SAMPLE_THREADS ? chunk / SAMPLE_THREADS : 1;
@@ -311,6 +313,109 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void k_chunk_sums(const cpx<R>* __r
   __syncthreads();
   const chunk_fold f = fold_chunk(nrm, chunk, per, wave_sums);
   if (threadIdx.x == 0) sums[blockIdx.x] = f.total;
+  if (wave_out && threadIdx.x < SAMPLE_WAVES)
+    wave_out[(uint64_t)blockIdx.x * SAMPLE_WAVES + threadIdx.x] = wave_sums[threadIdx.x];
+}
+
+// One wavefront per event, from the running sums S over whole chunks and the wave sums of
+// every chunk.  The lanes find the event's chunk together (each step samples 64 points of S:
+// 3 steps instead of the 14 of a binary search over 2^14 chunks), the wave of the chunk from
+// its 16 sums, and only that wave's amplitudes -- 8 per lane, 8 KiB for c128 -- are read: the
+// block that searched a chunk per event read and folded all 128 KiB of it.  C is monotone, so
+// the first index that exceeds the target lies in the first wave whose last C does, and C is
+// formed with the additions of fold_chunk: the same events bit for bit.  Bound: latency of the
+// fold's 64 dependent additions, hidden by the other events' waves; 100 000 events of a 2 GiB
+// c128 state take 0.37 ms (0.82 GB read; the search of whole chunks took 6.5 ms).
+constexpr int FIND_THREADS = 256;
+
+template <typename R>
+__global__ __launch_bounds__(FIND_THREADS) void k_find_events(const cpx<R>* __restrict__ a, uint32_t chunk,
+                                                             const double* __restrict__ S, uint64_t nchunks,
+                                                             double total, uint64_t last_chunk,
+                                                             const double* __restrict__ chunk_waves,
+                                                             const double* __restrict__ canonical,
+                                                             unsigned num_events, uint64_t* __restrict__ events) {
+  const unsigned e = blockIdx.x * (FIND_THREADS / 64) + (threadIdx.x >> 6);
+  if (e >= num_events) return;  // whole waves
+  const unsigned lane = threadIdx.x & 63u;
+  const double r = canonical[e] * total;
+  // the first chunk with S > r
+  uint64_t lo = 0, hi = nchunks;  // it is in [lo, hi]; hi: none before
+  while (lo < hi) {
+    const uint64_t step = (hi - lo + 63) / 64;
+    const uint64_t at = min(lo + (lane + 1) * step, hi) - 1;
+    const uint64_t over = __ballot(S[at] > r);
+    if (!over) {
+      lo = hi;
+      break;
+    }
+    const unsigned f = (unsigned)__builtin_ctzll(over);
+    hi = min(lo + (f + 1) * step, hi) - 1;
+    lo = lo + f * step;
+  }
+  const uint64_t c = lo >= nchunks ? last_chunk : lo;
+  const double start = c ? S[c - 1] : 0.0;
+  // the first wave whose last C exceeds r, and the sum before it
+  const double mine = lane < (unsigned)SAMPLE_WAVES ? chunk_waves[c * SAMPLE_WAVES + lane] : 0.0;
+  double wave_before = 0.0;
+  int wave = 0;
+  for (; wave < SAMPLE_WAVES; ++wave) {
+    const double next = wave_before + readlane_f64(mine, wave);
+    if (start + next > r) break;
+    wave_before = next;
+  }
+  const uint32_t per = chunk >= SAMPLE_THREADS ? chunk / SAMPLE_THREADS : 1;
+  const uint64_t base = c * chunk;
+  constexpr int PER = SAMPLE_CHUNK / SAMPLE_THREADS;
+  double p[PER];
+  auto load = [&](int w) {  // the lane's probabilities in wave w (0 beyond the chunk)
+    const uint32_t first = ((uint32_t)w * 64 + lane) * per;
+#pragma unroll
+    for (int k = 0; k < PER; ++k) {
+      p[k] = 0.0;
+      if ((uint32_t)k < per && first + k < chunk) {
+        const cpx<R> x = a[base + first + k];
+        p[k] = (double)x.re * x.re + (double)x.im * x.im;
+      }
+    }
+  };
+  if (wave < SAMPLE_WAVES) {
+    load(wave);
+    double t = 0.0;
+#pragma unroll
+    for (int k = 0; k < PER; ++k) t += p[k];  // (t + 0.0 = t: sums are never -0)
+    double run = 0.0, before = 0.0;
+    for (unsigned k = 0; k < 64; ++k) {
+      if (k == lane) before = run;
+      run += readlane_f64(t, (int)k);
+    }
+    double acc = 0.0;
+    int found = PER;
+#pragma unroll
+    for (int k = 0; k < PER; ++k) {
+      acc += p[k];
+      if (found == PER && start + (wave_before + (before + acc)) > r) found = k;
+    }
+    const uint64_t hit = __ballot(found < PER);
+    if (hit) {
+      if (lane == (unsigned)__builtin_ctzll(hit)) events[e] = base + ((uint32_t)wave * 64 + lane) * per + found;
+      return;
+    }
+  }
+  // none exceeds r (a target at the total): the chunk's last index of non-zero probability
+  for (int w = SAMPLE_WAVES - 1; w >= 0; --w) {
+    load(w);
+    int last = -1;
+#pragma unroll
+    for (int k = 0; k < PER; ++k)
+      if (p[k] > 0.0) last = k;
+    const uint64_t any = __ballot(last >= 0);
+    if (any) {
+      if (lane == 63u - (unsigned)__builtin_clzll(any)) events[e] = base + ((uint32_t)w * 64 + lane) * per + last;
+      return;
+    }
+  }
+  if (lane == 0) events[e] = base;
 }
 
 // One block per event: the first index of chunk chunk_of[e] whose C exceeds
@@ -751,23 +856,30 @@ int brk_generate_events(const void* first, uint64_t size, int dtype, const doubl
   const uint64_t nchunks = size / chunk;
   if (nchunks > 0x7fffffffull) return fail(BRK_ERR_INVALID_ARGUMENT, "state too large");
   hipStream_t s = as_stream(stream);
-  // device buffers: chunk sums, then their running sums | per event: draw, chunk, chunk start,
-  // target, result
-  const size_t bytes = sizeof(double) * nchunks + (sizeof(uint64_t) * 2 + sizeof(double) * 3) * num_events;
+  // device buffers: chunk sums, then their running sums | per event: draw, result | the wave sums
+  // of every chunk (1/1024 of a c128 state).  Without room for the wave sums an event searches its
+  // whole chunk, as in brk_generate_events_noalloc, and takes three more numbers.
+  const size_t event_bytes = (sizeof(uint64_t) * 2 + sizeof(double) * 3) * num_events;
+  const size_t bytes = sizeof(double) * nchunks + event_bytes;
   void* buffers = nullptr;
-  BRK_HIP_CHECK(hipMalloc(&buffers, bytes));
+  bool by_wave = hipMalloc(&buffers, bytes + sizeof(double) * SAMPLE_WAVES * nchunks) == hipSuccess;
+  if (!by_wave) {
+    (void)hipGetLastError();
+    BRK_HIP_CHECK(hipMalloc(&buffers, bytes));
+  }
   double* d_sums = static_cast<double*>(buffers);
   double* d_canonical = d_sums + nchunks;
   uint64_t* d_chunk = reinterpret_cast<uint64_t*>(d_canonical + num_events);
   double* d_start = reinterpret_cast<double*>(d_chunk + num_events);
   double* d_target = d_start + num_events;
   uint64_t* d_events = reinterpret_cast<uint64_t*>(d_target + num_events);
+  double* d_waves = by_wave ? reinterpret_cast<double*>(d_events + num_events) : nullptr;
   if (dtype == BRK_C128)
     hipLaunchKernelGGL(k_chunk_sums<double>, dim3((unsigned)nchunks), dim3(SAMPLE_THREADS), 0, s,
-                       (const cpx<double>*)first, chunk, d_sums);
+                       (const cpx<double>*)first, chunk, d_sums, d_waves);
   else
     hipLaunchKernelGGL(k_chunk_sums<float>, dim3((unsigned)nchunks), dim3(SAMPLE_THREADS), 0, s,
-                       (const cpx<float>*)first, chunk, d_sums);
+                       (const cpx<float>*)first, chunk, d_sums, d_waves);
   std::vector<double> sums(nchunks);
   int status = check_launch("chunk sums");
   if (!status && (hipMemcpyAsync(sums.data(), d_sums, sizeof(double) * nchunks, hipMemcpyDeviceToHost, s) != hipSuccess ||
@@ -789,20 +901,30 @@ int brk_generate_events(const void* first, uint64_t size, int dtype, const doubl
         hipMemcpyAsync(d_canonical, canonical, sizeof(double) * num_events, hipMemcpyHostToDevice, s) !=
             hipSuccess)
       status = fail(BRK_ERR_HIP, "uploading the running sums failed");
-    if (!status) {
-      hipLaunchKernelGGL(k_locate_events, dim3((num_events + 255) / 256), dim3(256), 0, s, d_sums, nchunks,
-                         S[nchunks - 1], last_chunk, d_canonical, num_events, d_chunk, d_start, d_target);
-      status = check_launch("locate events");
-    }
   }
-  if (!status) {
+  if (!status && by_wave) {
+    const unsigned per_block = FIND_THREADS / 64;
+    const dim3 grid((num_events + per_block - 1) / per_block), block(FIND_THREADS);
     if (dtype == BRK_C128)
-      hipLaunchKernelGGL(k_chunk_search<double>, dim3(num_events), dim3(SAMPLE_THREADS), 0, s,
-                         (const cpx<double>*)first, chunk, d_chunk, d_start, d_target, d_events);
+      hipLaunchKernelGGL(k_find_events<double>, grid, block, 0, s, (const cpx<double>*)first, chunk, d_sums, nchunks,
+                         S[nchunks - 1], last_chunk, d_waves, d_canonical, num_events, d_events);
     else
-      hipLaunchKernelGGL(k_chunk_search<float>, dim3(num_events), dim3(SAMPLE_THREADS), 0, s,
-                         (const cpx<float>*)first, chunk, d_chunk, d_start, d_target, d_events);
-    status = check_launch("chunk search");
+      hipLaunchKernelGGL(k_find_events<float>, grid, block, 0, s, (const cpx<float>*)first, chunk, d_sums, nchunks,
+                         S[nchunks - 1], last_chunk, d_waves, d_canonical, num_events, d_events);
+    status = check_launch("find events");
+  } else if (!status) {
+    hipLaunchKernelGGL(k_locate_events, dim3((num_events + 255) / 256), dim3(256), 0, s, d_sums, nchunks,
+                       S[nchunks - 1], last_chunk, d_canonical, num_events, d_chunk, d_start, d_target);
+    status = check_launch("locate events");
+    if (!status) {
+      if (dtype == BRK_C128)
+        hipLaunchKernelGGL(k_chunk_search<double>, dim3(num_events), dim3(SAMPLE_THREADS), 0, s,
+                           (const cpx<double>*)first, chunk, d_chunk, d_start, d_target, d_events);
+      else
+        hipLaunchKernelGGL(k_chunk_search<float>, dim3(num_events), dim3(SAMPLE_THREADS), 0, s,
+                           (const cpx<float>*)first, chunk, d_chunk, d_start, d_target, d_events);
+      status = check_launch("chunk search");
+    }
   }
   if (!status && (hipMemcpyAsync(events, d_events, sizeof(uint64_t) * num_events, hipMemcpyDeviceToHost, s) !=
                       hipSuccess ||
@@ -851,10 +973,10 @@ int brk_generate_events_noalloc(const void* first, uint64_t size, int dtype, con
   auto run = [&]() -> int {
     if (dtype == BRK_C128)
       hipLaunchKernelGGL(k_chunk_sums<double>, dim3((unsigned)nchunks), dim3(SAMPLE_THREADS), 0, s,
-                         (const cpx<double>*)first, chunk, d_sums);
+                         (const cpx<double>*)first, chunk, d_sums, (double*)nullptr);
     else
       hipLaunchKernelGGL(k_chunk_sums<float>, dim3((unsigned)nchunks), dim3(SAMPLE_THREADS), 0, s,
-                         (const cpx<float>*)first, chunk, d_sums);
+                         (const cpx<float>*)first, chunk, d_sums, (double*)nullptr);
     if (int st = check_launch("chunk sums")) return st;
     hipLaunchKernelGGL(k_running_sums, dim3(1), dim3(64), 0, s, d_sums, nchunks, d_meta);
     if (int st = check_launch("running sums")) return st;
