@@ -155,17 +155,151 @@ __device__ __forceinline__ double ising_diag(uint64_t k, const ising_args& a) {
   return e;
 }
 
+// <H> of the open-chain Ising Hamiltonian in a few passes over the state.  A pass holds chunks of
+// 2^L amplitudes (64 KiB: L = 12 for c128, 13 for c64) whose L local bits are the physical qubits
+// pos[]; a thread loads PER = 2^GB amplitudes differing in the GB highest local bits, adds those
+// bits' X terms in registers and, in the first pass, the ZZ terms; the chunk then goes to LDS once
+// and is read back in groups of PER amplitudes over the other local bits, GB bits a round.  The
+// next chunk's loads are in flight during the rounds.  The first pass takes qubits 0 .. L - 1, each
+// further one the 128-byte line's qubits and up to L - line others: 3 reads of a 28-qubit c128 state
+// instead of the 29 of one pass per term.  Bound: HBM reads (28 qubits c128: 0.81 ms a pass, 5.3 TB/s,
+// 2.4 ms in all; a pass per term took 22 ms).
+// LDS addresses are XOR-swizzled so that both access shapes spread over all banks.
+constexpr int ISING_THREADS = 512;
+constexpr int ISING_THREAD_BITS = 9;
+constexpr int ISING_GRID = 512;  // two workgroups per CU; fixed, so that the summation order is
+constexpr int ISING_TABLES = MAX_CHAIN / 8;
+constexpr int ISING_MAX_LOCAL = 13;
+
+struct ising_pass {
+  double J[MAX_CHAIN];
+  double h2[ISING_MAX_LOCAL];      // 2 h of the qubit at a local position
+  uint32_t pos[ISING_MAX_LOCAL];   // ascending; L entries
+  uint32_t measure;                // local positions whose X term is added
+  int n;
+  int zz;                          // add the ZZ terms (the local bits are then 0 .. L - 1)
+};
+
 template <typename R>
-__global__ __launch_bounds__(RED_THREADS) void k_ising_zz(const cpx<R>* __restrict__ a, uint64_t size,
-                                                         ising_args args, double* partial) {
-  dvec<1> acc{{0.0}};
-  const uint64_t stride = (uint64_t)RED_BLOCKS * RED_THREADS;
-  for (uint64_t i = (uint64_t)blockIdx.x * RED_THREADS + threadIdx.x; i < size; i += stride) {
-    cpx<R> x = a[i];
-    const double xr = x.re, xi = x.im;
-    acc.v[0] += (xr * xr + xi * xi) * ising_diag(i, args);
+struct ising_shape {
+  static constexpr int GB = sizeof(R) == 8 ? 3 : 4;
+  static constexpr int L = ISING_THREAD_BITS + GB;
+};
+
+template <typename R>
+__global__ __launch_bounds__(ISING_THREADS) void k_ising(const cpx<R>* __restrict__ a, uint64_t size,
+                                                        uint64_t nchunks, ising_pass P,
+                                                        double* __restrict__ partial) {
+  constexpr int GB = ising_shape<R>::GB, L = ising_shape<R>::L, PER = 1 << GB;
+  __shared__ cpx<R> lds[1 << L];
+  __shared__ double table[ISING_TABLES * 256];  // ZZ energy of a byte of the bond pattern i ^ (i >> 1)
+  __shared__ double wave_sums[ISING_THREADS / 64];
+  const uint32_t t = threadIdx.x;
+  if (P.zz) {
+    for (uint32_t e = t; e < (uint32_t)ISING_TABLES * 256; e += ISING_THREADS) {
+      double v = 0.0;
+      for (int b = 0; b < 8; ++b) {
+        const int bond = 8 * (int)(e >> 8) + b;
+        if (bond + 1 < P.n) v += ((e >> b) & 1u) ? -P.J[bond] : P.J[bond];
+      }
+      table[e] = v;
+    }
+    __syncthreads();
   }
-  block_store<1>(acc, partial);
+  auto swizzle = [](uint32_t j) { return j ^ ((j >> GB) & (uint32_t)(PER - 1)); };
+  uint64_t low = 0;
+#pragma unroll
+  for (int r = 0; r < ISING_THREAD_BITS; ++r) low |= (uint64_t)((t >> r) & 1u) << P.pos[r];
+  uint64_t high[PER];
+#pragma unroll
+  for (int k = 0; k < PER; ++k) {
+    high[k] = 0;
+#pragma unroll
+    for (int g = 0; g < GB; ++g)
+      if ((k >> g) & 1) high[k] |= 1ull << P.pos[ISING_THREAD_BITS + g];
+  }
+  auto base_of = [&](uint64_t c) {  // zeros inserted at the local positions
+#pragma unroll
+    for (int r = 0; r < L; ++r) {
+      const uint32_t q = P.pos[r];
+      c = ((c >> q) << (q + 1)) | (c & ((1ull << q) - 1ull));
+    }
+    return c;
+  };
+  cpx<R> x[PER];
+  auto load = [&](uint64_t c) {
+    const uint64_t b = base_of(c) | low;
+#pragma unroll
+    for (int k = 0; k < PER; ++k) {
+      const uint64_t i = b | high[k];
+      x[k] = i < size ? a[i] : cpx<R>{R(0), R(0)};  // (a state smaller than a chunk)
+    }
+  };
+  // the X terms of group bits [0, GB) of v, bit g at local position first + g
+  double acc = 0.0;
+  auto add_x = [&](const cpx<R> (&v)[PER], int first, uint32_t mask) {
+#pragma unroll
+    for (int g = 0; g < GB; ++g) {
+      if (!((mask >> g) & 1u)) continue;
+      double s = 0.0;
+#pragma unroll
+      for (int m = 0; m < PER; ++m) {
+        if ((m >> g) & 1) continue;
+        const cpx<R> v0 = v[m], v1 = v[m | (1 << g)];
+        s = __builtin_fma((double)v0.re, (double)v1.re, s);
+        s = __builtin_fma((double)v0.im, (double)v1.im, s);
+      }
+      acc = __builtin_fma(P.h2[first + g], s, acc);
+    }
+  };
+  const uint32_t in_registers = P.measure >> ISING_THREAD_BITS;
+  const bool rounds = (P.measure & ((1u << ISING_THREAD_BITS) - 1u)) != 0;
+  uint64_t c = blockIdx.x;
+  if (c < nchunks) load(c);
+  for (; c < nchunks; c += gridDim.x) {
+    add_x(x, ISING_THREAD_BITS, in_registers);
+    if (P.zz) {
+      // bond bits 0..7 depend on t alone, bits 16.. on the chunk alone
+      const uint64_t i0 = (c << L) | t, d0 = i0 ^ (i0 >> 1);
+      double fixed = table[d0 & 255u];
+      for (int b = 2; 8 * b + 1 < P.n; ++b) fixed += table[256 * b + ((d0 >> (8 * b)) & 255u)];
+#pragma unroll
+      for (int k = 0; k < PER; ++k) {
+        const uint64_t i = i0 | ((uint64_t)k << ISING_THREAD_BITS), d = i ^ (i >> 1);
+        const double re = x[k].re, im = x[k].im;
+        acc = __builtin_fma(__builtin_fma(re, re, im * im), fixed + table[256 + ((d >> 8) & 255u)], acc);
+      }
+    }
+    if (rounds) {
+#pragma unroll
+      for (int k = 0; k < PER; ++k) lds[swizzle(t + ISING_THREADS * k)] = x[k];
+      __syncthreads();
+    }
+    if (c + gridDim.x < nchunks) load(c + gridDim.x);
+    if (rounds) {
+#pragma unroll
+      for (int first = 0; first < ISING_THREAD_BITS; first += GB) {
+        uint32_t mask = (P.measure >> first) & (uint32_t)(PER - 1);
+        if (first + GB > ISING_THREAD_BITS) mask &= (1u << (ISING_THREAD_BITS - first)) - 1u;  // the rest: registers
+        if (!mask) continue;
+        const uint32_t j = ((t >> first) << (first + GB)) | (t & ((1u << first) - 1u));
+        cpx<R> v[PER];
+#pragma unroll
+        for (int m = 0; m < PER; ++m) v[m] = lds[swizzle(j | ((uint32_t)m << first))];
+        add_x(v, first, mask);
+      }
+      __syncthreads();
+    }
+  }
+  acc = wave_sum(acc);
+  if ((t & 63u) == 0) wave_sums[t >> 6] = acc;
+  __syncthreads();
+  if (t == 0) {
+    double sum = 0.0;
+#pragma unroll
+    for (int w = 0; w < ISING_THREADS / 64; ++w) sum += wave_sums[w];
+    partial[blockIdx.x] = sum;
+  }
 }
 
 template <typename R>
@@ -630,6 +764,62 @@ static int make_ising_args(unsigned nq, const double* J, const double* h, ising_
   return BRK_OK;
 }
 
+// <H> in passes of k_ising (terms with h = 0 are left out).
+template <typename R>
+static int ising_energy(const void* first, uint64_t size, const ising_args& args, double* result, void* stream) {
+  constexpr unsigned L = ising_shape<R>::L, line = sizeof(R) == 8 ? 3 : 4;  // qubits of a 128-byte line
+  const unsigned n = (unsigned)args.n;
+  const uint64_t nchunks = std::max<uint64_t>(1, size >> L);
+  const unsigned grid = (unsigned)std::min<uint64_t>(nchunks, ISING_GRID);
+  std::vector<ising_pass> passes;
+  for (unsigned next = 0; next == 0 || next < n;) {
+    ising_pass p{};
+    p.n = args.n;
+    p.zz = next == 0;
+    std::copy(args.J, args.J + MAX_CHAIN, p.J);
+    // the first L qubits, then the line's qubits and the next L - line ones (fewer: filled up with
+    // the lowest others)
+    const unsigned end = std::min(n, next == 0 ? L : next + (L - line));
+    uint64_t local = next == 0 ? 0 : (1ull << line) - 1ull;
+    for (unsigned q = next; q < end; ++q) local |= 1ull << q;
+    for (unsigned q = 0; (unsigned)__builtin_popcountll(local) < L; ++q) local |= 1ull << q;
+    unsigned r = 0;
+    for (unsigned q = 0; r < L; ++q) {
+      if (!(local >> q & 1ull)) continue;
+      p.pos[r] = q;
+      if (q >= next && q < end && args.h[q] != 0.0) {
+        p.measure |= 1u << r;
+        p.h2[r] = 2.0 * args.h[q];  // <X_q> = 2 sum Re conj(a0) a1
+      }
+      ++r;
+    }
+    if (p.zz || p.measure) passes.push_back(p);
+    next = next == 0 ? L : end;
+  }
+  reduce_scratch* sc;
+  if (int st = get_reduce_scratch(&sc)) return st;
+  const size_t values = passes.size() * grid;
+  if (values > (size_t)RED_BLOCKS * RED_MAX_VALUES) return fail(BRK_ERR_INVALID_ARGUMENT, "too many Ising passes");
+  std::lock_guard<std::mutex> hold(sc->busy);
+  hipStream_t s = as_stream(stream);
+  int status = BRK_OK;
+  for (size_t k = 0; !status && k < passes.size(); ++k) {
+    hipLaunchKernelGGL(k_ising<R>, dim3(grid), dim3(ISING_THREADS), 0, s, (const cpx<R>*)first, size, nchunks,
+                       passes[k], sc->device + k * grid);
+    status = check_launch("Ising energy");
+  }
+  const hipError_t copied =
+      status ? hipSuccess : hipMemcpyAsync(sc->host, sc->device, sizeof(double) * values, hipMemcpyDeviceToHost, s);
+  const hipError_t synced = hipStreamSynchronize(s);
+  if (status) return status;
+  if (copied != hipSuccess) return fail(BRK_ERR_HIP, "Ising read-back: %s", hipGetErrorString(copied));
+  if (synced != hipSuccess) return fail(BRK_ERR_HIP, "Ising energy: %s", hipGetErrorString(synced));
+  double total = 0.0;
+  for (size_t k = 0; k < values; ++k) total += sc->host[k];
+  *result = total;
+  return BRK_OK;
+}
+
 }  // namespace brk
 
 using namespace brk;
@@ -751,28 +941,8 @@ int brk_expectation_ising(const void* first, uint64_t size, int dtype, const dou
   if (!result) return fail(BRK_ERR_INVALID_ARGUMENT, "result is null");
   ising_args a;
   if (int st = make_ising_args(nq, J, h, &a)) return st;
-  double zz = 0.0;
-  int st = run_reduction<1>(
-      stream,
-      [&](double* partial, hipStream_t s) {
-        if (dtype == BRK_C128)
-          hipLaunchKernelGGL(k_ising_zz<double>, dim3(RED_BLOCKS), dim3(RED_THREADS), 0, s,
-                             (const cpx<double>*)first, size, a, partial);
-        else
-          hipLaunchKernelGGL(k_ising_zz<float>, dim3(RED_BLOCKS), dim3(RED_THREADS), 0, s,
-                             (const cpx<float>*)first, size, a, partial);
-      },
-      &zz);
-  if (st) return st;
-  double total = zz;
-  for (unsigned q = 0; q < nq; ++q) {
-    if (h[q] == 0.0) continue;
-    double raw[3];
-    if (int st2 = spin_raw(first, size, dtype, q, raw, stream)) return st2;
-    total += h[q] * 2.0 * raw[0];  // <X_q> = 2 sum Re conj(a0) a1
-  }
-  *result = total;
-  return BRK_OK;
+  if (dtype == BRK_C128) return ising_energy<double>(first, size, a, result, stream);
+  return ising_energy<float>(first, size, a, result, stream);
 }
 
 int brk_apply_ising(void* out, const void* psi, uint64_t size, int dtype, const double* J, const double* h,

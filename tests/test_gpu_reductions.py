@@ -73,6 +73,30 @@ def test_ising(oracle, n, dtype):
     out.free()
 
 
+@pytest.mark.parametrize("dtype", [brk.C128, brk.C64])
+@pytest.mark.parametrize("n", [1, 2, 5, 9, 11, 12, 13, 14, 21, 22])
+def test_ising_chunk_edges(oracle, n, dtype):
+    """Sizes around a chunk (2^12 or 2^13 amplitudes) and around the 9 further qubits of each pass, with terms
+    left out (h = 0); both sides sum 2^n terms of a unit state in FP64, each rounding at most eps of a partial
+    sum bounded by the sum of the coefficients."""
+    note(f"gpu ising chunk edges n={n} dtype={dtype}")
+    rng = np.random.default_rng(70 + n)
+    host = D.random_state(n, rng).astype(np.complex128 if dtype == brk.C128 else np.complex64)
+    J, h = rng.uniform(-1, 1, max(0, n - 1)), rng.uniform(-1, 1, n)
+    h[1::3] = 0.0
+    st = DeviceState.from_host(host, dtype)
+    e = brk.expectation_ising(st.ptr, st.size, dtype, J, h)
+    ref = oracle.expectation_ising(host.astype(np.complex128), J, h)
+    assert abs(e - ref) < 2 * (2.0 ** n + 16) * np.finfo(float).eps * (np.sum(np.abs(J)) + np.sum(np.abs(h)) + 1)
+    for q in {0, n // 2, n - 1}:  # one X term alone
+        one = np.zeros(n)
+        one[q] = 1.0
+        e = brk.expectation_ising(st.ptr, st.size, dtype, np.zeros(max(0, n - 1)), one)
+        assert abs(e - oracle.expectation_ising(host.astype(np.complex128), np.zeros(max(0, n - 1)), one)) < (
+            2 * (2.0 ** n + 16) * np.finfo(float).eps)
+    st.free()
+
+
 def test_mixed_precision_inner_product(oracle):
     note("gpu mixed inner product")
     rng = np.random.default_rng(9)
