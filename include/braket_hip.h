@@ -537,10 +537,10 @@ int brk_adjoint_ising_gradient(const brk_circuit* circuit, void* psi, void* work
                                void* stream);
 
 /* ------------------------------------------------------------------------ */
-/* Batching form: many small independent circuits in one persistent launch, */
-/* captured once as a HIP graph and replayed.  Each circuit runs on its own */
-/* complex64 state from |0...0> and yields its FP64 open-chain Ising energy */
-/* sum_i J_i <Z_i Z_i+1> + sum_i h_i <X_i>.  Reference ancestor: bra's      */
+/* Batching form: many small independent circuits in one persistent launch  */
+/* per stage, captured as one HIP graph and replayed.  Each circuit runs on  */
+/* its own complex64 state from |0...0> and yields its FP64 open-chain      */
+/* Ising energy sum_i J_i <Z_i Z_i+1> + sum_i h_i <X_i>.  Reference: bra's  */
 /* CIRCUITS mode, which advances several states in turn                     */
 /* (bra/src/bra.cpp:315-336, bra/src/interpreter.cpp:411-419).              */
 /* ------------------------------------------------------------------------ */

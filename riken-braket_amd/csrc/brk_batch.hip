@@ -3,9 +3,12 @@
 // CIRCUITS mode, which advances several states one after another,
 // bra/src/bra.cpp:315-336, bra/src/interpreter.cpp:411-419).
 //
-// Two 512-thread workgroups per CU take circuits from a global queue (most
-// expensive first); while one is in a barrier-separated LDS phase the other
-// computes.  The program layout is described in brk_batch.hpp.  Per
+// One launch per stage level; two 512-thread workgroups per CU take items (a few
+// chunks of one circuit's stage) from a queue, most expensive first; while one is
+// in a barrier-separated LDS phase the other computes.  The program layout is
+// described in brk_batch.hpp.  An item that measures writes an FP64 partial; the
+// item that finds the circuit's others done adds them in item order, so energies
+// do not depend on timing.  Per
 // chunk: load (or initialise) into LDS, apply the stage's instructions with a
 // barrier between them, accumulate the energy terms the stage measures, store.
 // A gate group holds up to 4 local positions: each thread keeps the 16
@@ -28,6 +31,7 @@ typedef const __attribute__((address_space(4))) uint32_t* cu32;
 typedef const __attribute__((address_space(4))) double* cf64;
 typedef const __attribute__((address_space(4))) batch_stage* cstage;
 typedef const __attribute__((address_space(4))) batch_circuit* ccircuit;
+typedef const __attribute__((address_space(4))) batch_item* citem;
 
 constexpr int ZZ_TABLES = 3;  // byte tables of the ZZ energy: n - 1 <= 23 bond bits
 
@@ -257,149 +261,174 @@ __global__ __launch_bounds__(BATCH_THREADS, BATCH_WAVES_PER_SIMD) void k_batch(b
   __shared__ __align__(16) f2 chunk[BATCH_CHUNK_PADDED];
   __shared__ uint32_t tlo[128], thi[128];
   __shared__ double zz[ZZ_TABLES * 256];  // ZZ energy byte tables
-  __shared__ uint32_t next[1];
-  double* red = reinterpret_cast<double*>(chunk);  // reuses the chunk after the last stage
+  __shared__ uint32_t next[1], last_item[1];
+  double* red = reinterpret_cast<double*>(chunk);  // reuses the chunk after an item's last chunk
   const uint32_t tid = threadIdx.x;
-  f2* slot = P.slots ? reinterpret_cast<f2*>(P.slots) + (size_t)blockIdx.x * P.slot_elems : nullptr;
   const ccircuit circuits = (ccircuit)P.circuits;
   const cstage stages = (cstage)P.stages;
+  const citem items = (citem)P.items;
   const cu32 words = (cu32)P.words;
   const cf64 ham = (cf64)P.ham;
-  const cu32 order = (cu32)P.order;
 
   for (;;) {
     if (tid == 0) *next = atomicAdd(P.counter, 1u);
     __syncthreads();
     const uint32_t k = __builtin_amdgcn_readfirstlane(*next);
-    if (k >= P.num_circuits) break;
-    const uint32_t ci = order[k];
+    if (k >= P.num_items) break;
+    const uint32_t ci = items[k].circuit;
     const uint32_t n = circuits[ci].n;
-    const uint32_t num_stages = circuits[ci].num_stages;
-    const uint32_t first_stage = circuits[ci].first_stage;
     const cf64 J = ham + circuits[ci].ham_offset;
     const cf64 h = J + (n - 1);
-    if (tid == 0) P.t_start[ci] = (uint64_t)wall_clock64();
-    // ZZ energy of a bond pattern d (bit i set: Z_i Z_i+1 = -1) = sum of its three byte-table entries
-    for (uint32_t t = tid; t < ZZ_TABLES * 256; t += BATCH_THREADS) {
-      const uint32_t byte = t >> 8, b = t & 255u;
-      double e = 0.0;
-      for (uint32_t i = 0; i < 8; ++i) {
-        const uint32_t bond = 8 * byte + i;
-        if (bond + 1 < n) e += ((b >> i) & 1u) ? -J[bond] : J[bond];
+    f2* const slot = reinterpret_cast<f2*>(P.slots) + circuits[ci].slot;
+    if (tid == 0 && items[k].first) P.t_start[ci] = (uint64_t)wall_clock64();
+    const cstage S = stages + items[k].stage;
+    const uint32_t L = S->L, flags = S->flags, chunk_mask = S->chunk_mask, measure_x = S->measure_x;
+    const uint32_t unreached = ~S->reached;
+    const uint32_t num_instr = S->num_instr;
+    const cu32 first_word = words + S->first_word;
+    if (flags & BS_ZZ) {
+      // ZZ energy of a bond pattern d (bit i set: Z_i Z_i+1 = -1) = sum of its three byte-table entries
+      for (uint32_t t = tid; t < ZZ_TABLES * 256; t += BATCH_THREADS) {
+        const uint32_t byte = t >> 8, b = t & 255u;
+        double e = 0.0;
+        for (uint32_t i = 0; i < 8; ++i) {
+          const uint32_t bond = 8 * byte + i;
+          if (bond + 1 < n) e += ((b >> i) & 1u) ? -J[bond] : J[bond];
+        }
+        zz[t] = e;
       }
-      zz[t] = e;
     }
     double acc = 0.0;
-
-    for (uint32_t s = 0; s < num_stages; ++s) {
-      const cstage S = stages + first_stage + s;
-      const uint32_t L = S->L, flags = S->flags, nonlocal = S->nonlocal_mask, measure_x = S->measure_x;
-      const uint32_t num_instr = S->num_instr;
-      const cu32 first_word = words + S->first_word;
-      if (tid < 128) {
-        uint32_t lo = 0, hi = 0;
-        for (uint32_t q = 0; q < 7; ++q) {
-          if (q < L && ((tid >> q) & 1u)) lo |= 1u << S->local[q];
-          if (q + 7 < L && ((tid >> q) & 1u)) hi |= 1u << S->local[q + 7];
-        }
-        tlo[tid] = lo;
-        thi[tid] = hi;
+    if (tid < 128) {
+      uint32_t lo = 0, hi = 0;
+      for (uint32_t q = 0; q < 7; ++q) {
+        if (q < L && ((tid >> q) & 1u)) lo |= 1u << S->local[q];
+        if (q + 7 < L && ((tid >> q) & 1u)) hi |= 1u << S->local[q + 7];
       }
-      __syncthreads();
-      const uint32_t csize = 1u << L;
-      const uint32_t nchunks = 1u << (n - L);
-      for (uint32_t cidx = 0; cidx < nchunks; ++cidx) {
-        const chunk_ctx c{chunk, tlo, thi, deposit(cidx, nonlocal), L, S};
-        if (flags & BS_INIT) {
-          for (uint32_t j = tid; j < csize; j += BATCH_THREADS)
-            chunk[lpad(j)] = f2{global_index(c, j) == 0 ? 1.0f : 0.0f, 0.0f};
-        } else {
-          // a circuit with stages after the first has n > BATCH_MAX_LOCAL, so its chunks are full
-          // (csize = BATCH_CHUNK); all of the thread's loads go out at once (a loop would wait for
-          // each in turn)
-          f2 v[CHUNK_PER_THREAD];
-#pragma unroll
-          for (int r = 0; r < CHUNK_PER_THREAD; ++r) v[r] = slot[global_index(c, tid + BATCH_THREADS * r)];
-#pragma unroll
-          for (int r = 0; r < CHUNK_PER_THREAD; ++r) chunk[lpad(tid + BATCH_THREADS * r)] = v[r];
-        }
-        __syncthreads();
-        cu32 w = first_word;
-        for (uint32_t i = 0; i < num_instr; ++i) {
-          const uint32_t w0 = w[0], op = w0 & 0xffu;
-          if (op == BI_GATES) {
-            const uint32_t npos = (w0 >> 8) & 0xffu;
-            switch (npos) {
-              case 1: gate_pass<1, BI_GATES>(c, w, tid); break;
-              case 2: gate_pass<2, BI_GATES>(c, w, tid); break;
-              case 3: gate_pass<3, BI_GATES>(c, w, tid); break;
-              default: gate_pass<4, BI_GATES>(c, w, tid); break;
-            }
-            w += 4 + 2 * (((w0 >> 16) & 0xffu) + (w0 >> 24)) + BATCH_GATE_WORDS * npos;
-          } else if (op == BI_GATES_REAL || op == BI_GATES_REAL_PRE) {
-            // the planner emits BI_GATES_REAL for 1..4 positions, BI_GATES_REAL_PRE for 2..4 (for one
-            // position with both tables the complex form is cheaper)
-            const uint32_t npos = (w0 >> 8) & 0xffu;
-            if (op == BI_GATES_REAL) {
-              switch (npos) {
-                case 1: gate_pass<1, BI_GATES_REAL>(c, w, tid); break;
-                case 2: gate_pass<2, BI_GATES_REAL>(c, w, tid); break;
-                case 3: gate_pass<3, BI_GATES_REAL>(c, w, tid); break;
-                default: gate_pass<4, BI_GATES_REAL>(c, w, tid); break;
-              }
-            } else {
-              switch (npos) {
-                case 2: gate_pass<2, BI_GATES_REAL_PRE>(c, w, tid); break;
-                case 3: gate_pass<3, BI_GATES_REAL_PRE>(c, w, tid); break;
-                default: gate_pass<4, BI_GATES_REAL_PRE>(c, w, tid); break;
-              }
-            }
-            w += 4 + 2 * (((w0 >> 16) & 0xffu) + (w0 >> 24)) + BATCH_REAL_WORDS * npos +
-                 2 * (1u << npos) * (op == BI_GATES_REAL_PRE ? 2u : 1u);
-          } else {
-            sign_pass(c, w, tid);
-            w += 1 + 2 * ((w0 >> 16) & 0xffffu);
-          }
-          __syncthreads();
-        }
-        if (flags & BS_ZZ) {
-          const uint32_t bonds = n > 1 ? (1u << (n - 1)) - 1u : 0u;
-          for (uint32_t j = tid; j < csize; j += BATCH_THREADS) {
-            const uint32_t x = global_index(c, j);
-            const f2 v = chunk[lpad(j)];
-            const double p = (double)v.re * (double)v.re + (double)v.im * (double)v.im;
-            const uint32_t d = (x ^ (x >> 1)) & bonds;
-            acc += p * (zz[d & 255u] + zz[256 + ((d >> 8) & 255u)] + zz[512 + (d >> 16)]);
-          }
-        }
-        for (uint32_t mx = measure_x; mx; mx &= mx - 1) {
-          const uint32_t pos = __builtin_ctz(mx);
-          const double h2 = 2.0 * h[S->local[pos]];
-          for (uint32_t g = tid; g < (csize >> 1); g += BATCH_THREADS) {
-            const uint32_t j0 = ((g >> pos) << (pos + 1)) | (g & ((1u << pos) - 1u));
-            const f2 a0 = chunk[lpad(j0)], a1 = chunk[lpad(j0 | (1u << pos))];
-            acc += h2 * ((double)a0.re * (double)a1.re + (double)a0.im * (double)a1.im);
-          }
-        }
-        if (flags & BS_STORE) {
-          f2 v[CHUNK_PER_THREAD];  // (full chunks, as for the loads)
-#pragma unroll
-          for (int r = 0; r < CHUNK_PER_THREAD; ++r) v[r] = chunk[lpad(tid + BATCH_THREADS * r)];
-#pragma unroll
-          for (int r = 0; r < CHUNK_PER_THREAD; ++r) slot[global_index(c, tid + BATCH_THREADS * r)] = v[r];
-        }
-        __syncthreads();
-      }
+      tlo[tid] = lo;
+      thi[tid] = hi;
     }
-
-    // fixed-shape tree over the workgroup: the energy does not depend on timing
-    red[tid] = acc;
     __syncthreads();
-    for (uint32_t half = BATCH_THREADS / 2; half > 0; half >>= 1) {
-      if (tid < half) red[tid] += red[tid + half];
+    const uint32_t csize = 1u << L;
+    const uint32_t end_chunk = items[k].first_chunk + items[k].num_chunks;
+    for (uint32_t cidx = items[k].first_chunk; cidx < end_chunk; ++cidx) {
+      const chunk_ctx c{chunk, tlo, thi, deposit(cidx, chunk_mask), L, S};
+      if (flags & BS_INIT) {
+        for (uint32_t j = tid; j < csize; j += BATCH_THREADS)
+          chunk[lpad(j)] = f2{global_index(c, j) == 0 ? 1.0f : 0.0f, 0.0f};
+      } else {
+        // a circuit with stages after the first has n > BATCH_MAX_LOCAL, so its chunks are full
+        // (csize = BATCH_CHUNK); all of the thread's loads go out at once (a loop would wait for
+        // each in turn).  Amplitudes no stage has reached are zero.
+        f2 v[CHUNK_PER_THREAD];
+#pragma unroll
+        for (int r = 0; r < CHUNK_PER_THREAD; ++r) {
+          const uint32_t x = global_index(c, tid + BATCH_THREADS * r);
+          v[r] = f2{0.0f, 0.0f};
+          if (!(x & unreached)) v[r] = slot[x];
+        }
+#pragma unroll
+        for (int r = 0; r < CHUNK_PER_THREAD; ++r) chunk[lpad(tid + BATCH_THREADS * r)] = v[r];
+      }
+      __syncthreads();
+      cu32 w = first_word;
+      for (uint32_t i = 0; i < num_instr; ++i) {
+        const uint32_t w0 = w[0], op = w0 & 0xffu;
+        if (op == BI_GATES) {
+          const uint32_t npos = (w0 >> 8) & 0xffu;
+          switch (npos) {
+            case 1: gate_pass<1, BI_GATES>(c, w, tid); break;
+            case 2: gate_pass<2, BI_GATES>(c, w, tid); break;
+            case 3: gate_pass<3, BI_GATES>(c, w, tid); break;
+            default: gate_pass<4, BI_GATES>(c, w, tid); break;
+          }
+          w += 4 + 2 * (((w0 >> 16) & 0xffu) + (w0 >> 24)) + BATCH_GATE_WORDS * npos;
+        } else if (op == BI_GATES_REAL || op == BI_GATES_REAL_PRE) {
+          // the planner emits BI_GATES_REAL for 1..4 positions, BI_GATES_REAL_PRE for 2..4 (for one
+          // position with both tables the complex form is cheaper)
+          const uint32_t npos = (w0 >> 8) & 0xffu;
+          if (op == BI_GATES_REAL) {
+            switch (npos) {
+              case 1: gate_pass<1, BI_GATES_REAL>(c, w, tid); break;
+              case 2: gate_pass<2, BI_GATES_REAL>(c, w, tid); break;
+              case 3: gate_pass<3, BI_GATES_REAL>(c, w, tid); break;
+              default: gate_pass<4, BI_GATES_REAL>(c, w, tid); break;
+            }
+          } else {
+            switch (npos) {
+              case 2: gate_pass<2, BI_GATES_REAL_PRE>(c, w, tid); break;
+              case 3: gate_pass<3, BI_GATES_REAL_PRE>(c, w, tid); break;
+              default: gate_pass<4, BI_GATES_REAL_PRE>(c, w, tid); break;
+            }
+          }
+          w += 4 + 2 * (((w0 >> 16) & 0xffu) + (w0 >> 24)) + BATCH_REAL_WORDS * npos +
+               2 * (1u << npos) * (op == BI_GATES_REAL_PRE ? 2u : 1u);
+        } else {
+          sign_pass(c, w, tid);
+          w += 1 + 2 * ((w0 >> 16) & 0xffffu);
+        }
+        __syncthreads();
+      }
+      if (flags & BS_ZZ) {
+        const uint32_t bonds = n > 1 ? (1u << (n - 1)) - 1u : 0u;
+        for (uint32_t j = tid; j < csize; j += BATCH_THREADS) {
+          const uint32_t x = global_index(c, j);
+          const f2 v = chunk[lpad(j)];
+          const double p = (double)v.re * (double)v.re + (double)v.im * (double)v.im;
+          const uint32_t d = (x ^ (x >> 1)) & bonds;
+          acc += p * (zz[d & 255u] + zz[256 + ((d >> 8) & 255u)] + zz[512 + (d >> 16)]);
+        }
+      }
+      for (uint32_t mx = measure_x; mx; mx &= mx - 1) {
+        const uint32_t pos = __builtin_ctz(mx);
+        const double h2 = 2.0 * h[S->local[pos]];
+        for (uint32_t g = tid; g < (csize >> 1); g += BATCH_THREADS) {
+          const uint32_t j0 = ((g >> pos) << (pos + 1)) | (g & ((1u << pos) - 1u));
+          const f2 a0 = chunk[lpad(j0)], a1 = chunk[lpad(j0 | (1u << pos))];
+          acc += h2 * ((double)a0.re * (double)a1.re + (double)a0.im * (double)a1.im);
+        }
+      }
+      if (flags & BS_STORE) {
+        f2 v[CHUNK_PER_THREAD];  // (full chunks, as for the loads)
+#pragma unroll
+        for (int r = 0; r < CHUNK_PER_THREAD; ++r) v[r] = chunk[lpad(tid + BATCH_THREADS * r)];
+#pragma unroll
+        for (int r = 0; r < CHUNK_PER_THREAD; ++r) slot[global_index(c, tid + BATCH_THREADS * r)] = v[r];
+      }
       __syncthreads();
     }
-    if (tid == 0) {
+
+    const uint32_t mine = items[k].partial;
+    if (mine == BATCH_NO_PARTIAL) continue;
+    // fixed-shape tree over the workgroup: the partial does not depend on timing
+    auto tree = [&](double v) {
+      red[tid] = v;
+      __syncthreads();
+      for (uint32_t half = BATCH_THREADS / 2; half > 0; half >>= 1) {
+        if (tid < half) red[tid] += red[tid + half];
+        __syncthreads();
+      }
+    };
+    tree(acc);
+    const uint32_t np = circuits[ci].num_partials, first = circuits[ci].first_partial;
+    bool last = np == 1;
+    if (np > 1) {
+      if (tid == 0) {
+        // published before the count goes down, and the others' read after it reached zero
+        __hip_atomic_store(P.partials + mine, red[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        *last_item =
+            __hip_atomic_fetch_sub(P.remaining + ci, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) == 1u ? 1u : 0u;
+      }
+      __syncthreads();
+      last = __builtin_amdgcn_readfirstlane(*last_item) != 0;
+      if (last) {
+        double sum = 0.0;
+        for (uint32_t i = tid; i < np; i += BATCH_THREADS)
+          sum += __hip_atomic_load(P.partials + first + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        tree(sum);
+      }
+    }
+    if (last && tid == 0) {
       P.energies[ci] = red[0];
       P.t_end[ci] = (uint64_t)wall_clock64();
     }
@@ -407,21 +436,22 @@ __global__ __launch_bounds__(BATCH_THREADS, BATCH_WAVES_PER_SIMD) void k_batch(b
   }
 }
 
-__global__ void k_batch_reset(uint32_t* counter) {
-  if (threadIdx.x == 0) *counter = 0u;
+__global__ __launch_bounds__(256) void k_batch_reset(batch_launch P, uint32_t* counters, uint32_t num_counters) {
+  const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+  if (i < num_counters) counters[i] = 0u;
+  if (i < P.num_circuits) P.remaining[i] = P.circuits[i].num_partials;
 }
 
 }  // namespace
 
-size_t batch_lds_bytes() {
-  return sizeof(f2) * BATCH_CHUNK_PADDED + 2 * 128 * sizeof(uint32_t) + ZZ_TABLES * 256 * sizeof(double) + 4;
+int launch_batch_reset(const batch_launch& L, uint32_t* counters, uint32_t num_counters, void* stream) {
+  const uint32_t items = std::max(num_counters, L.num_circuits);
+  hipLaunchKernelGGL(k_batch_reset, dim3((items + 255) / 256), dim3(256), 0, as_stream(stream), L, counters,
+                     num_counters);
+  return check_launch("batch reset");
 }
 
-int configure_batch() { return BRK_OK; }  // static LDS: nothing to opt in to
-
 int launch_batch(const batch_launch& L, unsigned grid, void* stream) {
-  hipLaunchKernelGGL(k_batch_reset, dim3(1), dim3(64), 0, as_stream(stream), L.counter);
-  if (int s = check_launch("batch queue reset")) return s;
   hipLaunchKernelGGL(k_batch, dim3(grid), dim3(BATCH_THREADS), 0, as_stream(stream), L);
   return check_launch("batch");
 }

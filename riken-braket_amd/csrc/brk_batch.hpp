@@ -3,10 +3,23 @@
 //
 // A batch is a list of small circuits.  Each circuit is compiled into stages;
 // a stage names up to BATCH_MAX_LOCAL "local" qubits.  The kernel walks the
-// 2^(n-L) chunks of the stage: a chunk is the 2^L amplitudes whose non-local
-// index bits are fixed; it is staged in LDS, every instruction of the stage is
-// applied to it there, and it is written back.  A circuit with n <= L has a
-// single stage whose one chunk is the whole state: it never leaves LDS.
+// chunks of the stage: a chunk is the 2^L amplitudes whose non-local index bits
+// are fixed; it is staged in LDS, every instruction of the stage is applied to
+// it there, and it is written back.  A circuit with n <= L has a single stage
+// whose one chunk is the whole state: it never leaves LDS.
+//
+// A circuit starts from |0...0>, so before a stage only amplitudes whose index
+// bits lie in the local qubits of the stages so far (`reached`) can differ from
+// zero.  A stage's gates act within its chunks, so chunks with another index bit
+// set stay zero and are left out, and the loads take such amplitudes as zero
+// without reading them (nothing ever wrote them).  The first stage is one chunk.
+//
+// The chunks of one stage are independent; a stage needs all chunks of the one
+// before.  Stages run level by level: one launch runs stage k of every circuit
+// (of a round, see host/batch.cpp) as a queue of items, each a few chunks of one
+// circuit's stage, so that a few large circuits fill the device too (24 circuits
+// of 13..19 qubits: 0.30 ms; one workgroup per circuit and all chunks: 7.4 ms.
+// 1024 of 10..20 qubits: 5.4 against 16.9 ms, the time of one 20-qubit circuit).
 #pragma once
 
 #include <cstdint>
@@ -71,40 +84,50 @@ struct batch_stage {
   uint8_t local[16];       // qubit at local position p (ascending), p < L
   uint32_t L;              // local qubits
   uint32_t flags;
-  uint32_t nonlocal_mask;  // global index bits enumerated by the chunk counter
+  uint32_t chunk_mask;     // global index bits enumerated by the chunk counter: reached, not local
+  uint32_t reached;        // index bits that can be set before the stage (chunk_mask and local bits)
   uint32_t measure_x;      // local positions p whose h_(local[p]) <X> is added (FP64)
   uint32_t first_word;     // instruction stream offset
   uint32_t num_instr;
-  uint32_t pad[2];
+  uint32_t pad;
 };
 
 struct batch_circuit {
+  uint64_t slot;           // first element of the state in the slots (circuits with several stages)
   uint32_t n;
-  uint32_t num_stages;
-  uint32_t first_stage;
   uint32_t ham_offset;     // J[0..n-2] then h[0..n-1] in the Hamiltonian array
+  uint32_t first_partial;  // energy partials of its items, in item order
+  uint32_t num_partials;
 };
+
+// Chunks [first_chunk, first_chunk + num_chunks) of one stage of one circuit.
+struct batch_item {
+  uint32_t circuit, stage, first_chunk, num_chunks;
+  uint32_t partial;        // energy partial it writes, or BATCH_NO_PARTIAL
+  uint32_t first;          // 1: the circuit's first item
+};
+constexpr uint32_t BATCH_NO_PARTIAL = 0xffffffffu;
 
 struct batch_launch {
   const batch_circuit* circuits;
   const batch_stage* stages;
   const uint32_t* words;
   const double* ham;
-  const uint32_t* order;   // circuit indices, most expensive first
+  const batch_item* items;  // of this launch, most expensive first
+  uint32_t num_items;
   uint32_t num_circuits;
-  uint32_t* counter;       // work queue head (zeroed by the reset kernel before each launch)
-  void* slots;             // complex64 [grid][slot_elems]; null when no circuit needs more than one stage
-  uint64_t slot_elems;
+  uint32_t* counter;       // work queue head of this launch (zeroed by the reset kernel)
+  uint32_t* remaining;     // [num_circuits] partials still to come (set by the reset kernel)
+  double* partials;
+  void* slots;             // complex64; null when no circuit needs more than one stage
   double* energies;        // [num_circuits]
   uint64_t* t_start;       // wall-clock ticks when the circuit was taken from the queue
   uint64_t* t_end;         // ... and when its energy was written
 };
 
-// LDS bytes the kernel needs (chunk + index tables + ZZ energy tables + queue slot).
-size_t batch_lds_bytes();
-// Lets the persistent kernel use more than 64 KiB of dynamic LDS (call once per device, outside capture).
-int configure_batch();
-// Enqueues the queue reset and the persistent kernel on `stream` (capturable: no memset nodes).
+// Enqueues the reset of `num_counters` queue heads and of every circuit's remaining partials, then
+// (launch_batch) one persistent launch over L.items, on `stream` (capturable: no memset nodes).
+int launch_batch_reset(const batch_launch& L, uint32_t* counters, uint32_t num_counters, void* stream);
 int launch_batch(const batch_launch& L, unsigned grid, void* stream);
 
 }  // namespace brk

@@ -1,6 +1,6 @@
 // Batching form, host side: compiles a list of small circuits into the stage
 // programs of csrc/brk_batch.hpp, uploads them once, and runs the persistent
-// kernel as a captured HIP graph (queue reset + one persistent launch).
+// kernel as a captured HIP graph (a reset, then one launch per stage level).
 //
 // Per circuit:
 //  1. ops -> planner ops: uncontrolled single-qubit ops become 2x2 gates
@@ -20,6 +20,11 @@
 //     one product matrix per position);
 //     a run of sign masks becomes popcount terms (a CZ ladder is one term)
 //     folded into the neighbouring gate group, or a pass of its own.
+//
+// Launches: the states of circuits with several stages live in slots of a buffer
+// of at most BATCH_WG_PER_CU per CU of the largest one's size; circuits beyond
+// that take the slots over in a further round.  A round's launch k runs stage k
+// of its circuits as items of a few chunks; circuits of one stage join the first.
 #include "circuit.hpp"
 #include "brk_batch.hpp"
 
@@ -403,13 +408,13 @@ struct brk_batch {
   std::vector<brk::batch_stage> stages;
   std::vector<uint32_t> words;
   std::vector<double> ham;
-  std::vector<uint32_t> order;
-  unsigned max_multi_n = 0;  // largest n with more than one stage (0: none)
+  std::vector<uint32_t> first_stage;  // per circuit
+  std::vector<double> instr_cost;  // per stage: relative time of a chunk
+  unsigned max_multi_n = 0;        // largest n with more than one stage (0: none)
 
   // device side, created on the first run
   int device = -1;
-  unsigned grid = 0;
-  void* d_program = nullptr;  // circuits, stages, words, ham, order, counter, energies, t_start, t_end
+  void* d_program = nullptr;  // circuits, stages, words, ham, items, counters, remaining, partials, energies, times
   void* d_slots = nullptr;
   brk::batch_launch launch{};
   hipStream_t stream = nullptr;
@@ -435,6 +440,87 @@ size_t aligned_bytes(size_t count) {
   return (count * sizeof(T) + 255) & ~(size_t)255;
 }
 
+// The launches of a batch: items of every round's stage levels (see the top of this file).
+struct schedule {
+  struct range {
+    size_t first, count;
+  };
+  std::vector<brk::batch_item> items;
+  std::vector<range> launches;
+  size_t num_partials = 0;
+  uint64_t slot_elems = 0;
+};
+
+schedule make_schedule(brk_batch& b, unsigned workgroups, uint64_t room) {
+  schedule out;
+  const size_t nc = b.circuits.size();
+  // rounds: the circuits with several stages, largest first, while their states fit in the room
+  std::vector<uint32_t> multi;
+  for (uint32_t c = 0; c < nc; ++c)
+    if (b.plans[c].stages.size() > 1) multi.push_back(c);
+  std::stable_sort(multi.begin(), multi.end(), [&](uint32_t x, uint32_t y) { return b.plans[x].n > b.plans[y].n; });
+  std::vector<std::vector<uint32_t>> rounds(1);
+  uint64_t used = 0;
+  for (uint32_t c : multi) {
+    const uint64_t elems = 1ull << b.plans[c].n;
+    if (used + elems > room) {
+      rounds.emplace_back();
+      used = 0;
+    }
+    b.circuits[c].slot = used;
+    used += elems;
+    out.slot_elems = std::max(out.slot_elems, used);
+    rounds.back().push_back(c);
+  }
+  for (uint32_t c = 0; c < nc; ++c)
+    if (b.plans[c].stages.size() == 1) rounds[0].push_back(c);
+
+  struct entry {
+    uint32_t circuit, stage, chunks;
+    double cost;  // of a chunk
+  };
+  std::vector<std::vector<uint32_t>> partial_items(nc);  // the circuit's items that write a partial
+  for (const auto& round : rounds) {
+    size_t levels = 0;
+    for (uint32_t c : round) levels = std::max(levels, b.plans[c].stages.size());
+    for (size_t k = 0; k < levels; ++k) {
+      std::vector<entry> entries;
+      uint64_t chunks = 0;
+      for (uint32_t c : round) {
+        if (k >= b.plans[c].stages.size()) continue;
+        const uint32_t stage = b.first_stage[c] + (uint32_t)k;
+        const uint32_t count = 1u << __builtin_popcount(b.stages[stage].chunk_mask);
+        entries.push_back({c, stage, count, b.instr_cost[stage]});
+        chunks += count;
+      }
+      // enough items to even out the workgroups' times, few enough that the setup of an item (its
+      // tables and the queue) stays a small part of it
+      const uint32_t per = (uint32_t)std::min<uint64_t>(16, std::max<uint64_t>(1, chunks / (16ull * workgroups)));
+      std::stable_sort(entries.begin(), entries.end(), [&](const entry& x, const entry& y) {
+        return x.cost * std::min(x.chunks, per) > y.cost * std::min(y.chunks, per);
+      });
+      const size_t first = out.items.size();
+      for (const entry& e : entries) {
+        const brk::batch_stage& bs = b.stages[e.stage];
+        const bool last_stage = k + 1 == b.plans[e.circuit].stages.size();
+        for (uint32_t c = 0; c < e.chunks; c += per) {
+          brk::batch_item it{e.circuit, e.stage, c, std::min(per, e.chunks - c), brk::BATCH_NO_PARTIAL, k == 0};
+          if (last_stage || bs.measure_x || (bs.flags & brk::BS_ZZ))
+            partial_items[e.circuit].push_back((uint32_t)out.items.size());
+          out.items.push_back(it);
+        }
+      }
+      out.launches.push_back({first, out.items.size() - first});
+    }
+  }
+  for (size_t c = 0; c < nc; ++c) {
+    b.circuits[c].first_partial = (uint32_t)out.num_partials;
+    b.circuits[c].num_partials = (uint32_t)partial_items[c].size();
+    for (uint32_t i : partial_items[c]) out.items[i].partial = (uint32_t)out.num_partials++;
+  }
+  return out;
+}
+
 int ensure_device(brk_batch* b) {
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess) return brk::fail(BRK_ERR_HIP, "hipGetDevice failed");
@@ -442,12 +528,25 @@ int ensure_device(brk_batch* b) {
     if (dev != b->device) return brk::fail(BRK_ERR_INVALID_ARGUMENT, "batch was set up on device %d", b->device);
     return BRK_OK;
   }
+  int cus = 0, rate_khz = 0;
+  if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
+    return brk::fail(BRK_ERR_HIP, "cannot read the CU count");
+  if (hipDeviceGetAttribute(&rate_khz, hipDeviceAttributeWallClockRate, dev) != hipSuccess || rate_khz <= 0)
+    return brk::fail(BRK_ERR_HIP, "cannot read the wall-clock rate");
+  b->tick_ms = 1.0 / (double)rate_khz;
   const size_t nc = b->circuits.size();
+  const unsigned workgroups = (unsigned)cus * brk::BATCH_WG_PER_CU;
+  const uint64_t slot_elems =
+      b->max_multi_n ? std::min<uint64_t>(workgroups, nc) << b->max_multi_n : 0;  // room for the slots
+  schedule plan = make_schedule(*b, workgroups, slot_elems);
   const size_t sizes[] = {aligned_bytes<brk::batch_circuit>(nc), aligned_bytes<brk::batch_stage>(b->stages.size()),
                           aligned_bytes<uint32_t>(std::max<size_t>(1, b->words.size())),
-                          aligned_bytes<double>(std::max<size_t>(1, b->ham.size())), aligned_bytes<uint32_t>(nc),
-                          aligned_bytes<uint32_t>(1), aligned_bytes<double>(nc), aligned_bytes<uint64_t>(nc),
-                          aligned_bytes<uint64_t>(nc)};
+                          aligned_bytes<double>(std::max<size_t>(1, b->ham.size())),
+                          aligned_bytes<brk::batch_item>(plan.items.size()),
+                          aligned_bytes<uint32_t>(plan.launches.size()), aligned_bytes<uint32_t>(nc),
+                          aligned_bytes<double>(plan.num_partials), aligned_bytes<double>(nc),
+                          aligned_bytes<uint64_t>(nc), aligned_bytes<uint64_t>(nc)};
+  constexpr int PARTS = sizeof(sizes) / sizeof(sizes[0]);
   size_t total = 0;
   for (size_t s : sizes) total += s;
   if (hipMalloc(&b->d_program, total) != hipSuccess) {
@@ -455,29 +554,20 @@ int ensure_device(brk_batch* b) {
     return brk::fail(BRK_ERR_OUT_OF_MEMORY, "cannot allocate %zu bytes for the batch program", total);
   }
   char* base = static_cast<char*>(b->d_program);
-  char* ptr[9];
-  for (int i = 0; i < 9; ++i) {
+  char* ptr[PARTS];
+  for (int i = 0; i < PARTS; ++i) {
     ptr[i] = base;
     base += sizes[i];
   }
-  const void* host[] = {b->circuits.data(), b->stages.data(), b->words.data(), b->ham.data(), b->order.data()};
+  const void* host[] = {b->circuits.data(), b->stages.data(), b->words.data(), b->ham.data(), plan.items.data()};
   const size_t bytes[] = {nc * sizeof(brk::batch_circuit), b->stages.size() * sizeof(brk::batch_stage),
-                          b->words.size() * sizeof(uint32_t), b->ham.size() * sizeof(double), nc * sizeof(uint32_t)};
+                          b->words.size() * sizeof(uint32_t), b->ham.size() * sizeof(double),
+                          plan.items.size() * sizeof(brk::batch_item)};
   for (int i = 0; i < 5; ++i)
     if (bytes[i] && hipMemcpy(ptr[i], host[i], bytes[i], hipMemcpyHostToDevice) != hipSuccess)
       return brk::fail(BRK_ERR_HIP, "uploading the batch program failed");
-
-  int cus = 0, rate_khz = 0;
-  if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
-    return brk::fail(BRK_ERR_HIP, "cannot read the CU count");
-  if (hipDeviceGetAttribute(&rate_khz, hipDeviceAttributeWallClockRate, dev) != hipSuccess || rate_khz <= 0)
-    return brk::fail(BRK_ERR_HIP, "cannot read the wall-clock rate");
-  b->tick_ms = 1.0 / (double)rate_khz;
-  b->grid = (unsigned)std::min<size_t>((size_t)cus * brk::BATCH_WG_PER_CU, nc);
-  uint64_t slot_elems = 0;
-  if (b->max_multi_n) {
-    slot_elems = 1ull << b->max_multi_n;
-    const size_t slot_bytes = (size_t)b->grid * slot_elems * 8;
+  if (plan.slot_elems) {
+    const size_t slot_bytes = (size_t)plan.slot_elems * 8;
     if (hipMalloc(&b->d_slots, slot_bytes) != hipSuccess) {
       b->d_slots = nullptr;
       return brk::fail(BRK_ERR_OUT_OF_MEMORY, "cannot allocate %zu bytes of batch state slots", slot_bytes);
@@ -488,25 +578,31 @@ int ensure_device(brk_batch* b) {
   L.stages = reinterpret_cast<const brk::batch_stage*>(ptr[1]);
   L.words = reinterpret_cast<const uint32_t*>(ptr[2]);
   L.ham = reinterpret_cast<const double*>(ptr[3]);
-  L.order = reinterpret_cast<const uint32_t*>(ptr[4]);
   L.num_circuits = (uint32_t)nc;
-  L.counter = reinterpret_cast<uint32_t*>(ptr[5]);
+  L.remaining = reinterpret_cast<uint32_t*>(ptr[6]);
+  L.partials = reinterpret_cast<double*>(ptr[7]);
   L.slots = b->d_slots;
-  L.slot_elems = slot_elems;
-  L.energies = reinterpret_cast<double*>(ptr[6]);
-  L.t_start = reinterpret_cast<uint64_t*>(ptr[7]);
-  L.t_end = reinterpret_cast<uint64_t*>(ptr[8]);
+  L.energies = reinterpret_cast<double*>(ptr[8]);
+  L.t_start = reinterpret_cast<uint64_t*>(ptr[9]);
+  L.t_end = reinterpret_cast<uint64_t*>(ptr[10]);
+  const auto* items = reinterpret_cast<const brk::batch_item*>(ptr[4]);
+  auto* counters = reinterpret_cast<uint32_t*>(ptr[5]);
 
   if (hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking) != hipSuccess)
     return brk::fail(BRK_ERR_HIP, "cannot create the batch stream");
   if (hipEventCreateWithFlags(&b->ev_in, hipEventDisableTiming) != hipSuccess ||
       hipEventCreate(&b->ev_begin) != hipSuccess || hipEventCreate(&b->ev_end) != hipSuccess)
     return brk::fail(BRK_ERR_HIP, "cannot create the batch events");
-  if (int s = brk::configure_batch()) return s;
-  // graph: queue reset + persistent kernel, captured once and replayed
+  // graph: the reset and the launches, captured once and replayed
   if (hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal) != hipSuccess)
     return brk::fail(BRK_ERR_HIP, "hipStreamBeginCapture failed");
-  const int launch_status = brk::launch_batch(L, b->grid, b->stream);
+  int launch_status = brk::launch_batch_reset(L, counters, (uint32_t)plan.launches.size(), b->stream);
+  for (size_t k = 0; !launch_status && k < plan.launches.size(); ++k) {
+    L.items = items + plan.launches[k].first;
+    L.num_items = (uint32_t)plan.launches[k].count;
+    L.counter = counters + k;
+    launch_status = brk::launch_batch(L, std::min<unsigned>(workgroups, L.num_items), b->stream);
+  }
   hipGraph_t graph = nullptr;
   const hipError_t end = hipStreamEndCapture(b->stream, &graph);
   if (launch_status) {
@@ -574,7 +670,6 @@ int brk_batch_create(const brk_circuit* const* circuits, unsigned num_circuits, 
   *out = nullptr;
   if (!circuits || num_circuits == 0) return fail(BRK_ERR_INVALID_ARGUMENT, "empty batch");
   auto* b = new brk_batch();
-  std::vector<double> cost(num_circuits);
   for (unsigned i = 0; i < num_circuits; ++i) {
     const brk_circuit* c = circuits[i];
     if (!c) {
@@ -600,11 +695,10 @@ int brk_batch_create(const brk_circuit* const* circuits, unsigned num_circuits, 
 
     brk::batch_circuit bc{};
     bc.n = n;
-    bc.num_stages = (uint32_t)pc.stages.size();
-    bc.first_stage = (uint32_t)b->stages.size();
+    b->first_stage.push_back((uint32_t)b->stages.size());
     bc.ham_offset = (uint32_t)b->ham.size();
     b->ham.insert(b->ham.end(), pc.ham.begin(), pc.ham.end());
-    double work = 0.0;
+    uint32_t reached = 0;  // index bits that can be set: the local qubits of the stages stored so far
     for (size_t s = 0; s < pc.stages.size(); ++s) {
       const planned_stage& st = pc.stages[s];
       // the kernel moves the chunks of a multi-stage circuit as full chunks
@@ -620,24 +714,22 @@ int brk_batch_create(const brk_circuit* const* circuits, unsigned num_circuits, 
         bs.local[p] = (uint8_t)st.local[p];
         local_mask |= 1u << st.local[p];
       }
-      bs.nonlocal_mask = all_qubits(n) & ~local_mask;
+      bs.reached = reached;
+      bs.chunk_mask = reached & ~local_mask;
       bs.first_word = (uint32_t)b->words.size();
       bool changes = false;
       for (const pop& o : st.ops) changes |= o.kind == BRK_BATCH_GATE || o.kind == BRK_BATCH_SIGN;
       bs.num_instr = emit_stage(st, b->words, bs.measure_x, bs.flags);
       if (s == 0) bs.flags |= brk::BS_INIT;
       if (s + 1 < pc.stages.size() && (changes || s == 0)) bs.flags |= brk::BS_STORE;
+      if (bs.flags & brk::BS_STORE) reached |= local_mask;
       b->stages.push_back(bs);
-      work += (double)(1ull << n) * (bs.num_instr + 3);
+      b->instr_cost.push_back((double)(bs.num_instr + 3) * (double)(1u << bs.L));
     }
     if (pc.stages.size() > 1) b->max_multi_n = std::max(b->max_multi_n, n);
-    cost[i] = work;
     b->circuits.push_back(bc);
     b->plans.push_back(std::move(pc));
   }
-  b->order.resize(num_circuits);
-  for (unsigned i = 0; i < num_circuits; ++i) b->order[i] = i;
-  std::stable_sort(b->order.begin(), b->order.end(), [&](uint32_t x, uint32_t y) { return cost[x] > cost[y]; });
   *out = b;
   return BRK_OK;
 }

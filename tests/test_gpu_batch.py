@@ -138,6 +138,38 @@ def test_independent_batches_share_nothing():
         assert abs(eb1[i] - plain_energy(n, ops, J, h)) < E_TOL
 
 
+def test_slots_taken_over_by_a_second_round():
+    # 600 two-stage circuits of one size: slots for 512 (two workgroups per CU), so 88 run in a second round,
+    # with single-stage circuits beside them
+    items = W.batch_ansatz(num_circuits=600, min_qubits=14, max_qubits=14, layers=2, seed=31)
+    items += W.batch_ansatz(num_circuits=5, min_qubits=9, max_qubits=13, layers=2, seed=32)
+    note("gpu batch: two rounds")
+    b = brk.Batch(items)
+    e = b.run()
+    assert np.array_equal(b.run(), e)
+    for i in (0, 87, 88, 300, 511, 512, 599, 600, 604):
+        n, ops, J, h = items[i]
+        assert abs(e[i] - plain_energy(n, ops, J, h)) < E_TOL, (i, n)
+
+
+@pytest.mark.parametrize("qubits", [(0, 18), (17,), (3, 4, 9, 14, 16, 18), ()])
+def test_qubits_no_gate_reaches(qubits):
+    # gates and Hamiltonian terms on some qubits only: the others stay |0>, their amplitudes are never stored
+    n = 19
+    rng = np.random.default_rng(40 + len(qubits))
+    ops = []
+    for _ in range(3):
+        for q in qubits:
+            ops.append(("U3", (q,), (), tuple(float(x) for x in rng.uniform(-3, 3, 3))))
+        for a in qubits:
+            ops.append(("Z", (a,), ((a + 5) % n,), ()))
+    note(f"gpu batch: gates on {qubits} of {n}")
+    J, h = rng.uniform(-1, 1, n - 1), rng.uniform(-1, 1, n)
+    for hh in (h, np.zeros(n), np.where(np.isin(np.arange(n), qubits), h, 0.0)):
+        e = brk.Batch([(n, ops, J, hh)]).run()
+        assert abs(e[0] - plain_energy(n, ops, J, hh)) < E_TOL, (qubits, e[0])
+
+
 @pytest.mark.slow
 def test_full_workload_sampled():
     # the batching workload: 4096 circuits, 10..20 qubits, 8 layers
