@@ -427,8 +427,8 @@ int brk_circuit_run_timed(const brk_circuit* circuit, void* first, int dtype, un
 /* Gate blocks: runs of consecutive gates applied per chunk of the state    */
 /* held in LDS (2^12 amplitudes for complex<double>, 2^13 for               */
 /* complex<float>), each gate with the per-gate kernels' arithmetic, so the */
-/* amplitudes are bit-identical to brk_circuit_run's.  One HBM read and     */
-/* write per block instead of per gate.  Replaces the gate application of   */
+/* amplitudes are bit-identical to one gate call after another.  One HBM    */
+/* read and write per block instead of per gate.  Replaces the gate application of   */
 /* bra's BEGIN/END FUSION (bra/src/state.cpp:2193-2217,                     */
 /* bra/src/nompi_state.cpp:1282-1357) and of ket's cache-aware gate         */
 /* functions (ket/include/ket/gate/detail/gate_bitmasks.hpp:587-2134).      */
@@ -444,7 +444,6 @@ typedef struct brk_block_plan brk_block_plan;
    brk_circuit_run.  Planning needs no device. */
 int brk_block_plan_create(const brk_circuit* circuit, int dtype, const unsigned* permutation,
                           brk_block_plan** out);
-/* Call after the work of brk_block_plan_run on its stream has completed. */
 int brk_block_plan_destroy(brk_block_plan* plan);
 int brk_block_plan_num_steps(const brk_block_plan* plan, unsigned* num_steps);
 /* Step i covers ops [first_op, first_op + num_ops) of the circuit; num_local
@@ -453,10 +452,13 @@ int brk_block_plan_num_steps(const brk_block_plan* plan, unsigned* num_steps);
 int brk_block_plan_step(const brk_block_plan* plan, unsigned i, unsigned* first_op, unsigned* num_ops,
                         unsigned* num_local, unsigned* local_qubits);
 int brk_block_plan_final_permutation(const brk_block_plan* plan, unsigned* permutation);
-/* Runs the plan on a state of 2^num_qubits amplitudes of the plan's dtype;
-   the first run uploads the block programs to the current device. */
+/* Runs the plan on a state of 2^num_qubits amplitudes of the plan's dtype.
+   Consecutive steps share a launch where the bits their gates flip fit in one
+   chunk (control bits and diagonal gates may lie outside it).  The block
+   programs travel in the launches' arguments: nothing is uploaded or kept on
+   the device. */
 int brk_block_plan_run(brk_block_plan* plan, void* first, void* stream);
-/* Plans, runs and destroys in one call (synchronises the stream); the
+/* Plans and runs in one call (synchronises the stream); the
    permutation is updated as by brk_circuit_run. */
 int brk_circuit_run_blocked(const brk_circuit* circuit, void* first, int dtype, unsigned* permutation,
                             void* stream);

@@ -5,11 +5,12 @@
 // code that computes the plain kernels' coefficients, so a block applies each
 // gate with the plain path's arithmetic and gives bit-identical amplitudes.
 // The planner (host/block.cpp) turns the descriptions of one block into a
-// block_program over local bit positions; the kernel (brk_gates.hip) loads
+// program over local bit positions; the kernel (brk_gates.hip) loads
 // the 2^L amplitudes of a chunk, applies the program in LDS and stores them.
 // Plain C++ only: included by host code compiled without HIP.
 #pragma once
 
+#include <cstddef>
 #include <cstdint>
 
 namespace brk {
@@ -42,11 +43,97 @@ struct gate_desc {
 int describe_physical_op(int code, const unsigned* targets, unsigned num_targets, const unsigned* controls,
                          unsigned num_controls, const double* params, gate_desc* out);
 
-// A gate of a block with its masks over local bit positions (bit r of a
-// chunk index <-> physical qubit pos[r]).  The gate visits only the local
-// indices it acts on: item v -> j = v with zeros inserted at ins[0..nins)
-// (ascending: the pair bit and the cond bits), then the cond bits set.
+// What a block's kernel does for a gate: the described mode, with a 2x2 matrix told apart by the
+// exact zeros of its coefficients (the forms of pair_math).
+enum block_kind {
+  BLOCK_KIND_H = 0, BLOCK_KIND_SWAP = 1, BLOCK_KIND_MATRIX = 2, BLOCK_KIND_ESWAP = 3, BLOCK_KIND_DIAG = 4,
+  BLOCK_KIND_REAL = 5,   // a real 2x2 (RY, EY); off-diagonal entries under the sign mask, if any
+  BLOCK_KIND_X = 6,      // [[r, i s], [i s', r']] (RX, EX); the same
+  BLOCK_KIND_NEGATE = 7, // diagonal with u = (-1, -1) (Z, CZ): an exact negation on cond
+  BLOCK_KIND_SIGNED = 8  // (kernels: any 2x2 under a sign mask)
+};
+
+// A gate of a block with its masks over local bit positions (bit r of a chunk index <-> physical
+// qubit pos[r]).  Only the bits a pair gate flips have to be local: control bits and diagonal
+// parity bits outside the chunk are the same for all its amplitudes (outer_cond: the gate acts on
+// the chunk only where all these physical bits are set; outer_zmask: their parity joins zmask's).
+// A single pass visits only the local indices the gate acts on: item v -> v with zeros inserted at
+// the bits of `inserted` (the pair bit and the cond bits), then the cond bits set.
 struct block_op {
+  uint8_t kind, pair_bit;
+  uint8_t group_flip, group_pair;   // register segments: flip and pair bit over the group index
+  uint8_t group_zmask, group_cond;  // register segments: the masks' parts over the group index
+                                    // (zmask, a pair gate's sign; cond),
+  uint16_t coef;                    // first of its coefficients (none for H, SWAP, NEGATE)
+  uint16_t flip, cond, sign, zmask;
+  uint16_t inserted;
+  uint16_t thread_cond, thread_zmask, pad;  // ... and over the other local bits
+  uint64_t outer_cond, outer_zmask;
+};
+static_assert(sizeof(block_op) == 40, "read as five 64-bit words");
+
+// A pass over the chunk.  A segment pass gives every thread one group of 2^(L - 9)
+// amplitudes -- local indices that differ only in the bits group[0..] -- in registers
+// and applies several gates to it: diagonal gates, and pair gates whose flipped bits
+// are group bits.  Gates that only move amplitudes (X, CNOT, SWAP, local swaps) on any
+// local bits come after them (num_moves ops): the segment writes its amplitudes to the
+// indices they move to.  A single pass applies one gate to the chunk in LDS with a
+// strided loop.
+enum block_pass_kind { BLOCK_PASS_SEGMENT = 0, BLOCK_PASS_SINGLE = 1 };
+enum block_pass_flags {
+  BLOCK_PASS_LOADS = 1,  // the first pass: its groups come straight from the state
+  BLOCK_PASS_STORES = 2  // the last pass: its groups go straight to the state
+};
+struct block_pass {
+  uint8_t kind, num_ops, num_moves, flags;
+  uint8_t group[4];  // ascending local bits of the group (L - 9 of them)
+  uint16_t first_op, pad;
+};
+
+struct block_header {
+  uint32_t num_ops;
+  uint32_t num_local;   // L
+  uint32_t num_passes;  // they follow the header
+  uint16_t ops_at, coefs_at;  // byte offsets from the header: the ops, the coefficients (double)
+  uint8_t pos[16];      // ascending physical qubits of the local bits
+};
+static_assert(sizeof(block_header) == 32 && sizeof(block_pass) == 12, "packed");
+
+// A block's program with room for every block.
+constexpr int BLOCK_COEFS = 8;  // at most, per op
+struct block_program {
+  block_header h;
+  block_pass passes[BLOCK_MAX_OPS];
+  block_op ops[BLOCK_MAX_OPS];
+  double coefs[BLOCK_COEFS * BLOCK_MAX_OPS + BLOCK_COEFS];  // (a kernel reads 8 from any op's first one)
+};
+
+// A program packed for a launch's kernel arguments: header, passes, ops and coefficients one after
+// the other.  The planner closes a block before its program outgrows them.  No device memory holds
+// the program, so a run allocates, uploads and keeps nothing, and its launches can be captured.
+constexpr size_t BLOCK_ARG_BYTES = 3840;
+struct alignas(8) block_args {
+  block_header h;
+  uint8_t data[BLOCK_ARG_BYTES - sizeof(block_header)];
+};
+// Room the ops may take in the arguments, each itself, a pass and its coefficients (beside the
+// alignment of the ops and the coefficients read past the last ones).
+constexpr size_t BLOCK_ARG_ROOM =
+    BLOCK_ARG_BYTES - sizeof(block_header) - sizeof(double) - BLOCK_COEFS * sizeof(double);
+inline int block_op_coefs(const gate_desc& d) {
+  if (d.mode == BLOCK_MATRIX) return 8;
+  if (d.mode == BLOCK_ESWAP) return 4;
+  if (d.mode != BLOCK_DIAG) return 0;
+  return d.u[0] == -1.0 && d.u[1] == 0.0 && d.u[2] == -1.0 && d.u[3] == 0.0 ? 0 : 4;
+}
+inline size_t block_op_room(const gate_desc& d) {
+  return sizeof(block_op) + sizeof(block_pass) + sizeof(double) * (size_t)block_op_coefs(d);
+}
+
+// A gate of an adjoint block with its masks over local bit positions (every qubit local): item
+// v -> j = v with zeros inserted at ins[0..nins) (ascending: the pair bit and the cond bits), then
+// the cond bits set.
+struct adjoint_op {
   int32_t mode;
   uint32_t pair_bit, flip, cond, sign, zmask;
   uint32_t nins;
@@ -57,26 +144,21 @@ struct block_op {
   double u[8];
 };
 
-// A pass over the chunk in LDS.  A segment pass gives every thread one group of
-// 2^(L - 9) amplitudes -- local indices that differ only in the bits group[0..]
-// -- in registers and applies several gates to it: diagonal gates, and pair
-// gates whose flipped bits are group bits.  A single pass applies one gate
-// with the strided loop.
-enum block_pass_kind { BLOCK_PASS_SEGMENT = 0, BLOCK_PASS_SINGLE = 1 };
-struct block_pass {
+// Its passes: segments of several gates on a thread's group, and single gates.
+struct adjoint_pass {
   int32_t kind;
   uint32_t first_op, num_ops;
   uint32_t group[4];  // ascending local bits of the group (L - 9 of them)
 };
 
-struct block_program {
+struct adjoint_base {
   uint32_t num_ops;
   uint32_t num_local;                   // L
   uint32_t num_passes;
   uint32_t pos[16];                     // ascending physical qubits of the local bits
   uint64_t deposit_high[16];            // physical offset of local index k << BLOCK_THREAD_BITS
-  block_pass passes[BLOCK_MAX_OPS];
-  block_op ops[BLOCK_MAX_OPS];
+  adjoint_pass passes[BLOCK_MAX_OPS];
+  adjoint_op ops[BLOCK_MAX_OPS];
 };
 
 // Reverse sweep of the adjoint method in blocks: chunks of psi and lambda are
@@ -97,7 +179,7 @@ constexpr int ADJ_SEGMENT_GRADIENTS = 8;  // parametric ops per register segment
 //   X: D = [[0, i a], [i b, 0]], the inverse op [[r, i s], [i s', r']] (RX, EX).
 enum adjoint_grad_kind { ADJ_GRAD_GENERAL = 0, ADJ_GRAD_Z = 1, ADJ_GRAD_Y = 2, ADJ_GRAD_X = 3 };
 struct adjoint_block_program {
-  block_program base;                  // the inverse ops; their passes
+  adjoint_base base;                   // the inverse ops; their passes
   int32_t grad_slot[BLOCK_MAX_OPS];    // -1: no gradient term
   int32_t grad_kind[BLOCK_MAX_OPS];    // adjoint_grad_kind of a parametric op
   double d[BLOCK_MAX_OPS][8];          // D = (dU/dtheta) U^dagger, (re, im) of d00, d01, d10, d11
@@ -112,11 +194,10 @@ int sum_gradient_partials(const double* partials, unsigned rows, uint64_t chunks
 // Whether the adjoint gradient runs in blocks (tuning adjoint_blocks).
 bool adjoint_blocks_enabled();
 
-// A block_program for the described gates (physical qubits of an n-qubit state):
-// local qubits are their qubits, the line_bits lowest qubits, then the lowest others,
-// num_local in all.
-block_program make_block_program(const gate_desc* descs, unsigned count, unsigned n, unsigned num_local,
-                                 unsigned line_bits);
+// An adjoint block's gates (physical qubits of an n-qubit state): local qubits are their qubits,
+// the line_bits lowest qubits, then the lowest others, num_local in all.  Makes no passes.
+void make_adjoint_base(const gate_desc* descs, unsigned count, unsigned n, unsigned num_local, unsigned line_bits,
+                       adjoint_base* out);
 
 // Local qubits of a chunk for this dtype under the current tuning (block_lds).
 unsigned block_max_local(int dtype);
@@ -124,9 +205,6 @@ unsigned block_max_local(int dtype);
 unsigned block_run_qubits(int dtype);
 
 // Launches one block over a state of `size` amplitudes: 2^(n - L) workgroups.
-// `device_program` points to a block_program in device memory whose copy on
-// the host is `program`.
-int launch_block(const block_program* device_program, const block_program& program, void* first, uint64_t size,
-                 int dtype, void* stream);
+int launch_block(const block_args& program, void* first, uint64_t size, int dtype, void* stream);
 
 }  // namespace brk

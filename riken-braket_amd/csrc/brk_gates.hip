@@ -34,6 +34,7 @@
 
 #include <cmath>
 #include <complex>
+#include <type_traits>
 
 namespace brk {
 
@@ -247,10 +248,466 @@ __global__ __launch_bounds__(GATE_THREADS) void k_diag(cpx<R>* __restrict__ s, u
 // arithmetic above; one HBM read and one write per amplitude per block.
 // ---------------------------------------------------------------------------
 
-typedef const __attribute__((address_space(4))) block_program* cprogram;
+// Two workgroups of 8 waves per CU (64 KiB of LDS each): 4 waves per SIMD, at most 128 VGPRs.
+constexpr int BLOCK_WAVES_PER_SIMD = 4;
+
+typedef const __attribute__((address_space(4))) char* cbytes;
+typedef const __attribute__((address_space(4))) block_header* cheader;
+typedef const __attribute__((address_space(4))) block_pass* cpass;
+typedef const __attribute__((address_space(4))) uint64_t* cu64;
+typedef const __attribute__((address_space(4))) double* cdouble;
+
+// A program in the constant address space (uniform: scalar loads).
+struct block_view {
+  cheader h;
+  cpass passes;
+  cu64 ops;  // WORDS words each
+  cdouble coefs;
+  static constexpr int WORDS = sizeof(block_op) / sizeof(uint64_t);
+  __device__ explicit block_view(cbytes program)
+      : h((cheader)program), passes((cpass)(program + sizeof(block_header))),
+        ops((cu64)(program + ((cheader)program)->ops_at)), coefs((cdouble)(program + ((cheader)program)->coefs_at)) {}
+};
+
+// The words of a block_op, and the gate they describe with its coefficients, in registers.
+struct op_words {
+  uint64_t w[block_view::WORDS];
+  __device__ __forceinline__ uint32_t coef() const { return (uint32_t)(w[0] >> 48); }
+};
+struct block_gate {
+  uint32_t kind, pair_bit, group_flip, group_pair, group_zmask, group_cond;
+  uint32_t flip, cond, sign, zmask, inserted, thread_cond, thread_zmask;
+  uint64_t outer_cond, outer_zmask;
+  double u[8];
+};
+
+__device__ __forceinline__ op_words load_op(const block_view& v, uint32_t o) {
+  op_words r;
+#pragma unroll
+  for (int k = 0; k < block_view::WORDS; ++k) r.w[k] = v.ops[(uint64_t)o * block_view::WORDS + k];
+  return r;
+}
+__device__ __forceinline__ void load_coefs(const block_view& v, uint32_t coef, double (&u)[8]) {
+#pragma unroll
+  for (int k = 0; k < 8; ++k) u[k] = v.coefs[coef + k];
+}
+__device__ __forceinline__ block_gate decode(const op_words& r, const double (&u)[8]) {
+  auto byte = [](uint64_t w, int k) { return (uint32_t)(w >> (8 * k)) & 0xffu; };
+  auto half = [](uint64_t w, int k) { return (uint32_t)(w >> (16 * k)) & 0xffffu; };
+  block_gate g;
+  g.kind = byte(r.w[0], 0);
+  g.pair_bit = byte(r.w[0], 1);
+  g.group_flip = byte(r.w[0], 2);
+  g.group_pair = byte(r.w[0], 3);
+  g.group_zmask = byte(r.w[0], 4);
+  g.group_cond = byte(r.w[0], 5);
+  g.flip = half(r.w[1], 0);
+  g.cond = half(r.w[1], 1);
+  g.sign = half(r.w[1], 2);
+  g.zmask = half(r.w[1], 3);
+  g.inserted = half(r.w[2], 0);
+  g.thread_cond = half(r.w[2], 1);
+  g.thread_zmask = half(r.w[2], 2);
+  g.outer_cond = r.w[3];
+  g.outer_zmask = r.w[4];
+#pragma unroll
+  for (int k = 0; k < 8; ++k) g.u[k] = u[k];
+  return g;
+}
+__device__ __forceinline__ block_gate load_gate(const block_view& v, uint32_t o) {
+  const op_words r = load_op(v, o);
+  double u[8];
+  load_coefs(v, r.coef(), u);
+  return decode(r, u);
+}
+// Whether the chunk with outer bits `base` satisfies the gate's conditions outside it.
+__device__ __forceinline__ bool acts_on(const block_gate& g, uint64_t base) {
+  return (base & g.outer_cond) == g.outer_cond;
+}
+// A diagonal gate's coefficients for even and odd parity of the local index & zmask in the chunk.
+template <typename R>
+__device__ __forceinline__ void chunk_diag(const block_gate& g, uint64_t base, cpx<R>& c0, cpx<R>& c1) {
+  const bool odd = (__popcll(base & g.outer_zmask) & 1) != 0;
+  c0 = {(R)(odd ? g.u[2] : g.u[0]), (R)(odd ? g.u[3] : g.u[1])};
+  c1 = {(R)(odd ? g.u[0] : g.u[2]), (R)(odd ? g.u[1] : g.u[3])};
+}
 
 // Chunk index -> global bits outside the local positions.
-__device__ __forceinline__ uint64_t chunk_base(uint64_t c, cprogram prog, uint32_t L) {
+__device__ __forceinline__ uint64_t chunk_base(uint64_t c, const block_view& v, uint32_t L) {
+  for (uint32_t r = 0; r < L; ++r) {
+    const uint32_t q = v.h->pos[r];
+    c = ((c >> q) << (q + 1)) | (c & ((1ull << q) - 1ull));
+  }
+  return c;
+}
+
+// Physical offset of local index t + (k << BLOCK_THREAD_BITS): the bits of t, and of k.
+__device__ __forceinline__ uint64_t thread_offset(uint32_t t, const block_view& v) {
+  uint64_t low = 0;
+#pragma unroll
+  for (int r = 0; r < BLOCK_THREAD_BITS; ++r) low |= (uint64_t)((t >> r) & 1u) << v.h->pos[r];
+  return low;
+}
+__device__ __forceinline__ uint64_t high_offset(int k, const block_view& v) {
+  uint64_t d = 0;
+#pragma unroll
+  for (int b = 0; b < 4; ++b)
+    if ((k >> b) & 1) d |= 1ull << v.h->pos[BLOCK_THREAD_BITS + b];
+  return d;
+}
+
+// Local index of item v of a gate: zeros inserted at the bits of `inserted`, then the
+// cond bits set.
+__device__ __forceinline__ uint32_t op_index(uint32_t v, uint32_t inserted, uint32_t set) {
+  for (uint32_t m = inserted; m; m &= m - 1) {
+    const uint32_t below = (m & (0u - m)) - 1u;
+    v = ((v & ~below) << 1) | (v & below);
+  }
+  return v | set;
+}
+
+// One amplitude pair of a gate of this kind, with the arithmetic of the plain kernels.
+template <typename R, int KIND>
+__device__ __forceinline__ void kind_math(const double (&u)[8], uint32_t sign, uint32_t j0, cpx<R> x0, cpx<R> x1,
+                                          cpx<R>& y0, cpx<R>& y1) {
+  if constexpr (KIND == BLOCK_KIND_REAL) {
+    const R m00 = (R)u[0], m01 = (R)u[2], m10 = (R)u[4], m11 = (R)u[6];
+    y0 = {m00 * x0.re + m01 * x1.re, m00 * x0.im + m01 * x1.im};
+    y1 = {m10 * x0.re + m11 * x1.re, m10 * x0.im + m11 * x1.im};
+  } else if constexpr (KIND == BLOCK_KIND_X) {
+    const R m00 = (R)u[0], m01 = (R)u[3], m10 = (R)u[5], m11 = (R)u[6];
+    y0 = {m00 * x0.re - m01 * x1.im, m00 * x0.im + m01 * x1.re};
+    y1 = {m11 * x1.re - m10 * x0.im, m11 * x1.im + m10 * x0.re};
+  } else if constexpr (KIND == BLOCK_KIND_MATRIX) {
+    cpx<R> m00, m01, m10, m11;
+    load_matrix(u, m00, m01, m10, m11);
+    y0 = cadd(cmul(m00, x0), cmul(m01, x1));
+    y1 = cadd(cmul(m10, x0), cmul(m11, x1));
+  } else {
+    constexpr int MODE = KIND == BLOCK_KIND_H ? MODE_H : KIND == BLOCK_KIND_SWAP ? MODE_SWAP
+                         : KIND == BLOCK_KIND_ESWAP ? MODE_ESWAP : MODE_MATRIX;
+    pair_math<R, MODE>(u, sign, j0, x0, x1, y0, y1);
+  }
+}
+
+// Calls f with the kind as a compile-time constant; a matrix with a sign mask takes pair_math.
+template <typename F>
+__device__ __forceinline__ void with_pair_kind(const block_gate& op, F f) {
+  switch (op.kind != BLOCK_KIND_ESWAP && op.sign != 0 ? (uint32_t)BLOCK_KIND_SIGNED : op.kind) {
+    case BLOCK_KIND_H: f(std::integral_constant<int, BLOCK_KIND_H>()); break;
+    case BLOCK_KIND_SWAP: f(std::integral_constant<int, BLOCK_KIND_SWAP>()); break;
+    case BLOCK_KIND_ESWAP: f(std::integral_constant<int, BLOCK_KIND_ESWAP>()); break;
+    case BLOCK_KIND_REAL: f(std::integral_constant<int, BLOCK_KIND_REAL>()); break;
+    case BLOCK_KIND_X: f(std::integral_constant<int, BLOCK_KIND_X>()); break;
+    case BLOCK_KIND_SIGNED: f(std::integral_constant<int, BLOCK_KIND_SIGNED>()); break;
+    default: f(std::integral_constant<int, BLOCK_KIND_MATRIX>()); break;
+  }
+}
+
+// LDS slot of local index j: an XOR swizzle, so that groups over low bits spread over all banks.
+__device__ __forceinline__ uint32_t block_slot(uint32_t j) { return j ^ ((j >> 3) & 7u) ^ ((j >> 6) & 7u); }
+
+// One gate over the whole chunk: a strided loop over exactly the local indices it changes.
+template <typename R, int PER>
+__device__ __forceinline__ void single_pass(cpx<R>* lds, const block_gate& op, uint64_t base, uint32_t t) {
+  constexpr uint32_t CAP = PER * BLOCK_THREADS;
+  const uint32_t inserted = op.inserted, set = op.cond;
+  const uint32_t items = CAP >> __popc(inserted);
+  if (op.kind == BLOCK_KIND_NEGATE) {  // the visited indices are exactly the cond subspace
+    for (uint32_t v = t; v < items; v += BLOCK_THREADS) {
+      const uint32_t j = block_slot(op_index(v, inserted, set));
+      lds[j] = cneg(lds[j]);
+    }
+  } else if (op.kind == BLOCK_KIND_DIAG) {
+    cpx<R> c0, c1;
+    chunk_diag(op, base, c0, c1);
+    const uint32_t zmask = op.zmask;
+    for (uint32_t v = t; v < items; v += BLOCK_THREADS) {
+      const uint32_t j = op_index(v, inserted, set);
+      lds[block_slot(j)] = cmul(lds[block_slot(j)], csel((__popc(j & zmask) & 1) != 0, c1, c0));
+    }
+  } else {
+    const uint32_t flip = op.flip;
+    with_pair_kind(op, [&](auto kind) {
+      for (uint32_t v = t; v < items; v += BLOCK_THREADS) {
+        const uint32_t j0 = op_index(v, inserted, set), j1 = j0 ^ flip;
+        const cpx<R> x0 = lds[block_slot(j0)], x1 = lds[block_slot(j1)];
+        cpx<R> y0, y1;
+        kind_math<R, kind>(op.u, op.sign, j0, x0, x1, y0, y1);
+        lds[block_slot(j0)] = y0;
+        lds[block_slot(j1)] = y1;
+      }
+    });
+  }
+}
+
+// A pair gate of a segment on pairs (m, m | F) whose group conditions hold.  A sign mask lies in
+// the group (it is part of the flipped bits), so which pairs it negates is uniform.
+template <int F, typename R, int PER>
+__device__ __forceinline__ void segment_pairs(cpx<R> (&x)[PER], const block_gate& op, bool on) {
+  if constexpr (F < PER) {
+    const uint32_t cond = op.group_cond, sign = op.group_zmask;
+    auto apply = [&](auto kind) {
+      if constexpr (kind != BLOCK_KIND_ESWAP) {
+        if ((cond | sign | op.thread_cond) == 0) {  // the common case: no branches, no selects
+#pragma unroll
+          for (int m = 0; m < PER; ++m) {
+            if ((m & F) != 0) continue;
+            cpx<R> y0, y1;
+            kind_math<R, kind>(op.u, 0, 0, x[m], x[m | F], y0, y1);
+            x[m] = y0;
+            x[m | F] = y1;
+          }
+          return;
+        }
+      }
+#pragma unroll
+      for (int m = 0; m < PER; ++m) {
+        if ((m & F) != 0) continue;
+        if ((m & cond) != cond) continue;  // uniform
+        cpx<R> y0, y1;
+        if constexpr (kind == BLOCK_KIND_ESWAP) {
+          // (pair_math selects per amplitude)
+          const cpx<R> e = {(R)op.u[0], (R)op.u[1]}, x0 = x[m], x1 = x[m | F];
+          const R c = (R)op.u[2], sn = (R)op.u[3];
+          if ((m & sign) != 0) {
+            y0 = {x0.re * c - x1.im * sn, x0.im * c + x1.re * sn};
+            y1 = {x1.re * c - x0.im * sn, x1.im * c + x0.re * sn};
+          } else {
+            y0 = cmul(x0, e);
+            y1 = cmul(x1, e);
+          }
+        } else {
+          double u[8];
+          for (int k = 0; k < 8; ++k) u[k] = op.u[k];
+          if constexpr (kind == BLOCK_KIND_REAL || kind == BLOCK_KIND_X) {
+            if ((__popc(m & sign) & 1) != 0)
+              for (int k = 2; k < 6; ++k) u[k] = -u[k];
+          }
+          kind_math<R, kind>(u, 0, 0, x[m], x[m | F], y0, y1);
+        }
+        x[m] = csel(on, y0, x[m]);
+        x[m | F] = csel(on, y1, x[m | F]);
+      }
+    };
+    switch (op.kind) {  // (X, CNOT and SWAP are moves)
+      case BLOCK_KIND_H: apply(std::integral_constant<int, BLOCK_KIND_H>()); break;
+      case BLOCK_KIND_REAL: apply(std::integral_constant<int, BLOCK_KIND_REAL>()); break;
+      case BLOCK_KIND_X: apply(std::integral_constant<int, BLOCK_KIND_X>()); break;
+      case BLOCK_KIND_ESWAP: apply(std::integral_constant<int, BLOCK_KIND_ESWAP>()); break;
+      default: apply(std::integral_constant<int, BLOCK_KIND_MATRIX>()); break;
+    }
+  }
+}
+
+// Exchanges the members with bit LO set that differ in bit HI: the pairs of a gate that flips both
+// bits then differ in LO alone, the member with LO clear in its place.
+template <int LO, int HI, typename R, int PER>
+__device__ __forceinline__ void segment_rename(cpx<R> (&x)[PER]) {
+  if constexpr (HI < PER) {
+#pragma unroll
+    for (int m = 0; m < PER; ++m) {
+      if ((m & LO) == 0 || (m & HI) != 0) continue;
+      const cpx<R> y = x[m];
+      x[m] = x[m | HI];
+      x[m | HI] = y;
+    }
+  }
+}
+template <typename R, int PER>
+__device__ __forceinline__ void segment_rename_any(cpx<R> (&x)[PER], uint32_t flip) {
+  switch (flip) {
+    case 3: segment_rename<1, 2>(x); break;
+    case 5: segment_rename<1, 4>(x); break;
+    case 6: segment_rename<2, 4>(x); break;
+    case 9: segment_rename<1, 8>(x); break;
+    case 10: segment_rename<2, 8>(x); break;
+    case 12: segment_rename<4, 8>(x); break;
+    default: break;
+  }
+}
+
+// A diagonal gate without conditions in the chunk whose parity bits in the chunk are the group bits
+// ZG (over the group index): each member's coefficient is fixed at compile time.
+template <int ZG, typename R, int PER>
+__device__ __forceinline__ void group_diag(cpx<R> (&x)[PER], cpx<R> c0, cpx<R> c1) {
+  if constexpr (ZG < PER) {
+#pragma unroll
+    for (int m = 0; m < PER; ++m) x[m] = cmul(x[m], (__builtin_popcount(m & ZG) & 1) ? c1 : c0);
+  }
+}
+
+// One gate of a segment on a thread's group, base the local index of member 0.  Conditions and parities split into the thread's part, one test for the group, and
+// the members', which are uniform.
+template <typename R, int PER>
+__device__ __forceinline__ void segment_gate(cpx<R> (&x)[PER], uint32_t base, const block_gate& op, uint64_t chunk) {
+  const bool on = (base & op.thread_cond) == op.thread_cond;
+  if (op.kind == BLOCK_KIND_NEGATE) {
+    const uint32_t sign = on ? 0x80000000u : 0u;
+#pragma unroll
+    for (int m = 0; m < PER; ++m) {
+      const uint32_t s = sign & ((m & op.group_cond) == op.group_cond ? ~0u : 0u);
+      x[m] = cflip(x[m], s);
+    }
+    return;
+  }
+  if (op.kind == BLOCK_KIND_DIAG) {
+    cpx<R> c0, c1;
+    chunk_diag(op, chunk, c0, c1);
+    if ((op.group_cond | op.thread_cond | op.thread_zmask) == 0) {  // the common case
+      switch (op.group_zmask) {
+        case 0: group_diag<0>(x, c0, c1); return;
+        case 1: group_diag<1>(x, c0, c1); return;
+        case 2: group_diag<2>(x, c0, c1); return;
+        case 4: group_diag<4>(x, c0, c1); return;
+        case 8: group_diag<8>(x, c0, c1); return;
+        default: break;
+      }
+    }
+    const bool swapped = (__popc(base & op.thread_zmask) & 1) != 0;
+    const cpx<R> k0 = csel(swapped, c1, c0), k1 = csel(swapped, c0, c1);
+#pragma unroll
+    for (int m = 0; m < PER; ++m) {
+      if ((m & op.group_cond) != op.group_cond) continue;  // uniform
+      const bool odd = (__popc(m & op.group_zmask) & 1) != 0;
+      x[m] = csel(on, cmul(x[m], odd ? k1 : k0), x[m]);
+    }
+    return;
+  }
+  const uint32_t flip = op.group_flip, low = flip & (0u - flip);
+  if (flip != low) segment_rename_any(x, flip);
+  switch (low) {
+    case 1: segment_pairs<1>(x, op, on); break;
+    case 2: segment_pairs<2>(x, op, on); break;
+    case 4: segment_pairs<4>(x, op, on); break;
+    default: segment_pairs<8>(x, op, on); break;
+  }
+  if (flip != low) segment_rename_any(x, flip);
+}
+
+// The physical offset of local index j.
+template <int L>
+__device__ __forceinline__ uint64_t local_offset(uint32_t j, const block_view& v) {
+  uint64_t d = 0;
+#pragma unroll
+  for (int r = 0; r < L; ++r) d |= (uint64_t)((j >> r) & 1u) << v.h->pos[r];
+  return d;
+}
+
+// One workgroup per chunk of exactly PER * BLOCK_THREADS amplitudes
+// (L = 9 + log2 PER), so every global access is unconditional.  The gates run as
+// passes: in a segment each thread takes one group of PER amplitudes (local indices
+// differing in the group bits only) into registers, applies the segment's gates and
+// writes them to where the segment's moves send them; a single pass runs one gate over
+// the chunk in LDS.  The first and the last segment load from and store to the state
+// where their lanes cover whole lines, so a block of two segments exchanges its
+// amplitudes through LDS once.  The program is the launch's second argument, read where
+// the kernel arguments lie.  In a segment the descriptions of the next two gates are on
+// their way while a gate runs: they are scalar loads of about 0.1 us each, which a chunk
+// that has its CU to itself would otherwise wait for.
+// Bound: the HBM round trip of the chunks (about 2.9 ms of a 29-qubit c128 state's 17.2 GB) plus what
+// the two workgroups of a CU do not hide of it in instructions: 4.1 ms a launch of 16 gates (4.2 TB/s)
+// on that state, 3.8 ms a launch of 8 with every qubit local and an LDS round trip per pass.  Waves of
+// 16 amplitudes per lane (256 threads) run large states 1-2 % faster and small ones 15 % slower;
+// 1024 threads, which do not fit twice on a CU, half as fast.
+template <typename R, bool NT, int PER>
+__global__ __launch_bounds__(BLOCK_THREADS, BLOCK_WAVES_PER_SIMD) void k_block(cpx<R>* __restrict__ s, block_args) {
+  constexpr int GB = PER == 1 ? 0 : PER == 2 ? 1 : PER == 4 ? 2 : PER == 8 ? 3 : 4;
+  constexpr int L = BLOCK_THREAD_BITS + GB;
+  __shared__ cpx<R> lds[PER * BLOCK_THREADS];
+  const block_view v((cbytes)__builtin_amdgcn_kernarg_segment_ptr() + sizeof(s));
+  // XCD-contiguous chunk order: consecutive chunks (neighbouring runs of memory) on one XCD
+  const uint64_t chunk = chunk_base(xcd_tile(blockIdx.x, gridDim.x, 1), v, L);
+  const uint32_t t = threadIdx.x;
+  const uint32_t npasses = v.h->num_passes;
+  if (!(v.passes[0].flags & BLOCK_PASS_LOADS)) {
+    const uint64_t low = chunk | thread_offset(t, v);
+#pragma unroll
+    for (uint32_t k = 0; k < PER; ++k)
+      lds[block_slot(t + BLOCK_THREADS * k)] = load_amp<NT>(s + (low | high_offset(k, v)));
+    __syncthreads();
+  }
+  for (uint32_t pi = 0; pi < npasses; ++pi) {
+    const cpass pass = v.passes + pi;
+    const uint32_t first = pass->first_op;
+    if (pass->kind == BLOCK_PASS_SINGLE) {
+      const block_gate op = load_gate(v, first);
+      if (!acts_on(op, chunk)) continue;
+      single_pass<R, PER>(lds, op, chunk, t);
+      __syncthreads();
+      continue;
+    }
+    const uint32_t num_ops = pass->num_ops, num_moves = pass->num_moves, flags = pass->flags;
+    const uint32_t last = first + (num_ops ? num_ops - 1 : 0);
+    op_words cur = load_op(v, first);
+    uint32_t base = t, dep[PER];
+    dep[0] = 0;
+#pragma unroll
+    for (int i = 0; i < GB; ++i) {
+      const uint32_t q = pass->group[i];
+      base = ((base >> q) << (q + 1)) | (base & ((1u << q) - 1u));
+#pragma unroll
+      for (int m = 0; m < (1 << i); ++m) dep[m | 1 << i] = dep[m] | 1u << q;
+    }
+    cpx<R> x[PER];
+    if (flags & BLOCK_PASS_LOADS) {
+      const uint64_t low = chunk | local_offset<L>(base, v);
+#pragma unroll
+      for (int m = 0; m < PER; ++m) x[m] = load_amp<NT>(s + (low | local_offset<L>(dep[m], v)));
+    } else {
+      const uint32_t slot = block_slot(base);  // (the swizzle is linear)
+#pragma unroll
+      for (int m = 0; m < PER; ++m) x[m] = lds[slot ^ block_slot(dep[m])];
+    }
+    for (uint32_t o = 0; o < num_ops; ++o) {
+      const op_words next = load_op(v, min(first + o + 1, last));
+      double u[8];
+      load_coefs(v, cur.coef(), u);
+      const block_gate op = decode(cur, u);
+      if (acts_on(op, chunk)) segment_gate(x, base, op, chunk);
+      cur = next;
+    }
+    uint32_t j[PER];
+#pragma unroll
+    for (int m = 0; m < PER; ++m) j[m] = base | dep[m];
+    for (uint32_t o = first + num_ops; o < first + num_ops + num_moves; ++o) {
+      const op_words w = load_op(v, o);
+      const double none[8] = {};
+      const block_gate op = decode(w, none);
+      if (!acts_on(op, chunk)) continue;
+      const uint32_t flip = op.flip;
+      if ((flip & op.cond) == 0) {  // X, CNOT
+#pragma unroll
+        for (int m = 0; m < PER; ++m) j[m] ^= (j[m] & op.cond) == op.cond ? flip : 0u;
+      } else {  // SWAP: both members of a pair, the one with the pair bit clear has the cond bits set
+        const uint32_t tested = op.cond | 1u << op.pair_bit;
+#pragma unroll
+        for (int m = 0; m < PER; ++m)
+          j[m] ^= (j[m] & tested) == op.cond || ((j[m] ^ flip) & tested) == op.cond ? flip : 0u;
+      }
+    }
+    if (flags & BLOCK_PASS_STORES) {
+      // (without moves: the very addresses this thread loaded; with moves the chunk's loads ended
+      // before an earlier pass's barrier)
+#pragma unroll
+      for (int m = 0; m < PER; ++m) store_amp<NT>(s + (chunk | local_offset<L>(j[m], v)), x[m]);
+      return;
+    }
+    if (num_moves && !(flags & BLOCK_PASS_LOADS)) __syncthreads();  // every group is read before the first is written
+#pragma unroll
+    for (int m = 0; m < PER; ++m) lds[block_slot(j[m])] = x[m];
+    __syncthreads();
+  }
+  const uint64_t low = chunk | thread_offset(t, v);
+#pragma unroll
+  for (uint32_t k = 0; k < PER; ++k)
+    store_amp<NT>(s + (low | high_offset(k, v)), lds[block_slot(t + BLOCK_THREADS * k)]);
+}
+
+typedef const __attribute__((address_space(4))) adjoint_base* cbase;
+
+// Chunk index -> global bits outside the local positions.
+__device__ __forceinline__ uint64_t adjoint_chunk_base(uint64_t c, cbase prog, uint32_t L) {
   for (uint32_t r = 0; r < L; ++r) {
     const uint32_t q = prog->pos[r];
     c = ((c >> q) << (q + 1)) | (c & ((1ull << q) - 1ull));
@@ -261,7 +718,7 @@ __device__ __forceinline__ uint64_t chunk_base(uint64_t c, cprogram prog, uint32
 // Local index of item v of a gate: zeros inserted at op.ins[0 .. nins), then
 // the cond bits set.  The common cases (no insertion: uncontrolled diagonal
 // gates; one: uncontrolled pair gates) avoid the loop.
-__device__ __forceinline__ uint32_t op_index(uint32_t v, const __attribute__((address_space(4))) block_op& op,
+__device__ __forceinline__ uint32_t adjoint_index(uint32_t v, const __attribute__((address_space(4))) adjoint_op& op,
                                              uint32_t nins, uint32_t set, uint32_t lower0) {
   if (nins == 0) return v;
   if (nins == 1) return ((v & ~lower0) << 1) | (v & lower0) | set;
@@ -272,11 +729,11 @@ __device__ __forceinline__ uint32_t op_index(uint32_t v, const __attribute__((ad
   return v | set;
 }
 
-typedef const __attribute__((address_space(4))) block_op& cop;
+typedef const __attribute__((address_space(4))) adjoint_op& cop;
 
 // One gate over the whole chunk: a strided loop over exactly the local indices it changes.
 template <typename R, int PER>
-__device__ __forceinline__ void single_pass(cpx<R>* lds, cop op, uint32_t t) {
+__device__ __forceinline__ void adjoint_single(cpx<R>* lds, cop op, uint32_t t) {
   constexpr uint32_t CAP = PER * BLOCK_THREADS;
   const int mode = op.mode;
   const uint32_t nins = op.nins, set = op.cond;
@@ -287,13 +744,13 @@ __device__ __forceinline__ void single_pass(cpx<R>* lds, cop op, uint32_t t) {
     const uint32_t zmask = op.zmask;
     if (op.negate) {  // the visited indices are exactly the cond subspace
       for (uint32_t v = t; v < items; v += BLOCK_THREADS) {
-        const uint32_t j = op_index(v, op, nins, set, lower0);
+        const uint32_t j = adjoint_index(v, op, nins, set, lower0);
         lds[j] = cneg(lds[j]);
       }
       return;
     }
     for (uint32_t v = t; v < items; v += BLOCK_THREADS) {
-      const uint32_t j = op_index(v, op, nins, set, lower0);
+      const uint32_t j = adjoint_index(v, op, nins, set, lower0);
       lds[j] = cmul(lds[j], csel((__popc(j & zmask) & 1) != 0, c1, c0));
     }
   } else {
@@ -301,7 +758,7 @@ __device__ __forceinline__ void single_pass(cpx<R>* lds, cop op, uint32_t t) {
     double u[8];
     for (int k = 0; k < 8; ++k) u[k] = op.u[k];
     for (uint32_t v = t; v < items; v += BLOCK_THREADS) {
-      const uint32_t j0 = op_index(v, op, nins, set, lower0), j1 = j0 ^ flip;
+      const uint32_t j0 = adjoint_index(v, op, nins, set, lower0), j1 = j0 ^ flip;
       const cpx<R> x0 = lds[j0], x1 = lds[j1];
       cpx<R> y0, y1;
       switch (mode) {
@@ -373,124 +830,6 @@ __device__ __forceinline__ void group_pairs(cpx<R> (&x)[PER], const uint32_t (&j
   }
 }
 
-// An unconditioned diagonal gate whose parity bits are group bits ZG (over the group index):
-// each member's coefficient is fixed at compile time.
-template <int ZG, typename R, int PER>
-__device__ __forceinline__ void group_diag(cpx<R> (&x)[PER], cpx<R> c0, cpx<R> c1) {
-  if constexpr (ZG < PER) {
-#pragma unroll
-    for (int m = 0; m < PER; ++m) x[m] = cmul(x[m], (__builtin_popcount(m & ZG) & 1) ? c1 : c0);
-  }
-}
-
-// A segment: each thread loads one group of PER amplitudes (local indices differing in
-// the group bits only), applies the segment's gates in registers and stores it back.
-template <typename R, int PER>
-__device__ __forceinline__ void segment_pass(cpx<R>* lds, cprogram prog, uint32_t first_op, uint32_t num_ops,
-                                             const __attribute__((address_space(4))) uint32_t* group, uint32_t t) {
-  constexpr int GB = PER == 1 ? 0 : PER == 2 ? 1 : PER == 4 ? 2 : PER == 8 ? 3 : 4;
-  uint32_t base = t;
-#pragma unroll
-  for (int i = 0; i < GB; ++i) {
-    const uint32_t q = group[i];
-    base = ((base >> q) << (q + 1)) | (base & ((1u << q) - 1u));
-  }
-  uint32_t j[PER];
-  cpx<R> x[PER];
-#pragma unroll
-  for (int m = 0; m < PER; ++m) {
-    uint32_t dep = 0;
-#pragma unroll
-    for (int i = 0; i < GB; ++i)
-      if ((m >> i) & 1) dep |= 1u << group[i];
-    j[m] = base | dep;
-    x[m] = lds[j[m]];
-  }
-  for (uint32_t o = 0; o < num_ops; ++o) {
-    cop op = prog->ops[first_op + o];
-    if (op.mode == BLOCK_DIAG) {
-      // in a segment: negations under conditions, and unconditioned diagonal gates (the
-      // planner gives the others a pass)
-      if (op.negate) {
-        const uint32_t cond = op.cond;
-#pragma unroll
-        for (int m = 0; m < PER; ++m) x[m] = cneg_if(x[m], (j[m] & cond) == cond);
-        continue;
-      }
-      const cpx<R> c0 = {(R)op.u[0], (R)op.u[1]}, c1 = {(R)op.u[2], (R)op.u[3]};
-      switch (op.group_zmask) {  // parity bits among the group bits: no per-amplitude select
-        case 0: group_diag<0>(x, c0, c1); continue;
-        case 1: group_diag<1>(x, c0, c1); continue;
-        case 2: group_diag<2>(x, c0, c1); continue;
-        case 3: group_diag<3>(x, c0, c1); continue;
-        case 4: group_diag<4>(x, c0, c1); continue;
-        case 5: group_diag<5>(x, c0, c1); continue;
-        case 6: group_diag<6>(x, c0, c1); continue;
-        case 7: group_diag<7>(x, c0, c1); continue;
-        case 8: group_diag<8>(x, c0, c1); continue;
-        case 9: group_diag<9>(x, c0, c1); continue;
-        case 10: group_diag<10>(x, c0, c1); continue;
-        case 11: group_diag<11>(x, c0, c1); continue;
-        case 12: group_diag<12>(x, c0, c1); continue;
-        case 13: group_diag<13>(x, c0, c1); continue;
-        case 14: group_diag<14>(x, c0, c1); continue;
-        case 15: group_diag<15>(x, c0, c1); continue;
-        default: break;
-      }
-      const uint32_t zmask = op.zmask;
-#pragma unroll
-      for (int m = 0; m < PER; ++m) x[m] = cmul(x[m], csel((__popc(j[m] & zmask) & 1) != 0, c1, c0));
-    } else {
-      switch (op.group_flip) {
-        case 1: group_pairs<1>(x, j, op); break;
-        case 2: group_pairs<2>(x, j, op); break;
-        case 3: group_pairs<3>(x, j, op); break;
-        case 4: group_pairs<4>(x, j, op); break;
-        case 5: group_pairs<5>(x, j, op); break;
-        case 6: group_pairs<6>(x, j, op); break;
-        case 8: group_pairs<8>(x, j, op); break;
-        case 9: group_pairs<9>(x, j, op); break;
-        case 10: group_pairs<10>(x, j, op); break;
-        default: group_pairs<12>(x, j, op); break;
-      }
-    }
-  }
-#pragma unroll
-  for (int m = 0; m < PER; ++m) lds[j[m]] = x[m];
-}
-
-// One workgroup per chunk of exactly PER * BLOCK_THREADS amplitudes
-// (L = 9 + log2 PER), so every global access of the load and store phases is
-// unconditional.  The gates run as passes over the chunk in LDS: segments
-// (several gates on register-resident groups) and single-gate passes.
-template <typename R, bool NT, int PER>
-__global__ __launch_bounds__(BLOCK_THREADS) void k_block(cpx<R>* __restrict__ s, const block_program* program) {
-  constexpr uint32_t CAP = PER * BLOCK_THREADS;
-  __shared__ cpx<R> lds[CAP];
-  const cprogram prog = (cprogram)program;  // uniform: scalar loads
-  const uint32_t L = prog->num_local;
-  // XCD-contiguous chunk order: consecutive chunks (neighbouring runs of memory) on one XCD
-  const uint64_t base = chunk_base(xcd_tile(blockIdx.x, gridDim.x, 1), prog, L);
-  // local index j = t + BLOCK_THREADS * k: the bits of t go to pos[0 .. 8]
-  const uint32_t t = threadIdx.x;
-  uint64_t low = 0;
-  for (uint32_t r = 0; r < (uint32_t)BLOCK_THREAD_BITS; ++r) low |= (uint64_t)((t >> r) & 1u) << prog->pos[r];
-#pragma unroll
-  for (uint32_t k = 0; k < PER; ++k)
-    lds[t + BLOCK_THREADS * k] = load_amp<NT>(s + (base | low | prog->deposit_high[k]));
-  __syncthreads();
-  const uint32_t npasses = prog->num_passes;
-  for (uint32_t pi = 0; pi < npasses; ++pi) {
-    const auto& pass = prog->passes[pi];
-    if (pass.kind == BLOCK_PASS_SINGLE) single_pass<R, PER>(lds, prog->ops[pass.first_op], t);
-    else segment_pass<R, PER>(lds, prog, pass.first_op, pass.num_ops, pass.group, t);
-    __syncthreads();
-  }
-#pragma unroll
-  for (uint32_t k = 0; k < PER; ++k)
-    store_amp<NT>(s + (base | low | prog->deposit_high[k]), lds[t + BLOCK_THREADS * k]);
-}
-
 // Reverse sweep of the adjoint method over one chunk of psi and lambda (both in
 // LDS).  The program's passes (the circuit's inverse ops in reverse order) are
 // register segments or single ops.  A parametric op reads each amplitude pair of
@@ -499,8 +838,6 @@ __global__ __launch_bounds__(BLOCK_THREADS) void k_block(cpx<R>* __restrict__ s,
 // the plain arithmetic; the RX / RY / RZ-type parametric forms use fused
 // multiply-adds (the sweep's results are sums, not amplitudes compared bitwise).
 typedef const __attribute__((address_space(4))) adjoint_block_program* cadjoint;
-
-typedef const __attribute__((address_space(4))) double* cdouble;
 
 // A lane's value from another lane of its row by a DPP control (both 32-bit halves).  Every
 // control used below selects a lane inside the row, so all lanes read a valid source.
@@ -743,7 +1080,7 @@ __device__ __forceinline__ void adjoint_segment(cpx<R>* lp, cpx<R>* ll, cadjoint
                                                 const __attribute__((address_space(4))) uint32_t* group, uint32_t t,
                                                 double (*wave_sums)[BLOCK_THREADS / 64], double* partials) {
   constexpr int GB = PER == 1 ? 0 : PER == 2 ? 1 : PER == 4 ? 2 : PER == 8 ? 3 : 4;
-  const cprogram prog = (cprogram)&aprog->base;
+  const cbase prog = (cbase)&aprog->base;
   uint32_t base = t;
 #pragma unroll
   for (int i = 0; i < GB; ++i) {
@@ -846,10 +1183,10 @@ __global__ __launch_bounds__(BLOCK_THREADS) void k_adjoint_block(cpx<R>* __restr
   __shared__ double wave_sums[2][ADJ_SEGMENT_GRADIENTS][BLOCK_THREADS / 64];
   uint32_t wbuf = 0;
   const cadjoint aprog = (cadjoint)program;
-  const cprogram prog = (cprogram)&program->base;
+  const cbase prog = (cbase)&program->base;
   const uint32_t L = prog->num_local;
   const uint32_t chunk = (uint32_t)xcd_tile(blockIdx.x, gridDim.x, 1);  // XCD-contiguous chunk order
-  const uint64_t base = chunk_base(chunk, prog, L);
+  const uint64_t base = adjoint_chunk_base(chunk, prog, L);
   const uint32_t t = threadIdx.x;
   uint64_t low = 0;
   for (uint32_t r = 0; r < (uint32_t)BLOCK_THREAD_BITS; ++r) low |= (uint64_t)((t >> r) & 1u) << prog->pos[r];
@@ -873,8 +1210,8 @@ __global__ __launch_bounds__(BLOCK_THREADS) void k_adjoint_block(cpx<R>* __restr
     const auto& op = prog->ops[o];
     const int slot = aprog->grad_slot[o];
     if (slot < 0) {
-      single_pass<R, PER>(lp, op, t);
-      single_pass<R, PER>(ll, op, t);
+      adjoint_single<R, PER>(lp, op, t);
+      adjoint_single<R, PER>(ll, op, t);
       __syncthreads();
       continue;
     }
@@ -943,14 +1280,14 @@ unsigned block_run_qubits(int dtype) {
 }
 
 template <typename R, bool NT, int PER>
-static int launch_block_inst(uint64_t chunks, hipStream_t st, cpx<R>* s, const block_program* p) {
+static int launch_block_inst(uint64_t chunks, hipStream_t st, cpx<R>* s, const block_args& p) {
   hipLaunchKernelGGL((k_block<R, NT, PER>), dim3((unsigned)chunks), dim3(BLOCK_THREADS), 0, st, s, p);
   return BRK_OK;
 }
 
 // Picks the instantiation whose chunk is exactly 2^L amplitudes (L = 9 .. 13).
 template <typename R, bool NT>
-static int launch_block_per(uint64_t chunks, hipStream_t st, cpx<R>* s, const block_program* p, unsigned L) {
+static int launch_block_per(uint64_t chunks, hipStream_t st, cpx<R>* s, const block_args& p, unsigned L) {
   switch (L - BLOCK_THREAD_BITS) {
     case 0: return launch_block_inst<R, NT, 1>(chunks, st, s, p);
     case 1: return launch_block_inst<R, NT, 2>(chunks, st, s, p);
@@ -962,27 +1299,27 @@ static int launch_block_per(uint64_t chunks, hipStream_t st, cpx<R>* s, const bl
   }
 }
 
-int launch_block(const block_program* device_program, const block_program& program, void* first, uint64_t size,
-                 int dtype, void* stream) {
+int launch_block(const block_args& program, void* first, uint64_t size, int dtype, void* stream) {
   unsigned nq;
   if (int st = check_state(first, size, dtype, &nq)) return st;
   const uint32_t cap = dtype == BRK_C128 ? BLOCK_MAX_LOCAL_C128 : BLOCK_MAX_LOCAL_C64;
-  if (program.num_local > cap || program.num_local < (uint32_t)BLOCK_THREAD_BITS || program.num_local > nq ||
-      program.num_ops > (uint32_t)BLOCK_MAX_OPS || program.num_passes > (uint32_t)BLOCK_MAX_OPS)
+  const block_header& h = program.h;
+  if (h.num_local > cap || h.num_local < (uint32_t)BLOCK_THREAD_BITS || h.num_local > nq ||
+      h.num_ops > (uint32_t)BLOCK_MAX_OPS || h.num_passes > (uint32_t)BLOCK_MAX_OPS)
     return fail(BRK_ERR_INVALID_ARGUMENT, "block program does not fit (%u local qubits, %u ops, %u passes)",
-                program.num_local, program.num_ops, program.num_passes);
-  const uint64_t chunks = size >> program.num_local;
+                h.num_local, h.num_ops, h.num_passes);
+  const uint64_t chunks = size >> h.num_local;
   if (chunks > 0x7fffffffull) return fail(BRK_ERR_INVALID_ARGUMENT, "too many chunks");
   const bool nt = size * amp_bytes(dtype) >= get_tuning().nt_min_bytes;
   hipStream_t st = as_stream(stream);
-  const unsigned L = program.num_local;
+  const unsigned L = h.num_local;
   int rc;
   if (dtype == BRK_C128)
-    rc = nt ? launch_block_per<double, true>(chunks, st, (cpx<double>*)first, device_program, L)
-            : launch_block_per<double, false>(chunks, st, (cpx<double>*)first, device_program, L);
+    rc = nt ? launch_block_per<double, true>(chunks, st, (cpx<double>*)first, program, L)
+            : launch_block_per<double, false>(chunks, st, (cpx<double>*)first, program, L);
   else
-    rc = nt ? launch_block_per<float, true>(chunks, st, (cpx<float>*)first, device_program, L)
-            : launch_block_per<float, false>(chunks, st, (cpx<float>*)first, device_program, L);
+    rc = nt ? launch_block_per<float, true>(chunks, st, (cpx<float>*)first, program, L)
+            : launch_block_per<float, false>(chunks, st, (cpx<float>*)first, program, L);
   if (rc) return rc;
   return check_launch("block");
 }

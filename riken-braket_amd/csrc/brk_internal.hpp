@@ -74,6 +74,15 @@ __device__ __forceinline__ cpx<float> cneg_if(cpx<float> a, bool on) {
   return {__uint_as_float(__float_as_uint(a.re) ^ m), __uint_as_float(__float_as_uint(a.im) ^ m)};
 }
 
+// a with its components' sign bits flipped by `sign` (0 or 0x80000000)
+__device__ __forceinline__ cpx<double> cflip(cpx<double> a, uint32_t sign) {
+  return {__hiloint2double(__double2hiint(a.re) ^ (int)sign, __double2loint(a.re)),
+          __hiloint2double(__double2hiint(a.im) ^ (int)sign, __double2loint(a.im))};
+}
+__device__ __forceinline__ cpx<float> cflip(cpx<float> a, uint32_t sign) {
+  return {__uint_as_float(__float_as_uint(a.re) ^ sign), __uint_as_float(__float_as_uint(a.im) ^ sign)};
+}
+
 inline size_t amp_bytes(int dtype) { return dtype == BRK_C128 ? 16 : 8; }
 
 // One amplitude as a native 2-vector, so that it can carry the non-temporal

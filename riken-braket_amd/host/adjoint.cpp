@@ -265,7 +265,7 @@ static int get_partials(size_t doubles, hipStream_t stream, partials_lease& leas
 
 // The arithmetic form of parametric op k (adjoint_grad_kind) from the exact zeros of D and of
 // the inverse op's coefficients.
-static int32_t grad_kind(const block_op& op, const double* d) {
+static int32_t grad_kind(const adjoint_op& op, const double* d) {
   const bool d00 = d[0] == 0.0 && d[1] == 0.0, d01 = d[2] == 0.0 && d[3] == 0.0, d10 = d[4] == 0.0 && d[5] == 0.0,
              d11 = d[6] == 0.0 && d[7] == 0.0;
   if (op.mode == BLOCK_DIAG) {
@@ -290,13 +290,13 @@ static int32_t grad_kind(const block_op& op, const double* d) {
 // negations (Z, CZ) and everything else get a pass of their own, as does a segment
 // of one op.
 static void make_adjoint_passes(adjoint_block_program& ap) {
-  block_program& prog = ap.base;
+  adjoint_base& prog = ap.base;
   const unsigned gb = prog.num_local - (unsigned)BLOCK_THREAD_BITS;
   prog.num_passes = 0;
   uint32_t bits = 0, first = 0, count = 0, grads = 0;
   auto single = [&](uint32_t i) {
-    block_pass& p = prog.passes[prog.num_passes++];
-    p = block_pass{};
+    adjoint_pass& p = prog.passes[prog.num_passes++];
+    p = adjoint_pass{};
     p.kind = BLOCK_PASS_SINGLE;
     p.first_op = i;
     p.num_ops = 1;
@@ -304,8 +304,8 @@ static void make_adjoint_passes(adjoint_block_program& ap) {
   auto close = [&]() {
     if (count == 1) single(first);
     if (count > 1) {
-      block_pass& p = prog.passes[prog.num_passes++];
-      p = block_pass{};
+      adjoint_pass& p = prog.passes[prog.num_passes++];
+      p = adjoint_pass{};
       p.kind = BLOCK_PASS_SEGMENT;
       p.first_op = first;
       p.num_ops = count;
@@ -314,7 +314,7 @@ static void make_adjoint_passes(adjoint_block_program& ap) {
       for (unsigned b = 0; b < prog.num_local; ++b)
         if (bits >> b & 1u) p.group[k++] = b;
       for (uint32_t i = first; i < first + count; ++i) {
-        block_op& o = prog.ops[i];
+        adjoint_op& o = prog.ops[i];
         o.group_flip = o.group_pair = 0;
         o.group_zmask = ~0u;  // the reverse segments select diagonal coefficients per amplitude
         for (unsigned g = 0; g < k; ++g) {
@@ -328,7 +328,7 @@ static void make_adjoint_passes(adjoint_block_program& ap) {
     grads = 0;
   };
   for (uint32_t i = 0; i < prog.num_ops; ++i) {
-    const block_op& o = prog.ops[i];
+    const adjoint_op& o = prog.ops[i];
     const bool grad = ap.grad_slot[i] >= 0;
     const uint32_t mixing = (o.mode == BLOCK_DIAG ? 0u : o.flip) | (grad ? 1u << o.pair_bit : 0u);
     const bool alone = (o.mode == BLOCK_DIAG && !grad && o.cond != 0 && !o.negate) ||
@@ -388,7 +388,7 @@ static int blocked_gradient(const brk_circuit* given, const std::vector<int>& gi
     programs.emplace_back();
     adjoint_block_program& ap = programs.back();
     ap = adjoint_block_program{};
-    ap.base = make_block_program(descs.data(), (unsigned)descs.size(), n, L, line_bits);
+    make_adjoint_base(descs.data(), (unsigned)descs.size(), n, L, line_bits, &ap.base);
     for (size_t k = 0; k < descs.size(); ++k) {
       ap.grad_slot[k] = slots[k];
       std::copy(dmats[k].begin(), dmats[k].end(), ap.d[k]);
@@ -439,8 +439,7 @@ static int blocked_gradient(const brk_circuit* given, const std::vector<int>& gi
   if (!status) status = build_programs();
   double ip[2] = {0.0, 0.0};
   if (!status) status = brk_inner_product(lam, dtype, psi, dtype, size, ip, stream);
-  else (void)hipStreamSynchronize(st);  // the plan's device programs are idle before they are freed
-  (void)brk_block_plan_destroy(plan);   // (brk_inner_product synchronised the stream)
+  (void)brk_block_plan_destroy(plan);
   if (status) return status;
   *energy = ip[0];
 

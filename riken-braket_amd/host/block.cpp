@@ -1,17 +1,24 @@
 // Gate-block planner and its C ABI (brk_block_plan_*, brk_circuit_run_blocked).
 //
 // The circuit's ops are walked in order with the logical -> physical qubit
-// map (as brk_circuit_run does).  Consecutive ops are grouped greedily while
-// the union of their qubits, together with the qubits that address one
-// 128-byte line (so every chunk access is whole lines), fits in the local
-// bits of a chunk; the local set is then filled up with the lowest remaining
-// qubits.  A local swap joins a block as the SWAP gate of its two physical
-// qubits (the map changes for the ops after it).  A group of two or more ops
-// becomes one block launch; a single op runs on the plain kernels.  This is the role of bra's
-// BEGIN/END FUSION (bra/src/state.cpp:2193-2217, nompi_state.cpp:1282-1357)
-// and of ket's cache-aware gate functions (gate_bitmasks.hpp:587-2134): a
-// run of gates applied per group of amplitudes held near the core, with the
-// per-gate arithmetic unchanged.
+// map (as brk_circuit_run_timed does).  Consecutive ops are grouped greedily;
+// a local swap joins as the SWAP gate of its two physical qubits (the map
+// changes for the ops after it).  This is the role of bra's BEGIN/END FUSION
+// (bra/src/state.cpp:2193-2217, nompi_state.cpp:1282-1357) and of ket's
+// cache-aware gate functions (gate_bitmasks.hpp:587-2134): a run of gates
+// applied per group of amplitudes held near the core, with the per-gate
+// arithmetic unchanged.
+//
+// Two groupings:
+//  * steps, which the plan reports: the union of a block's qubits, together
+//    with the qubits that address one 128-byte line, fits in the local bits of
+//    a chunk; the local set is filled up with the lowest remaining qubits;
+//  * launches, which run: only the bits that a gate flips need to be local --
+//    control bits and the parity bits of diagonal gates (RZ, CZ, ...) outside
+//    the chunk are the same for all its amplitudes -- so a launch takes the
+//    gates of about two steps (the 32-qubit circuit of 208 ops: 12 launches
+//    for 27 steps; 20 qubits with 10 layers of RZ and CNOT: 12 for 41).
+// A group of one op runs on the plain kernels.
 #include <hip/hip_runtime_api.h>
 
 #include <algorithm>
@@ -30,120 +37,196 @@ int fail(int status, const char* fmt, ...) __attribute__((format(printf, 2, 3)))
 struct brk_block_plan {
   struct step {
     unsigned first_op = 0, num_ops = 0;  // ops of the circuit covered by this step
-    int program = -1;                    // index into programs, or -1: plain op
-    brk_circuit::op physical;            // the op at physical qubits (plain steps)
+    uint64_t local = 0;                  // the block's local qubits, 0: plain op
+  };
+  struct launch {
+    bool plain = false;
+    brk_circuit::op physical;  // the op at physical qubits (plain)
+    brk::block_args args;      // the block's program
   };
   unsigned num_qubits = 0;
   int dtype = BRK_C128;
   std::vector<step> steps;
-  std::vector<brk::block_program> programs;
+  std::vector<launch> launches;
   std::vector<unsigned> final_permutation;
-  brk::block_program* device = nullptr;
-  int device_id = -1;
-  ~brk_block_plan() {
-    if (device) (void)hipFree(device);
-  }
 };
 
 namespace brk {
 
 static unsigned popcount64(uint64_t x) { return (unsigned)__builtin_popcountll(x); }
 
-struct block_builder {
-  unsigned n, max_local, line_bits;
-  uint64_t qubits = 0;  // union of the ops' qubits
-  std::vector<gate_desc> descs;
-  std::vector<brk_circuit::op> ops;
-  unsigned first_op = 0;
-
-  uint64_t line_mask() const { return (1ull << std::min(line_bits, n)) - 1ull; }
-  // a chunk is 2^L amplitudes with L >= 9 (one per thread of a workgroup at least)
-  bool enabled() const { return std::min(max_local, n) >= (unsigned)BLOCK_THREAD_BITS; }
-  bool fits(const gate_desc& d) const {
-    return enabled() && descs.size() < (size_t)BLOCK_MAX_OPS &&
-           popcount64(qubits | d.qubits | line_mask()) <= max_local;
+// The shape of a dtype's chunks on n qubits.
+struct chunk_shape {
+  unsigned n, max_local;
+  uint64_t line;  // the qubits addressing one 128-byte line (block_run_bytes)
+  chunk_shape(unsigned n, int dtype) : n(n), max_local(block_max_local(dtype)) {
+    line = (1ull << std::min(block_run_qubits(dtype), n)) - 1ull;
   }
+  unsigned num_local() const { return std::min(max_local, n); }
+  // a chunk is 2^L amplitudes with L >= 9 (one per thread of a workgroup at least)
+  bool enabled() const { return num_local() >= (unsigned)BLOCK_THREAD_BITS; }
+  bool fits(uint64_t qubits) const { return popcount64(qubits | line) <= max_local; }
 };
 
-// Groups the program's gates into passes over LDS.  A segment holds consecutive
-// gates whose flipped bits (at most two per gate) all lie in the segment's
-// L - 9 group bits; diagonal gates join any segment.  Other gates get a pass
-// of their own.
-static void make_passes(block_program& prog) {
-  const unsigned gb = prog.num_local > (unsigned)BLOCK_THREAD_BITS ? prog.num_local - BLOCK_THREAD_BITS : 0;
-  prog.num_passes = 0;
-  uint32_t bits = 0;
-  auto close = [&](uint32_t first, uint32_t count) {
-    if (!count) return;
-    block_pass& p = prog.passes[prog.num_passes++];
-    p = block_pass{};
-    if (count == 1) {  // one gate: the strided pass visits only what it changes
-      p.kind = BLOCK_PASS_SINGLE;
-      p.first_op = first;
-      p.num_ops = 1;
-      return;
-    }
-    p.kind = BLOCK_PASS_SEGMENT;
-    p.first_op = first;
-    p.num_ops = count;
-    for (unsigned b = 0; b < prog.num_local && (unsigned)__builtin_popcount(bits) < gb; ++b) bits |= 1u << b;
-    unsigned k = 0;
-    for (unsigned b = 0; b < prog.num_local; ++b)
-      if (bits >> b & 1u) p.group[k++] = b;
-    for (uint32_t i = first; i < first + count; ++i) {  // flip / pair bit / zmask over the group index
-      block_op& o = prog.ops[i];
-      o.group_flip = o.group_pair = 0;
-      uint32_t zg = 0, zrest = o.zmask;
-      for (unsigned g = 0; g < k; ++g) {
-        if (o.mode != BLOCK_DIAG && (o.flip >> p.group[g] & 1u)) o.group_flip |= 1u << g;
-        if (o.mode != BLOCK_DIAG && p.group[g] == o.pair_bit) o.group_pair = 1u << g;
-        if (o.zmask >> p.group[g] & 1u) {
-          zg |= 1u << g;
-          zrest &= ~(1u << p.group[g]);
-        }
-      }
-      o.group_zmask = zrest == 0 ? zg : ~0u;
-    }
-  };
-  uint32_t first = 0, count = 0;
-  for (uint32_t i = 0; i < prog.num_ops; ++i) {
-    const block_op& o = prog.ops[i];
-    const uint32_t mixing = o.mode == BLOCK_DIAG ? 0u : o.flip;
-    // a diagonal gate under conditions visits only its subspace in a pass of its own, unless
-    // it is a negation (Z, CZ), which a segment applies with a select
-    const bool alone = o.mode == BLOCK_DIAG ? o.cond != 0 && !o.negate : (unsigned)__builtin_popcount(mixing) > 2;
-    if (alone || (unsigned)__builtin_popcount(mixing) > gb) {
-      close(first, count);
-      block_pass& p = prog.passes[prog.num_passes++];
-      p = block_pass{};
-      p.kind = BLOCK_PASS_SINGLE;
-      p.first_op = i;
-      p.num_ops = 1;
-      first = i + 1;
-      count = 0;
-      bits = 0;
-      continue;
-    }
-    if ((unsigned)__builtin_popcount(bits | mixing) > gb) {
-      close(first, count);
-      first = i;
-      count = 0;
-      bits = 0;
-    }
-    bits |= mixing;
-    ++count;
-  }
-  close(first, count);
+// `qubits` filled up with the lowest others to num_local in all.
+static uint64_t fill_local(uint64_t qubits, unsigned n, unsigned num_local) {
+  for (unsigned q = 0; q < n && popcount64(qubits) < num_local; ++q) qubits |= 1ull << q;
+  return qubits;
 }
 
-// Local positions: the block's qubits, the line qubits, then the lowest others up to L.
-static block_program make_program(const block_builder& b) {
-  block_program prog{};
-  const unsigned L = std::min(b.max_local, b.n);
-  uint64_t local = b.qubits | b.line_mask();
-  for (unsigned q = 0; q < b.n && popcount64(local) < L; ++q) local |= 1ull << q;
+// The bits a gate flips: these have to be local.
+static uint64_t mixing_bits(const gate_desc& d) { return d.mode == BLOCK_DIAG ? 0 : d.flip; }
+
+// Groups the program's gates into passes, reordering them only where that is exact.  A segment
+// takes gates whose flipped bits (at most two per gate) lie in its L - 9 group bits, diagonal
+// gates, and the moves (X, CNOT, SWAP) among them, which it applies last: a gate after a move joins
+// the segment if it mixes none of the move's qubits and none of its bits is one the move flips --
+// a move only renames the indices such a gate acts on, so the order of the two changes no bit of
+// the result.  Matrix gates flipping more bits get a pass of their own.
+static void make_passes(block_program& prog, unsigned line_bits) {
+  const unsigned L = prog.h.num_local;
+  const unsigned gb = L > (unsigned)BLOCK_THREAD_BITS ? L - BLOCK_THREAD_BITS : 0;
+  const uint32_t line = (1u << std::min(line_bits, L)) - 1u;
+  prog.h.num_passes = 0;
+  block_op order[BLOCK_MAX_OPS];
+  uint32_t placed = 0;
+  uint32_t bits = 0, moved = 0, moved_by = 0;  // group bits; bits the moves flip and test
+  std::vector<uint32_t> gates, moves;
+  auto pass = [&](block_pass_kind kind) -> block_pass& {
+    block_pass& p = prog.passes[prog.h.num_passes++];
+    p = block_pass{};
+    p.kind = (uint8_t)kind;
+    p.first_op = (uint16_t)placed;
+    return p;
+  };
+  auto close = [&]() {
+    if (gates.empty() && moves.empty()) return;
+    block_pass& p = pass(BLOCK_PASS_SEGMENT);
+    p.num_ops = (uint8_t)gates.size();
+    p.num_moves = (uint8_t)moves.size();
+    for (unsigned b = L; b-- > 0 && (unsigned)__builtin_popcount(bits) < gb;) bits |= 1u << b;
+    unsigned k = 0;
+    for (unsigned b = 0; b < L; ++b)
+      if (bits >> b & 1u) p.group[k++] = (uint8_t)b;
+    // straight from or to the state where every access covers whole lines.  A segment that loads
+    // and moves stores by way of LDS: another thread may not have loaded the target yet.
+    if (prog.h.num_passes == 1 && !(bits & line)) p.flags |= BLOCK_PASS_LOADS;
+    if (!(bits & line) && (moves.empty() || (!((moved | moved_by) & line) && !(p.flags & BLOCK_PASS_LOADS))))
+      p.flags |= BLOCK_PASS_STORES;
+    for (uint32_t i : gates) {  // the masks over the group index and over the thread's bits
+      block_op o = prog.ops[i];
+      const bool diagonal = o.kind == BLOCK_KIND_DIAG || o.kind == BLOCK_KIND_NEGATE;
+      o.thread_cond = (uint16_t)(o.cond & ~bits);
+      o.thread_zmask = (uint16_t)(o.zmask & ~bits);
+      for (unsigned g = 0; g < k; ++g) {
+        const uint32_t bit = 1u << p.group[g];
+        if (!diagonal && (o.flip & bit)) o.group_flip |= (uint8_t)(1u << g);
+        if (!diagonal && p.group[g] == o.pair_bit) o.group_pair = (uint8_t)(1u << g);
+        if ((diagonal ? o.zmask : o.sign) & bit) o.group_zmask |= (uint8_t)(1u << g);
+        if (o.cond & bit) o.group_cond |= (uint8_t)(1u << g);
+      }
+      order[placed++] = o;
+    }
+    for (uint32_t i : moves) order[placed++] = prog.ops[i];
+    gates.clear();
+    moves.clear();
+    bits = moved = moved_by = 0;
+  };
+  for (uint32_t i = 0; i < prog.h.num_ops; ++i) {
+    const block_op& o = prog.ops[i];
+    if (o.kind == BLOCK_KIND_SWAP) {
+      moves.push_back(i);
+      moved |= o.flip;
+      moved_by |= o.cond & (uint32_t)~o.flip;
+      continue;
+    }
+    const bool diagonal = o.kind == BLOCK_KIND_DIAG || o.kind == BLOCK_KIND_NEGATE;
+    const uint32_t mixing = diagonal ? 0u : o.flip;
+    const unsigned flips = (unsigned)__builtin_popcount(mixing);
+    if (flips > 2 || flips > gb || (o.kind == BLOCK_KIND_MATRIX && o.sign)) {
+      close();
+      pass(BLOCK_PASS_SINGLE).num_ops = 1;
+      order[placed++] = o;
+      continue;
+    }
+    const bool before_moves = !(mixing & (moved | moved_by)) && !((o.cond | o.zmask) & moved);
+    if (!before_moves || (unsigned)__builtin_popcount(bits | mixing) > gb) close();
+    bits |= mixing;
+    gates.push_back(i);
+  }
+  close();
+  // only the last pass stores
+  for (uint32_t k = 0; k + 1 < prog.h.num_passes; ++k) prog.passes[k].flags &= (uint8_t)~BLOCK_PASS_STORES;
+  std::copy(order, order + placed, prog.ops);
+}
+
+static uint8_t kind_of(const gate_desc& d) {
+  switch (d.mode) {
+    case BLOCK_H: return BLOCK_KIND_H;
+    case BLOCK_SWAP: return BLOCK_KIND_SWAP;
+    case BLOCK_ESWAP: return BLOCK_KIND_ESWAP;
+    case BLOCK_DIAG: return block_op_coefs(d) == 0 ? BLOCK_KIND_NEGATE : BLOCK_KIND_DIAG;
+    default: break;
+  }
+  const double* u = d.u;
+  if (u[1] == 0.0 && u[3] == 0.0 && u[5] == 0.0 && u[7] == 0.0) return BLOCK_KIND_REAL;
+  if (u[1] == 0.0 && u[2] == 0.0 && u[4] == 0.0 && u[7] == 0.0) return BLOCK_KIND_X;
+  return BLOCK_KIND_MATRIX;
+}
+
+static void make_block_program(const gate_desc* descs, unsigned count, unsigned n, uint64_t local, unsigned num_local,
+                        unsigned line_bits, block_program* out) {
+  block_program& prog = *out;
+  prog.h = block_header{};
+  prog.h.ops_at = (uint16_t)offsetof(block_program, ops);
+  prog.h.coefs_at = (uint16_t)offsetof(block_program, coefs);
+  const unsigned L = std::min(num_local, n);
+  local = fill_local(local | ((1ull << std::min(line_bits, n)) - 1ull), n, L);
   unsigned r = 0, rank[64] = {};
-  for (unsigned q = 0; q < b.n; ++q)
+  for (uint64_t m = local; m; m &= m - 1) {
+    const unsigned q = (unsigned)__builtin_ctzll(m);
+    rank[q] = r;
+    prog.h.pos[r++] = (uint8_t)q;
+  }
+  prog.h.num_local = r;
+  auto to_local = [&](uint64_t m) {
+    uint32_t bits = 0;
+    for (m &= local; m; m &= m - 1) bits |= 1u << rank[__builtin_ctzll(m)];
+    return (uint16_t)bits;
+  };
+  prog.h.num_ops = count;
+  unsigned coef = 0;
+  for (unsigned i = 0; i < count; ++i) {
+    const gate_desc& d = descs[i];
+    block_op& o = prog.ops[i];
+    o = block_op{};
+    const bool diagonal = d.mode == BLOCK_DIAG;
+    o.pair_bit = diagonal ? 0 : (uint8_t)rank[d.pair_bit];
+    o.flip = to_local(d.flip);
+    o.cond = to_local(d.cond);
+    o.sign = to_local(d.sign);
+    // the pair's first index has the pair bit clear: that bit of the sign mask never counts
+    if (d.mode == BLOCK_MATRIX) o.sign &= (uint16_t)~(1u << o.pair_bit);
+    o.zmask = to_local(d.zmask);
+    o.outer_cond = d.cond & ~local;
+    o.outer_zmask = d.zmask & ~local;
+    o.kind = kind_of(d);
+    o.inserted = (uint16_t)(o.cond | (diagonal ? 0u : 1u << o.pair_bit));
+    o.coef = (uint16_t)coef;
+    std::copy(d.u, d.u + block_op_coefs(d), prog.coefs + coef);
+    coef += (unsigned)block_op_coefs(d);
+  }
+}
+
+void make_adjoint_base(const gate_desc* descs, unsigned count, unsigned n, unsigned num_local, unsigned line_bits,
+                       adjoint_base* out) {
+  adjoint_base& prog = *out;
+  prog = adjoint_base{};
+  uint64_t local = (1ull << std::min(line_bits, n)) - 1ull;
+  for (unsigned i = 0; i < count; ++i) local |= descs[i].qubits;
+  local = fill_local(local, n, std::min(num_local, n));
+  unsigned r = 0, rank[64] = {};
+  for (unsigned q = 0; q < n; ++q)
     if (local >> q & 1u) {
       rank[q] = r;
       prog.pos[r++] = q;
@@ -151,12 +234,12 @@ static block_program make_program(const block_builder& b) {
   prog.num_local = r;
   auto to_local = [&](uint64_t m) {
     uint32_t out = 0;
-    for (unsigned q = 0; q < b.n; ++q)
+    for (unsigned q = 0; q < n; ++q)
       if (m >> q & 1u) out |= 1u << rank[q];
     return out;
   };
   // local index j = t + BLOCK_THREADS * k: the physical offset of the k part
-  const uint32_t count = 1u << r, per = count > (uint32_t)BLOCK_THREADS ? count / BLOCK_THREADS : 1;
+  const uint32_t size = 1u << r, per = size > (uint32_t)BLOCK_THREADS ? size / BLOCK_THREADS : 1;
   for (uint32_t k = 0; k < per; ++k) {
     const uint32_t j = k << BLOCK_THREAD_BITS;
     uint64_t dep = 0;
@@ -164,10 +247,10 @@ static block_program make_program(const block_builder& b) {
       if (j >> bit & 1u) dep |= 1ull << prog.pos[bit];
     prog.deposit_high[k] = dep;
   }
-  prog.num_ops = (uint32_t)b.descs.size();
-  for (size_t i = 0; i < b.descs.size(); ++i) {
-    const gate_desc& d = b.descs[i];
-    block_op& o = prog.ops[i];
+  prog.num_ops = count;
+  for (unsigned i = 0; i < count; ++i) {
+    const gate_desc& d = descs[i];
+    adjoint_op& o = prog.ops[i];
     o.mode = d.mode;
     o.pair_bit = d.mode == BLOCK_DIAG ? 0 : rank[d.pair_bit];
     o.flip = to_local(d.flip);
@@ -183,21 +266,29 @@ static block_program make_program(const block_builder& b) {
       if (inserted >> bit & 1u) o.ins[o.nins++] = bit;
     std::copy(d.u, d.u + 8, o.u);
   }
-  make_passes(prog);
-  return prog;
 }
 
-block_program make_block_program(const gate_desc* descs, unsigned count, unsigned n, unsigned num_local,
-                                 unsigned line_bits) {
-  block_builder b;
-  b.n = n;
-  b.max_local = num_local;
-  b.line_bits = line_bits;
-  for (unsigned i = 0; i < count; ++i) {
-    b.qubits |= descs[i].qubits;
-    b.descs.push_back(descs[i]);
+// The program as launch arguments (its ops fit: BLOCK_ARG_ROOM).
+static void pack(const block_program& prog, block_args* out) {
+  unsigned coefs = 0;
+  for (unsigned i = 0; i < prog.h.num_ops; ++i) {
+    const block_op& o = prog.ops[i];
+    const unsigned k = o.kind == BLOCK_KIND_DIAG || o.kind == BLOCK_KIND_ESWAP ? 4
+                       : o.kind == BLOCK_KIND_H || o.kind == BLOCK_KIND_SWAP || o.kind == BLOCK_KIND_NEGATE ? 0 : 8;
+    coefs = std::max(coefs, o.coef + k);
   }
-  return make_program(b);
+  out->h = prog.h;
+  char* at = reinterpret_cast<char*>(out) + sizeof(block_header);
+  auto put = [&](const void* from, size_t bytes) {
+    std::memcpy(at, from, bytes);
+    at += bytes;
+  };
+  put(prog.passes, sizeof(block_pass) * prog.h.num_passes);
+  if (prog.h.num_passes & 1u) at += 4;  // 64-bit words follow
+  out->h.ops_at = (uint16_t)(at - reinterpret_cast<char*>(out));
+  put(prog.ops, sizeof(block_op) * prog.h.num_ops);
+  out->h.coefs_at = (uint16_t)(at - reinterpret_cast<char*>(out));
+  put(prog.coefs, sizeof(double) * coefs);
 }
 
 op_dependences dependences_of(const std::vector<brk_circuit::op>& ops) {
@@ -313,25 +404,74 @@ static brk_circuit::op map_op(const brk_circuit::op& o, const permutation& perm)
   return m;
 }
 
-static void flush(block_builder& b, brk_block_plan& plan) {
-  if (b.ops.empty()) return;
-  if (b.ops.size() == 1 || !b.enabled()) {
-    brk_block_plan::step s;
-    s.first_op = b.first_op;
-    s.num_ops = 1;
-    s.physical = b.ops[0];
-    plan.steps.push_back(std::move(s));
-  } else {
-    brk_block_plan::step s;
-    s.first_op = b.first_op;
-    s.num_ops = (unsigned)b.ops.size();
-    s.program = (int)plan.programs.size();
-    plan.programs.push_back(make_program(b));
-    plan.steps.push_back(std::move(s));
+// Describes op i of the circuit at physical qubits and advances the map over it.
+static int physical_op(const brk_circuit::op& o, permutation& perm, brk_circuit::op* m, gate_desc* d) {
+  if (o.code == BRK_OP_LOCAL_SWAP) {
+    // the data of a local swap is a SWAP gate on its two physical qubits
+    // (swap_permutated_local_qubits.hpp:64-77); the map changes for the ops after it
+    *m = o;
+    if (int st = describe_physical_op(BRK_OP_SWAP, o.targets.data(), 2, nullptr, 0, nullptr, d)) return st;
+    perm.permutate(perm.inverse[o.targets[0]], perm.inverse[o.targets[1]]);
+    return BRK_OK;
   }
-  b.qubits = 0;
-  b.descs.clear();
-  b.ops.clear();
+  *m = map_op(o, perm);
+  return describe_physical_op(m->code, m->targets.data(), (unsigned)m->targets.size(),
+                              m->controls.empty() ? nullptr : m->controls.data(), (unsigned)m->controls.size(),
+                              m->params.data(), d);
+}
+
+// Collects consecutive ops into launches and hands each over as soon as it is complete.
+// plain(op) / block(args) return a status.
+template <typename Plain, typename Block>
+struct launch_builder {
+  chunk_shape shape;
+  unsigned line_bits;
+  Plain plain;
+  Block block;
+  uint64_t mixing = 0;
+  size_t room = 0;
+  std::vector<gate_desc> descs;
+  brk_circuit::op single;  // the first op of the group
+  block_program prog;
+  block_args args{};
+
+  launch_builder(unsigned n, int dtype, Plain p, Block b)
+      : shape(n, dtype), line_bits(block_run_qubits(dtype)), plain(p), block(b) {}
+  int add(const brk_circuit::op& m, const gate_desc& d) {
+    if (!shape.enabled() || !shape.fits(mixing_bits(d))) {
+      if (int st = flush()) return st;
+      return plain(m);
+    }
+    if (descs.size() == (size_t)BLOCK_MAX_OPS || room + block_op_room(d) > BLOCK_ARG_ROOM ||
+        !shape.fits(mixing | mixing_bits(d)))
+      if (int st = flush()) return st;
+    if (descs.empty()) single = m;
+    mixing |= mixing_bits(d);
+    room += block_op_room(d);
+    descs.push_back(d);
+    return BRK_OK;
+  }
+  int flush() {
+    int st = BRK_OK;
+    if (descs.size() == 1) {
+      st = plain(single);
+    } else if (!descs.empty()) {
+      make_block_program(descs.data(), (unsigned)descs.size(), shape.n, mixing, shape.num_local(), line_bits, &prog);
+      make_passes(prog, line_bits);
+      pack(prog, &args);
+      st = block(args);
+    }
+    mixing = 0;
+    room = 0;
+    descs.clear();
+    return st;
+  }
+};
+
+static int check_permutation(permutation& perm, const unsigned* given, unsigned n) {
+  if (given && !perm.load(given, n))
+    return fail(BRK_ERR_INVALID_ARGUMENT, "permutation is not a permutation of 0..%u", n - 1);
+  return BRK_OK;
 }
 
 static int build_plan(const brk_circuit* circuit, int dtype, const unsigned* permutation_in, brk_block_plan* plan) {
@@ -339,68 +479,67 @@ static int build_plan(const brk_circuit* circuit, int dtype, const unsigned* per
   plan->num_qubits = n;
   plan->dtype = dtype;
   permutation perm(n);
-  if (permutation_in && !perm.load(permutation_in, n))
-    return fail(BRK_ERR_INVALID_ARGUMENT, "permutation is not a permutation of 0..%u", n - 1);
-  block_builder b;
-  b.n = n;
-  b.max_local = block_max_local(dtype);
-  b.line_bits = block_run_qubits(dtype);  // default: one 128-byte line
+  if (int st = check_permutation(perm, permutation_in, n)) return st;
+  const chunk_shape shape(n, dtype);
+  // the step in the making
+  brk_block_plan::step s;
+  uint64_t qubits = 0;
+  auto close_step = [&]() {
+    if (!s.num_ops) return;
+    if (s.num_ops > 1) s.local = fill_local(qubits | shape.line, n, shape.num_local());
+    plan->steps.push_back(s);
+    s = brk_block_plan::step{};
+    qubits = 0;
+  };
+  auto plain = [&](const brk_circuit::op& m) {
+    plan->launches.emplace_back();
+    plan->launches.back().plain = true;
+    plan->launches.back().physical = m;
+    return BRK_OK;
+  };
+  auto block = [&](const block_args& a) {
+    plan->launches.emplace_back();
+    plan->launches.back().args = a;
+    return BRK_OK;
+  };
+  launch_builder<decltype(plain), decltype(block)> b(n, dtype, plain, block);
   for (unsigned i = 0; i < circuit->ops.size(); ++i) {
-    const auto& o = circuit->ops[i];
     gate_desc d;
     brk_circuit::op m;
-    if (o.code == BRK_OP_LOCAL_SWAP) {
-      // the data of a local swap is a SWAP gate on its two physical qubits
-      // (swap_permutated_local_qubits.hpp:64-77); the map changes for the ops after it
-      m = o;
-      if (int st = describe_physical_op(BRK_OP_SWAP, o.targets.data(), 2, nullptr, 0, nullptr, &d)) return st;
-      perm.permutate(perm.inverse[o.targets[0]], perm.inverse[o.targets[1]]);
-    } else {
-      m = map_op(o, perm);
-      if (int st = describe_physical_op(m.code, m.targets.data(), (unsigned)m.targets.size(),
-                                        m.controls.empty() ? nullptr : m.controls.data(),
-                                        (unsigned)m.controls.size(), m.params.data(), &d))
-        return st;
-    }
-    if (!b.fits(d)) flush(b, *plan);
-    if (b.ops.empty()) b.first_op = i;
-    b.qubits |= d.qubits;
-    b.descs.push_back(d);
-    b.ops.push_back(m);
+    if (int st = physical_op(circuit->ops[i], perm, &m, &d)) return st;
+    if (!shape.enabled() || s.num_ops == (unsigned)BLOCK_MAX_OPS || !shape.fits(qubits | d.qubits)) close_step();
+    if (!s.num_ops) s.first_op = i;
+    ++s.num_ops;
+    qubits |= d.qubits;
+    if (int st = b.add(m, d)) return st;
   }
-  flush(b, *plan);
+  close_step();
+  if (int st = b.flush()) return st;
   plan->final_permutation = perm.perm;
   return BRK_OK;
 }
 
-static int upload(brk_block_plan* plan) {
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess) return fail(BRK_ERR_HIP, "hipGetDevice failed");
-  if (plan->device && plan->device_id == dev) return BRK_OK;
-  if (plan->device) (void)hipFree(plan->device);
-  plan->device = nullptr;
-  if (plan->programs.empty()) {
-    plan->device_id = dev;
-    return BRK_OK;
-  }
-  const size_t bytes = sizeof(block_program) * plan->programs.size();
-  if (hipMalloc((void**)&plan->device, bytes) != hipSuccess) return fail(BRK_ERR_OUT_OF_MEMORY, "block programs");
-  if (hipMemcpy(plan->device, plan->programs.data(), bytes, hipMemcpyHostToDevice) != hipSuccess)
-    return fail(BRK_ERR_HIP, "uploading the block programs failed");
-  plan->device_id = dev;
+static int run_plan(const brk_block_plan* plan, void* first, void* stream) {
+  const uint64_t size = 1ull << plan->num_qubits;
+  for (const auto& l : plan->launches)
+    if (int st = l.plain ? apply_physical_op(l.physical, first, size, plan->dtype, stream)
+                         : launch_block(l.args, first, size, plan->dtype, stream))
+      return st;
   return BRK_OK;
 }
 
-static int run_plan(brk_block_plan* plan, void* first, void* stream) {
-  if (int st = upload(plan)) return st;
-  const uint64_t size = 1ull << plan->num_qubits;
-  for (const auto& s : plan->steps) {
-    int st;
-    if (s.program < 0) st = apply_physical_op(s.physical, first, size, plan->dtype, stream);
-    else st = launch_block(plan->device + s.program, plan->programs[s.program], first, size, plan->dtype, stream);
-    if (st) return st;
+int run_in_blocks(const brk_circuit* circuit, void* first, int dtype, permutation& perm, void* stream) {
+  const uint64_t size = 1ull << circuit->num_qubits;
+  auto plain = [&](const brk_circuit::op& m) { return apply_physical_op(m, first, size, dtype, stream); };
+  auto block = [&](const block_args& a) { return launch_block(a, first, size, dtype, stream); };
+  launch_builder<decltype(plain), decltype(block)> b(circuit->num_qubits, dtype, plain, block);
+  for (const auto& o : circuit->ops) {
+    gate_desc d;
+    brk_circuit::op m;
+    if (int st = physical_op(o, perm, &m, &d)) return st;
+    if (int st = b.add(m, d)) return st;
   }
-  return BRK_OK;
+  return b.flush();
 }
 
 }  // namespace brk
@@ -441,9 +580,9 @@ int brk_block_plan_step(const brk_block_plan* plan, unsigned i, unsigned* first_
   const auto& s = plan->steps[i];
   if (first_op) *first_op = s.first_op;
   if (num_ops) *num_ops = s.num_ops;
-  const unsigned L = s.program < 0 ? 0 : plan->programs[s.program].num_local;
-  if (num_local) *num_local = L;
-  if (local_qubits && L) std::copy(plan->programs[s.program].pos, plan->programs[s.program].pos + L, local_qubits);
+  if (num_local) *num_local = popcount64(s.local);
+  if (local_qubits)
+    for (uint64_t m = s.local; m; m &= m - 1) *local_qubits++ = (unsigned)__builtin_ctzll(m);
   return BRK_OK;
 }
 
@@ -469,14 +608,14 @@ int brk_circuit_block_order(const brk_circuit* circuit, unsigned num_local, unsi
 
 int brk_circuit_run_blocked(const brk_circuit* circuit, void* first, int dtype, unsigned* permutation,
                             void* stream) {
-  brk_block_plan* plan = nullptr;
-  if (int st = brk_block_plan_create(circuit, dtype, permutation, &plan)) return st;
-  int st = run_plan(plan, first, stream);
-  // the programs must stay resident until the launches that read them are done
+  if (!circuit) return fail(BRK_ERR_INVALID_ARGUMENT, "null argument");
+  if (dtype != BRK_C128 && dtype != BRK_C64) return fail(BRK_ERR_UNSUPPORTED_DTYPE, "dtype %d", dtype);
+  brk::permutation perm(circuit->num_qubits);
+  if (int st = check_permutation(perm, permutation, circuit->num_qubits)) return st;
+  int st = run_in_blocks(circuit, first, dtype, perm, stream);
   if (hipStreamSynchronize(reinterpret_cast<hipStream_t>(stream)) != hipSuccess && !st)
     st = fail(BRK_ERR_HIP, "hipStreamSynchronize failed");
-  if (!st && permutation) std::copy(plan->final_permutation.begin(), plan->final_permutation.end(), permutation);
-  delete plan;
+  if (!st && permutation) std::copy(perm.perm.begin(), perm.perm.end(), permutation);
   return st;
 }
 

@@ -40,6 +40,11 @@ struct permutation {
 // Applies one operation at physical positions (targets/controls already mapped).
 int apply_physical_op(const brk_circuit::op& o, void* first, uint64_t size, int dtype, void* stream);
 
+// Enqueues the circuit as gate blocks (host/block.cpp), each launched as soon as its ops are
+// collected: the amplitudes of one op after the other bit for bit.  Advances the map.  Without
+// allocation, upload or synchronisation on the device.
+int run_in_blocks(const brk_circuit* circuit, void* first, int dtype, permutation& perm, void* stream);
+
 // The 2x2 (or 2^k x 2^k for multi-target ops) unitary of an op on its
 // operated qubits, in the order targets ++ controls (bit j of the local index
 // <-> qubit j of that list).  Used by the fusion planner.  Returns false for

@@ -74,6 +74,35 @@ def test_blocked_equals_plain_bitwise(oracle, n, dtype, seed, access):
         assert np.max(np.abs(blocked - ref)) < 1e-12
 
 
+@pytest.mark.parametrize("n,dtype,seed", [(2, brk.C128, 31), (8, brk.C64, 32), (9, brk.C128, 33), (10, brk.C64, 34),
+                                          (11, brk.C128, 35), (12, brk.C128, 36), (13, brk.C64, 37),
+                                          (13, brk.C128, 38), (16, brk.C64, 39), (19, brk.C128, 40),
+                                          (21, brk.C64, 41)])
+def test_run_equals_gate_by_gate_bitwise(n, dtype, seed, access):
+    """brk_circuit_run and a block plan (launches of many gates, controls and diagonal gates on any qubit,
+    moves deferred) against brk_circuit_run_timed, which launches the plain kernel of every op: the same
+    bits, zeros' signs included (a state with zeros), for every op kind."""
+    note(f"gpu run vs gate by gate n={n} dtype={dtype} seed={seed} ({access})")
+    rng = np.random.default_rng(seed)
+    ops = random_ops(n, 220, seed, local_swaps=6 if n >= 4 else 0)
+    ops += [("X", (0,), (), ()), ("X", (n - 1,), (0,), ()), ("SWAP", (0, n - 1), (), ())] * (n > 1)
+    perm0 = [int(q) for q in rng.permutation(n)]
+    s = D.random_state(n, rng)
+    s[rng.random(s.size) < 0.3] = 0.0
+    c = brk.Circuit(n, ops)
+    plan = brk.BlockPlan(c, dtype, perm0)
+    states = [DeviceState.from_host(s, dtype) for _ in range(3)]
+    final, _ = c.run_timed(states[0].ptr, dtype, perm0)
+    assert c.run(states[1].ptr, dtype, perm0) == final
+    plan.run(states[2].ptr)
+    assert plan.final_permutation == final
+    want, *got = [st.download() for st in states]
+    for st in states:
+        st.free()
+    for x in got:
+        assert same_bits(want, x)
+
+
 def test_dense_low_qubit_blocks(oracle):
     """Many gates on the line qubits and their neighbours: long blocks, every pair mode."""
     n = 18
