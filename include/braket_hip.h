@@ -370,8 +370,8 @@ int brk_generate_events_noalloc(const void* first, uint64_t size, int dtype, con
                                 unsigned num_events, uint64_t* events, void* stream);
 
 /* ------------------------------------------------------------------------ */
-/* Circuits: an ordered list of operations on logical qubits, run with the  */
-/* plain per-gate kernels.  Stands in for the gate list bra's interpreter   */
+/* Circuits: an ordered list of operations on logical qubits, applied with  */
+/* the plain path's arithmetic.  The gate list bra's interpreter            */
 /* builds (bra/src/interpreter.cpp:371-825) and executes through            */
 /* bra::nompi_state (interpreter::apply_circuit, interpreter.cpp:851-872).  */
 /* ------------------------------------------------------------------------ */
@@ -416,10 +416,12 @@ int brk_circuit_op(const brk_circuit* circuit, unsigned i, int* op, unsigned* ta
    (num_qubits entries, logical -> physical, in/out) maps each logical qubit
    to its bit in the state, as ket::mpi::qubit_permutation does
    (ket/include/ket/mpi/qubit_permutation.hpp:40-302); NULL = identity,
-   local swaps then update an internal copy only. */
+   local swaps then update an internal copy only.  Asynchronous, allocates
+   nothing on the device.  Consecutive operations run as gate blocks (below):
+   bit for bit the amplitudes of one gate call after another. */
 int brk_circuit_run(const brk_circuit* circuit, void* first, int dtype, unsigned* permutation, void* stream);
-/* Same, recording HIP events around every operation; op_ms[i] receives the
-   device time of operation i (synchronises the stream). */
+/* Same, every operation with a plain kernel of its own between HIP events;
+   op_ms[i] receives the device time of operation i (synchronises the stream). */
 int brk_circuit_run_timed(const brk_circuit* circuit, void* first, int dtype, unsigned* permutation,
                           float* op_ms, void* stream);
 

@@ -267,22 +267,15 @@ int brk_circuit_op(const brk_circuit* circuit, unsigned i, int* op, unsigned* ta
   return BRK_OK;
 }
 
-static int run_impl(const brk_circuit* circuit, void* first, int dtype, unsigned* permutation_io, float* op_ms,
-                    void* stream) {
-  if (!circuit) return fail(BRK_ERR_INVALID_ARGUMENT, "circuit is null");
-  const unsigned n = circuit->num_qubits;
-  const uint64_t size = 1ull << n;
-  brk::permutation perm(n);
-  if (permutation_io && !perm.load(permutation_io, n))
-    return fail(BRK_ERR_INVALID_ARGUMENT, "permutation is not a permutation of 0..%u", n - 1);
+// One operation after the other on the plain kernels, with the device time of each.
+static int run_timed(const brk_circuit* circuit, void* first, int dtype, brk::permutation& perm, float* op_ms,
+                     void* stream) {
+  const uint64_t size = 1ull << circuit->num_qubits;
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-  std::vector<hipEvent_t> events;
-  if (op_ms) {
-    events.resize(circuit->ops.size() + 1);
-    for (auto& e : events)
-      if (hipEventCreate(&e) != hipSuccess) return fail(BRK_ERR_HIP, "hipEventCreate failed");
-    (void)hipEventRecord(events[0], st);
-  }
+  std::vector<hipEvent_t> events(circuit->ops.size() + 1);
+  for (auto& e : events)
+    if (hipEventCreate(&e) != hipSuccess) return fail(BRK_ERR_HIP, "hipEventCreate failed");
+  (void)hipEventRecord(events[0], st);
   int status = BRK_OK;
   brk_circuit::op mapped;
   for (size_t i = 0; i < circuit->ops.size() && status == BRK_OK; ++i) {
@@ -300,17 +293,27 @@ static int run_impl(const brk_circuit* circuit, void* first, int dtype, unsigned
       for (size_t j = 0; j < o.controls.size(); ++j) mapped.controls[j] = perm.perm[o.controls[j]];
       status = apply_physical_op(mapped, first, size, dtype, stream);
     }
-    if (op_ms && status == BRK_OK) (void)hipEventRecord(events[i + 1], st);
+    if (status == BRK_OK) (void)hipEventRecord(events[i + 1], st);
   }
-  if (op_ms) {
-    if (status == BRK_OK) {
-      if (hipEventSynchronize(events.back()) != hipSuccess) status = fail(BRK_ERR_HIP, "hipEventSynchronize failed");
-      for (size_t i = 0; status == BRK_OK && i < circuit->ops.size(); ++i)
-        if (hipEventElapsedTime(&op_ms[i], events[i], events[i + 1]) != hipSuccess)
-          status = fail(BRK_ERR_HIP, "hipEventElapsedTime failed");
-    }
-    for (auto& e : events) (void)hipEventDestroy(e);
+  if (status == BRK_OK) {
+    if (hipEventSynchronize(events.back()) != hipSuccess) status = fail(BRK_ERR_HIP, "hipEventSynchronize failed");
+    for (size_t i = 0; status == BRK_OK && i < circuit->ops.size(); ++i)
+      if (hipEventElapsedTime(&op_ms[i], events[i], events[i + 1]) != hipSuccess)
+        status = fail(BRK_ERR_HIP, "hipEventElapsedTime failed");
   }
+  for (auto& e : events) (void)hipEventDestroy(e);
+  return status;
+}
+
+static int run_impl(const brk_circuit* circuit, void* first, int dtype, unsigned* permutation_io, float* op_ms,
+                    void* stream) {
+  if (!circuit) return fail(BRK_ERR_INVALID_ARGUMENT, "circuit is null");
+  const unsigned n = circuit->num_qubits;
+  brk::permutation perm(n);
+  if (permutation_io && !perm.load(permutation_io, n))
+    return fail(BRK_ERR_INVALID_ARGUMENT, "permutation is not a permutation of 0..%u", n - 1);
+  const int status = op_ms ? run_timed(circuit, first, dtype, perm, op_ms, stream)
+                           : run_in_blocks(circuit, first, dtype, perm, stream);
   if (status == BRK_OK && permutation_io)
     for (unsigned i = 0; i < n; ++i) permutation_io[i] = perm.perm[i];
   return status;
