@@ -82,11 +82,13 @@ static_assert(sizeof(block_op) == 40, "read as five 64-bit words");
 enum block_pass_kind { BLOCK_PASS_SEGMENT = 0, BLOCK_PASS_SINGLE = 1 };
 enum block_pass_flags {
   BLOCK_PASS_LOADS = 1,  // the first pass: its groups come straight from the state
-  BLOCK_PASS_STORES = 2  // the last pass: its groups go straight to the state
+  BLOCK_PASS_STORES = 2, // the last pass: its groups go straight to the state
+  BLOCK_PASS_LINEAR = 4  // every move is linear in the index bits (X, CNOT, SWAP: at most one local condition)
 };
 struct block_pass {
   uint8_t kind, num_ops, num_moves, flags;
-  uint8_t group[4];  // ascending local bits of the group (L - 9 of them)
+  uint8_t group[4];   // ascending local bits of the group (L - 9 of them)
+  uint8_t qubits[4];  // ... and the physical qubits they are
   uint16_t first_op, pad;
 };
 
@@ -97,7 +99,7 @@ struct block_header {
   uint16_t ops_at, coefs_at;  // byte offsets from the header: the ops, the coefficients (double)
   uint8_t pos[16];      // ascending physical qubits of the local bits
 };
-static_assert(sizeof(block_header) == 32 && sizeof(block_pass) == 12, "packed");
+static_assert(sizeof(block_header) == 32 && sizeof(block_pass) == 16, "packed");
 
 // A block's program with room for every block.
 constexpr int BLOCK_COEFS = 8;  // at most, per op
@@ -117,9 +119,9 @@ struct alignas(8) block_args {
   uint8_t data[BLOCK_ARG_BYTES - sizeof(block_header)];
 };
 // Room the ops may take in the arguments, each itself, a pass and its coefficients (beside the
-// alignment of the ops and the coefficients read past the last ones).
+// coefficients read past the last ones).
 constexpr size_t BLOCK_ARG_ROOM =
-    BLOCK_ARG_BYTES - sizeof(block_header) - sizeof(double) - BLOCK_COEFS * sizeof(double);
+    BLOCK_ARG_BYTES - sizeof(block_header) - BLOCK_COEFS * sizeof(double);
 inline int block_op_coefs(const gate_desc& d) {
   if (d.mode == BLOCK_MATRIX) return 8;
   if (d.mode == BLOCK_ESWAP) return 4;

@@ -341,18 +341,21 @@ __device__ __forceinline__ uint64_t chunk_base(uint64_t c, const block_view& v, 
   return c;
 }
 
-// Physical offset of local index t + (k << BLOCK_THREAD_BITS): the bits of t, and of k.
-__device__ __forceinline__ uint64_t thread_offset(uint32_t t, const block_view& v) {
-  uint64_t low = 0;
+// Physical offset of local index t + (k << BLOCK_THREAD_BITS): the bits of t, and of k.  I: the type
+// of an amplitude index (32 bits up to 32 qubits: half the instructions).
+template <typename I>
+__device__ __forceinline__ I thread_offset(uint32_t t, const block_view& v) {
+  I low = 0;
 #pragma unroll
-  for (int r = 0; r < BLOCK_THREAD_BITS; ++r) low |= (uint64_t)((t >> r) & 1u) << v.h->pos[r];
+  for (int r = 0; r < BLOCK_THREAD_BITS; ++r) low |= (I)((t >> r) & 1u) << v.h->pos[r];
   return low;
 }
-__device__ __forceinline__ uint64_t high_offset(int k, const block_view& v) {
-  uint64_t d = 0;
+template <typename I>
+__device__ __forceinline__ I high_offset(int k, const block_view& v) {
+  I d = 0;
 #pragma unroll
   for (int b = 0; b < 4; ++b)
-    if ((k >> b) & 1) d |= 1ull << v.h->pos[BLOCK_THREAD_BITS + b];
+    if ((k >> b) & 1) d |= (I)1 << v.h->pos[BLOCK_THREAD_BITS + b];
   return d;
 }
 
@@ -586,12 +589,20 @@ __device__ __forceinline__ void segment_gate(cpx<R> (&x)[PER], uint32_t base, co
 }
 
 // The physical offset of local index j.
-template <int L>
-__device__ __forceinline__ uint64_t local_offset(uint32_t j, const block_view& v) {
-  uint64_t d = 0;
+template <typename I, int L>
+__device__ __forceinline__ I local_offset(uint32_t j, const block_view& v) {
+  I d = 0;
 #pragma unroll
-  for (int r = 0; r < L; ++r) d |= (uint64_t)((j >> r) & 1u) << v.h->pos[r];
+  for (int r = 0; r < L; ++r) d |= (I)((j >> r) & 1u) << v.h->pos[r];
   return d;
+}
+
+// Where an X, CNOT or SWAP (linear moves: see BLOCK_PASS_LINEAR) sends local index j; the constant
+// part of X only if `affine`, so that images of index differences follow too.
+__device__ __forceinline__ uint32_t move_linear(uint32_t j, const block_gate& op, bool affine) {
+  if (op.cond == 0) return affine ? j ^ op.flip : j;
+  const uint32_t tested = (op.flip & op.cond) ? op.flip : op.cond;  // SWAP: where its two bits differ
+  return j ^ ((__popc(j & tested) & 1) ? op.flip : 0u);
 }
 
 // One workgroup per chunk of exactly PER * BLOCK_THREADS amplitudes
@@ -606,11 +617,12 @@ __device__ __forceinline__ uint64_t local_offset(uint32_t j, const block_view& v
 // their way while a gate runs: they are scalar loads of about 0.1 us each, which a chunk
 // that has its CU to itself would otherwise wait for.
 // Bound: the HBM round trip of the chunks (about 2.9 ms of a 29-qubit c128 state's 17.2 GB) plus what
-// the two workgroups of a CU do not hide of it in instructions: 4.1 ms a launch of 16 gates (4.2 TB/s)
-// on that state, 3.8 ms a launch of 8 with every qubit local and an LDS round trip per pass.  Waves of
+// the two workgroups of a CU do not hide of it in instructions: 4.0 ms a launch of 16 gates (4.3 TB/s)
+// on that state (4.4 ms with 64-bit indices and every move applied to every amplitude's index; 3.8 ms a
+// launch of 8 gates with every qubit local and an LDS round trip per pass).  Waves of
 // 16 amplitudes per lane (256 threads) run large states 1-2 % faster and small ones 15 % slower;
 // 1024 threads, which do not fit twice on a CU, half as fast.
-template <typename R, bool NT, int PER>
+template <typename R, bool NT, int PER, typename I>
 __global__ __launch_bounds__(BLOCK_THREADS, BLOCK_WAVES_PER_SIMD) void k_block(cpx<R>* __restrict__ s, block_args) {
   constexpr int GB = PER == 1 ? 0 : PER == 2 ? 1 : PER == 4 ? 2 : PER == 8 ? 3 : 4;
   constexpr int L = BLOCK_THREAD_BITS + GB;
@@ -621,10 +633,10 @@ __global__ __launch_bounds__(BLOCK_THREADS, BLOCK_WAVES_PER_SIMD) void k_block(c
   const uint32_t t = threadIdx.x;
   const uint32_t npasses = v.h->num_passes;
   if (!(v.passes[0].flags & BLOCK_PASS_LOADS)) {
-    const uint64_t low = chunk | thread_offset(t, v);
+    const I low = (I)chunk | thread_offset<I>(t, v);
 #pragma unroll
     for (uint32_t k = 0; k < PER; ++k)
-      lds[block_slot(t + BLOCK_THREADS * k)] = load_amp<NT>(s + (low | high_offset(k, v)));
+      lds[block_slot(t + BLOCK_THREADS * k)] = load_amp<NT>(s + (low | high_offset<I>(k, v)));
     __syncthreads();
   }
   for (uint32_t pi = 0; pi < npasses; ++pi) {
@@ -640,24 +652,33 @@ __global__ __launch_bounds__(BLOCK_THREADS, BLOCK_WAVES_PER_SIMD) void k_block(c
     const uint32_t num_ops = pass->num_ops, num_moves = pass->num_moves, flags = pass->flags;
     const uint32_t last = first + (num_ops ? num_ops - 1 : 0);
     op_words cur = load_op(v, first);
-    uint32_t base = t, dep[PER];
-    dep[0] = 0;
+    uint32_t base = t, bit[GB + 1];
 #pragma unroll
     for (int i = 0; i < GB; ++i) {
       const uint32_t q = pass->group[i];
       base = ((base >> q) << (q + 1)) | (base & ((1u << q) - 1u));
-#pragma unroll
-      for (int m = 0; m < (1 << i); ++m) dep[m | 1 << i] = dep[m] | 1u << q;
+      bit[i] = 1u << q;
     }
     cpx<R> x[PER];
     if (flags & BLOCK_PASS_LOADS) {
-      const uint64_t low = chunk | local_offset<L>(base, v);
+      const I low = (I)chunk | local_offset<I, L>(base, v);
+      I high[PER];
+      high[0] = 0;
 #pragma unroll
-      for (int m = 0; m < PER; ++m) x[m] = load_amp<NT>(s + (low | local_offset<L>(dep[m], v)));
+      for (int i = 0; i < GB; ++i)
+#pragma unroll
+        for (int m = 0; m < (1 << i); ++m) high[m | 1 << i] = high[m] | (I)1 << pass->qubits[i];
+#pragma unroll
+      for (int m = 0; m < PER; ++m) x[m] = load_amp<NT>(s + (low | high[m]));
     } else {
-      const uint32_t slot = block_slot(base);  // (the swizzle is linear)
+      uint32_t slot[PER];
+      slot[0] = block_slot(base);  // (the swizzle is linear)
 #pragma unroll
-      for (int m = 0; m < PER; ++m) x[m] = lds[slot ^ block_slot(dep[m])];
+      for (int i = 0; i < GB; ++i)
+#pragma unroll
+        for (int m = 0; m < (1 << i); ++m) slot[m | 1 << i] = slot[m] ^ block_slot(bit[i]);
+#pragma unroll
+      for (int m = 0; m < PER; ++m) x[m] = lds[slot[m]];
     }
     for (uint32_t o = 0; o < num_ops; ++o) {
       const op_words next = load_op(v, min(first + o + 1, last));
@@ -667,30 +688,60 @@ __global__ __launch_bounds__(BLOCK_THREADS, BLOCK_WAVES_PER_SIMD) void k_block(c
       if (acts_on(op, chunk)) segment_gate(x, base, op, chunk);
       cur = next;
     }
+    // where the moves send the amplitudes: linear ones act on the thread's base and, the same for all
+    // threads, on the group's bits
+    const bool linear = (flags & BLOCK_PASS_LINEAR) != 0;
     uint32_t j[PER];
+    if (linear) {
+      for (uint32_t o = first + num_ops; o < first + num_ops + num_moves; ++o) {
+        const double none[8] = {};
+        const block_gate op = decode(load_op(v, o), none);
+        if (!acts_on(op, chunk)) continue;
+        base = move_linear(base, op, true);
 #pragma unroll
-    for (int m = 0; m < PER; ++m) j[m] = base | dep[m];
-    for (uint32_t o = first + num_ops; o < first + num_ops + num_moves; ++o) {
-      const op_words w = load_op(v, o);
-      const double none[8] = {};
-      const block_gate op = decode(w, none);
-      if (!acts_on(op, chunk)) continue;
-      const uint32_t flip = op.flip;
-      if ((flip & op.cond) == 0) {  // X, CNOT
+        for (int i = 0; i < GB; ++i) bit[i] = move_linear(bit[i], op, false);
+      }
+    }
+    j[0] = base;
 #pragma unroll
-        for (int m = 0; m < PER; ++m) j[m] ^= (j[m] & op.cond) == op.cond ? flip : 0u;
-      } else {  // SWAP: both members of a pair, the one with the pair bit clear has the cond bits set
-        const uint32_t tested = op.cond | 1u << op.pair_bit;
+    for (int i = 0; i < GB; ++i)
 #pragma unroll
-        for (int m = 0; m < PER; ++m)
-          j[m] ^= (j[m] & tested) == op.cond || ((j[m] ^ flip) & tested) == op.cond ? flip : 0u;
+      for (int m = 0; m < (1 << i); ++m) j[m | 1 << i] = j[m] ^ bit[i];
+    if (!linear) {
+      for (uint32_t o = first + num_ops; o < first + num_ops + num_moves; ++o) {
+        const double none[8] = {};
+        const block_gate op = decode(load_op(v, o), none);
+        if (!acts_on(op, chunk)) continue;
+        const uint32_t flip = op.flip;
+        if ((flip & op.cond) == 0) {  // X
+#pragma unroll
+          for (int m = 0; m < PER; ++m) j[m] ^= (j[m] & op.cond) == op.cond ? flip : 0u;
+        } else {  // SWAP: both members of a pair, the one with the pair bit clear has the cond bits set
+          const uint32_t tested = op.cond | 1u << op.pair_bit;
+#pragma unroll
+          for (int m = 0; m < PER; ++m)
+            j[m] ^= (j[m] & tested) == op.cond || ((j[m] ^ flip) & tested) == op.cond ? flip : 0u;
+        }
       }
     }
     if (flags & BLOCK_PASS_STORES) {
       // (without moves: the very addresses this thread loaded; with moves the chunk's loads ended
       // before an earlier pass's barrier)
+      if (linear) {
+        I at[PER];
+        at[0] = (I)chunk | local_offset<I, L>(base, v);
 #pragma unroll
-      for (int m = 0; m < PER; ++m) store_amp<NT>(s + (chunk | local_offset<L>(j[m], v)), x[m]);
+        for (int i = 0; i < GB; ++i) {
+          const I d = local_offset<I, L>(bit[i], v);
+#pragma unroll
+          for (int m = 0; m < (1 << i); ++m) at[m | 1 << i] = at[m] ^ d;
+        }
+#pragma unroll
+        for (int m = 0; m < PER; ++m) store_amp<NT>(s + at[m], x[m]);
+      } else {
+#pragma unroll
+        for (int m = 0; m < PER; ++m) store_amp<NT>(s + ((I)chunk | local_offset<I, L>(j[m], v)), x[m]);
+      }
       return;
     }
     if (num_moves && !(flags & BLOCK_PASS_LOADS)) __syncthreads();  // every group is read before the first is written
@@ -698,10 +749,10 @@ __global__ __launch_bounds__(BLOCK_THREADS, BLOCK_WAVES_PER_SIMD) void k_block(c
     for (int m = 0; m < PER; ++m) lds[block_slot(j[m])] = x[m];
     __syncthreads();
   }
-  const uint64_t low = chunk | thread_offset(t, v);
+  const I low = (I)chunk | thread_offset<I>(t, v);
 #pragma unroll
   for (uint32_t k = 0; k < PER; ++k)
-    store_amp<NT>(s + (low | high_offset(k, v)), lds[block_slot(t + BLOCK_THREADS * k)]);
+    store_amp<NT>(s + (low | high_offset<I>(k, v)), lds[block_slot(t + BLOCK_THREADS * k)]);
 }
 
 typedef const __attribute__((address_space(4))) adjoint_base* cbase;
@@ -838,15 +889,6 @@ __device__ __forceinline__ void group_pairs(cpx<R> (&x)[PER], const uint32_t (&j
 // the plain arithmetic; the RX / RY / RZ-type parametric forms use fused
 // multiply-adds (the sweep's results are sums, not amplitudes compared bitwise).
 typedef const __attribute__((address_space(4))) adjoint_block_program* cadjoint;
-
-// A lane's value from another lane of its row by a DPP control (both 32-bit halves).  Every
-// control used below selects a lane inside the row, so all lanes read a valid source.
-template <int CTRL>
-__device__ __forceinline__ double dpp_f64(double v) {
-  const int lo = __double2loint(v), hi = __double2hiint(v);
-  return __hiloint2double(__builtin_amdgcn_update_dpp(0, hi, CTRL, 0xF, 0xF, false),
-                          __builtin_amdgcn_update_dpp(0, lo, CTRL, 0xF, 0xF, false));
-}
 
 // The sum of v over the 64 lanes of the wave, in a fixed order, without LDS traffic: pairs and
 // quads (quad permutations), 8 and 16 lanes (half-row and row mirrors; every lane then holds
@@ -1281,7 +1323,10 @@ unsigned block_run_qubits(int dtype) {
 
 template <typename R, bool NT, int PER>
 static int launch_block_inst(uint64_t chunks, hipStream_t st, cpx<R>* s, const block_args& p) {
-  hipLaunchKernelGGL((k_block<R, NT, PER>), dim3((unsigned)chunks), dim3(BLOCK_THREADS), 0, st, s, p);
+  if (chunks << p.h.num_local <= 1ull << 32)
+    hipLaunchKernelGGL((k_block<R, NT, PER, uint32_t>), dim3((unsigned)chunks), dim3(BLOCK_THREADS), 0, st, s, p);
+  else
+    hipLaunchKernelGGL((k_block<R, NT, PER, uint64_t>), dim3((unsigned)chunks), dim3(BLOCK_THREADS), 0, st, s, p);
   return BRK_OK;
 }
 

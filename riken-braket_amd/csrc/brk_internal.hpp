@@ -83,6 +83,15 @@ __device__ __forceinline__ cpx<float> cflip(cpx<float> a, uint32_t sign) {
   return {__uint_as_float(__float_as_uint(a.re) ^ sign), __uint_as_float(__float_as_uint(a.im) ^ sign)};
 }
 
+// A lane's value from another lane of its row by a DPP control (both 32-bit halves).  Every
+// control used below selects a lane inside the row, so all lanes read a valid source.
+template <int CTRL>
+__device__ __forceinline__ double dpp_f64(double v) {
+  const int lo = __double2loint(v), hi = __double2hiint(v);
+  return __hiloint2double(__builtin_amdgcn_mov_dpp(hi, CTRL, 0xF, 0xF, true),
+                          __builtin_amdgcn_mov_dpp(lo, CTRL, 0xF, 0xF, true));
+}
+
 inline size_t amp_bytes(int dtype) { return dtype == BRK_C128 ? 16 : 8; }
 
 // One amplitude as a native 2-vector, so that it can carry the non-temporal

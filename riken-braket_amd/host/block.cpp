@@ -107,7 +107,10 @@ static void make_passes(block_program& prog, unsigned line_bits) {
     for (unsigned b = L; b-- > 0 && (unsigned)__builtin_popcount(bits) < gb;) bits |= 1u << b;
     unsigned k = 0;
     for (unsigned b = 0; b < L; ++b)
-      if (bits >> b & 1u) p.group[k++] = (uint8_t)b;
+      if (bits >> b & 1u) {
+        p.qubits[k] = prog.h.pos[b];
+        p.group[k++] = (uint8_t)b;
+      }
     // straight from or to the state where every access covers whole lines.  A segment that loads
     // and moves stores by way of LDS: another thread may not have loaded the target yet.
     if (prog.h.num_passes == 1 && !(bits & line)) p.flags |= BLOCK_PASS_LOADS;
@@ -127,7 +130,14 @@ static void make_passes(block_program& prog, unsigned line_bits) {
       }
       order[placed++] = o;
     }
-    for (uint32_t i : moves) order[placed++] = prog.ops[i];
+    bool linear = true;
+    for (uint32_t i : moves) {
+      const block_op& o = prog.ops[i];
+      const uint32_t tested = o.cond & (uint32_t)~o.flip;  // (a SWAP's own condition lies in its flip)
+      linear &= (o.cond & o.flip) ? tested == 0 : (unsigned)__builtin_popcount(tested) <= 1;
+      order[placed++] = o;
+    }
+    if (linear) p.flags |= BLOCK_PASS_LINEAR;
     gates.clear();
     moves.clear();
     bits = moved = moved_by = 0;
@@ -284,7 +294,6 @@ static void pack(const block_program& prog, block_args* out) {
     at += bytes;
   };
   put(prog.passes, sizeof(block_pass) * prog.h.num_passes);
-  if (prog.h.num_passes & 1u) at += 4;  // 64-bit words follow
   out->h.ops_at = (uint16_t)(at - reinterpret_cast<char*>(out));
   put(prog.ops, sizeof(block_op) * prog.h.num_ops);
   out->h.coefs_at = (uint16_t)(at - reinterpret_cast<char*>(out));
