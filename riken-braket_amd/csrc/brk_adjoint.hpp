@@ -41,4 +41,9 @@ struct sign_terms {
 };
 int launch_sign_terms(const sign_terms& t, void* first, uint64_t size, int dtype, void* stream);
 
+// The block partials of <b|a> (INNER_BLOCKS pairs, real and imaginary part) without waiting for them;
+// their sum in order is brk_inner_product's result.
+constexpr int INNER_BLOCKS = 1024;
+int launch_inner_partials(const void* a, const void* b, uint64_t size, int dtype, double* partials, void* stream);
+
 }  // namespace brk

@@ -10,6 +10,7 @@
 // partials and then std::accumulate's them, inner_product.hpp:43-55; spin
 // values use long double, spin_expectation_value.hpp:31-64).
 #include "brk_internal.hpp"
+#include "brk_adjoint.hpp"
 #include "brk_block.hpp"
 
 #include <algorithm>
@@ -726,6 +727,17 @@ static int noalloc_scratch(int device, double** out) {
   }
   *out = g_noalloc_ptr[device];
   return BRK_OK;
+}
+
+static_assert(INNER_BLOCKS == RED_BLOCKS, "one grid");
+int launch_inner_partials(const void* a, const void* b, uint64_t size, int dtype, double* partials, void* stream) {
+  if (dtype == BRK_C128)
+    hipLaunchKernelGGL((k_inner<double, double>), dim3(RED_BLOCKS), dim3(RED_THREADS), 0, as_stream(stream),
+                       (const cpx<double>*)a, (const cpx<double>*)b, size, partials);
+  else
+    hipLaunchKernelGGL((k_inner<float, float>), dim3(RED_BLOCKS), dim3(RED_THREADS), 0, as_stream(stream),
+                       (const cpx<float>*)a, (const cpx<float>*)b, size, partials);
+  return check_launch("inner product");
 }
 
 constexpr int ROW_THREADS = 256;

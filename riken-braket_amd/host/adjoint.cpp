@@ -27,12 +27,14 @@
 #include "circuit.hpp"
 #include "brk_adjoint.hpp"
 #include "brk_block.hpp"
+#include "sweep.hpp"
 
 #include <hip/hip_runtime_api.h>
 
 #include <algorithm>
 #include <array>
 #include <complex>
+#include <cstring>
 #include <memory>
 #include <mutex>
 #include <vector>
@@ -222,6 +224,8 @@ struct partials_slot {
   std::mutex busy;
   double* ptr = nullptr;
   size_t doubles = 0;
+  char* pinned = nullptr;  // staging of the sweeps' programs
+  size_t pinned_bytes = 0;
 };
 static std::mutex g_partials_mutex;
 static std::vector<std::unique_ptr<partials_slot>> g_partials;
@@ -229,6 +233,7 @@ static std::vector<std::unique_ptr<partials_slot>> g_partials;
 struct partials_lease {
   std::unique_lock<std::mutex> hold;
   double* ptr = nullptr;
+  char* pinned = nullptr;
   hipStream_t stream = nullptr;
   // an early return may leave kernels that write the buffer in flight: drain them first
   ~partials_lease() {
@@ -236,7 +241,7 @@ struct partials_lease {
   }
 };
 
-static int get_partials(size_t doubles, hipStream_t stream, partials_lease& lease) {
+static int get_partials(size_t doubles, size_t pinned_bytes, hipStream_t stream, partials_lease& lease) {
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess) return fail(BRK_ERR_HIP, "hipGetDevice failed");
   partials_slot* slot = nullptr;
@@ -257,7 +262,18 @@ static int get_partials(size_t doubles, hipStream_t stream, partials_lease& leas
     }
     slot->doubles = doubles;
   }
+  if (slot->pinned_bytes < pinned_bytes) {
+    if (slot->pinned) (void)hipHostFree(slot->pinned);
+    slot->pinned = nullptr;
+    slot->pinned_bytes = 0;
+    if (hipHostMalloc((void**)&slot->pinned, pinned_bytes) != hipSuccess) {
+      slot->pinned = nullptr;
+      return fail(BRK_ERR_OUT_OF_MEMORY, "cannot allocate %zu bytes of pinned memory", pinned_bytes);
+    }
+    slot->pinned_bytes = pinned_bytes;
+  }
   lease.hold = std::move(hold);
+  lease.pinned = slot->pinned;
   lease.ptr = slot->ptr;
   lease.stream = stream;
   return BRK_OK;
@@ -449,7 +465,7 @@ static int blocked_gradient(const brk_circuit* given, const std::vector<int>& gi
   const size_t nsums = std::max(1u, nparams);
   const size_t bytes = sizeof(adjoint_block_program) * programs.size();
   partials_lease lease;
-  if (int s = get_partials((size_t)nparams * chunks + nsums + (bytes + sizeof(double) - 1) / sizeof(double), st, lease))
+  if (int s = get_partials((size_t)nparams * chunks + nsums + (bytes + sizeof(double) - 1) / sizeof(double), 0, st, lease))
     return s;
   double* partials = lease.ptr;
   double* sums = partials + (size_t)nparams * chunks;
@@ -464,6 +480,90 @@ static int blocked_gradient(const brk_circuit* given, const std::vector<int>& gi
     status = fail(BRK_ERR_HIP, "copying the gradient failed");
   if (hipStreamSynchronize(st) != hipSuccess && !status) status = fail(BRK_ERR_HIP, "hipStreamSynchronize failed");
   return status;
+}
+
+// A gate of the sweeps from op o (uncontrolled one-qubit ops, Z and CZ): U forward, U^dagger and the
+// parameter's D in the reverse sweep.
+static bool to_sweep_gate(const brk_circuit::op& o, int param, bool reverse, sweep_gate* g) {
+  *g = sweep_gate{};
+  uint32_t d;
+  uint64_t a;
+  if (sign_term_of(o, &d, &a)) {
+    g->sign = true;
+    g->mask = (uint32_t)(a | a << d);
+    return true;
+  }
+  if (!chainable(o)) return false;
+  adj_op m;
+  if (!make_adj_op(o, m)) return false;
+  g->q = o.targets[0];
+  // U^dagger's diagonal is U's conjugated; its off-diagonal entries change places as well
+  for (int r = 0; r < 2; ++r)
+    for (int c = 0; c < 2; ++c) {
+      const int from = reverse ? 2 * r + c : 2 * c + r;
+      g->u[2 * (2 * r + c)] = m.m[2 * from];
+      g->u[2 * (2 * r + c) + 1] = reverse ? m.m[2 * from + 1] : -m.m[2 * from + 1];
+    }
+  switch (o.code) {  // by the op, not by zeros: D's form is the op's
+    case BRK_OP_RZ: case BRK_OP_EZ: case BRK_OP_U1: g->diagonal = true; break;
+    case BRK_OP_RX: case BRK_OP_EX: case BRK_OP_RY: case BRK_OP_EY: break;
+    default: g->diagonal = g->u[2] == 0.0 && g->u[3] == 0.0 && g->u[4] == 0.0 && g->u[5] == 0.0;
+  }
+  if (reverse) {
+    g->param = param;
+    std::copy(m.d, m.d + 8, g->d);
+  }
+  return true;
+}
+
+// The gradient of a circuit of uncontrolled one-qubit ops, Z and CZ in merged sweeps (csrc/brk_sweep.hpp).
+// Blocks are launched as they are planned: the host plans the reverse sweep while the device runs the
+// forward pass, and nothing waits for the device before the end.
+static int sweep_gradient(const std::vector<sweep_gate>& forward_gates, const std::vector<sweep_gate>& reverse_gates,
+                          unsigned n, unsigned nparams, void* psi, void* lam, int dtype, const double* J,
+                          const double* h, double* energy, double* gradient, void* stream) {
+  const uint64_t size = 1ull << n;
+  hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+  const unsigned line_bits = dtype == BRK_C128 ? 3 : 4;  // one 128-byte line
+  const unsigned L = dtype == BRK_C128 ? SWEEP_REVERSE_LOCAL_C128 : SWEEP_REVERSE_LOCAL_C64;
+  const uint64_t chunks = size >> L;
+  // one leased buffer: nparams x chunks partials, the nparams gradients, the energy's partials, then
+  // the programs, which go up from pinned memory
+  const size_t nsums = std::max(1u, nparams), room = 2 * sweep_program_bound(forward_gates.size());
+  const size_t doubles = (size_t)nparams * chunks + nsums + 2 * INNER_BLOCKS;
+  partials_lease lease;
+  if (int s = get_partials(doubles + room / sizeof(double) + 8, room, st, lease)) return s;
+  double* partials = lease.ptr;
+  double* sums = partials + (size_t)nparams * chunks;
+  double* energy_partials = sums + nsums;
+  char* device = reinterpret_cast<char*>(((uintptr_t)(energy_partials + 2 * INNER_BLOCKS) + 63) & ~(uintptr_t)63);
+  size_t used = 0;
+  auto run = [&](const std::vector<sweep_gate>& gates, unsigned num_local, void* second) {
+    return plan_sweep(gates, n, num_local, line_bits, [&](const void* program, size_t bytes) -> int {
+      if (used + bytes > room) return fail(BRK_ERR_INVALID_ARGUMENT, "sweep programs outgrow their buffer");
+      std::memcpy(lease.pinned + used, program, bytes);
+      if (hipMemcpyAsync(device + used, lease.pinned + used, bytes, hipMemcpyHostToDevice, st) != hipSuccess)
+        return fail(BRK_ERR_HIP, "uploading the sweep programs failed");
+      const int status = launch_sweep(device + used, num_local, psi, second, size, dtype, partials, stream);
+      used += bytes;
+      return status;
+    });
+  };
+  int status = run(forward_gates, SWEEP_FORWARD_LOCAL, nullptr);
+  if (!status) status = brk_apply_ising(lam, psi, size, dtype, J, h, stream);
+  if (!status) status = launch_inner_partials(lam, psi, size, dtype, energy_partials, stream);
+  if (!status) status = run(reverse_gates, L, lam);
+  if (!status) status = sum_gradient_partials(partials, nparams, chunks, 2.0, sums, stream);
+  std::vector<double> host(nsums + 2 * INNER_BLOCKS);
+  if (!status && hipMemcpyAsync(host.data(), sums, host.size() * sizeof(double), hipMemcpyDeviceToHost, st) != hipSuccess)
+    status = fail(BRK_ERR_HIP, "copying the gradient failed");
+  if (hipStreamSynchronize(st) != hipSuccess && !status) status = fail(BRK_ERR_HIP, "hipStreamSynchronize failed");
+  if (status) return status;
+  std::copy(host.begin(), host.begin() + nparams, gradient);
+  double e = 0.0;
+  for (int b = 0; b < INNER_BLOCKS; ++b) e += host[nsums + 2 * b];
+  *energy = e;
+  return BRK_OK;
 }
 
 }  // namespace brk
@@ -513,6 +613,21 @@ int brk_adjoint_ising_gradient(const brk_circuit* circuit, void* psi, void* work
     for (unsigned q : o.controls) m |= 1ull << q;
     if ((unsigned)__builtin_popcountll(m) > L) all_fit = false;
   }
+  const unsigned n = circuit->num_qubits;
+  if (adjoint_blocks_enabled() && n >= (unsigned)SWEEP_FORWARD_LOCAL && n <= (unsigned)SWEEP_MAX_QUBITS) {
+    std::vector<sweep_gate> up, down;  // forward, and the inverses last first
+    sweep_gate g;
+    bool simple = true;
+    for (size_t i = 0; simple && i < ops.size(); ++i) {
+      simple = to_sweep_gate(ops[i], -1, false, &g);
+      up.push_back(g);
+    }
+    for (size_t i = ops.size(); simple && i-- > 0;) {
+      simple = to_sweep_gate(ops[i], pidx[i], true, &g);
+      down.push_back(g);
+    }
+    if (simple) return sweep_gradient(up, down, n, nparams, psi, work, dtype, J, h, energy, gradient, stream);
+  }
   if (adjoint_blocks_enabled() && circuit->num_qubits >= L && all_fit)
     return blocked_gradient(circuit, pidx, nparams, psi, work, dtype, J, h, energy, gradient, stream);
   const uint64_t size = 1ull << circuit->num_qubits;
@@ -529,7 +644,7 @@ int brk_adjoint_ising_gradient(const brk_circuit* circuit, void* psi, void* work
   size_t nchains = 0;
   for (size_t i = 0; i < ops.size(); ++i) nchains += chainable(ops[i]) ? 1 : 0;  // upper bound
   partials_lease lease;
-  if (int s = get_partials(std::max<size_t>(1, nchains) * ADJ_MAX_CHAIN * ADJ_BLOCKS, st, lease)) return s;
+  if (int s = get_partials(std::max<size_t>(1, nchains) * ADJ_MAX_CHAIN * ADJ_BLOCKS, 0, st, lease)) return s;
   double* partials = lease.ptr;
   struct slot {
     int param;

@@ -1,0 +1,290 @@
+// Planner of the adjoint gradient's sweeps: blocks, segments and macros (csrc/brk_sweep.hpp).
+//
+// A mixing gate depends on the gates before it on its qubit; a diagonal gate (phase or sign) only on
+// the mixing gates before it, since diagonal gates commute.  Blocks, and the segments of a block, are
+// built greedily: one qubit at a time is added to the set -- the block's local qubits, the segment's
+// group -- that lets the most gates run, where gates on one qubit need it in the set and signs run
+// anywhere.  On a layered ansatz that walks the light cone: a block takes a triangle or parallelogram
+// of layers and qubits, a segment up to three layers of three qubits.
+#include "sweep.hpp"
+
+#include <algorithm>
+#include <cstring>
+
+namespace brk {
+
+namespace {
+
+struct planner {
+  const std::vector<sweep_gate>& gates;
+  unsigned n;
+  std::vector<std::vector<uint32_t>> succ;
+  std::vector<uint32_t> indeg;
+  std::vector<uint32_t> ready;  // runnable gates, any order
+  std::vector<uint32_t> stamp, left;
+  uint32_t now = 0;
+  std::vector<uint32_t> stack;
+
+  uint32_t qubits(const sweep_gate& g) const { return g.sign ? g.mask : 1u << g.q; }
+
+  planner(const std::vector<sweep_gate>& g, unsigned num_qubits) : gates(g), n(num_qubits) {
+    const uint32_t count = (uint32_t)gates.size();
+    succ.assign(count, {});
+    indeg.assign(count, 0);
+    stamp.assign(count, 0);
+    left.assign(count, 0);
+    std::vector<long> last_mix(n, -1);
+    std::vector<std::vector<uint32_t>> since(n);  // diagonal gates on a qubit since its last mixing gate
+    for (uint32_t i = 0; i < count; ++i) {
+      const sweep_gate& gate = gates[i];
+      auto after = [&](uint32_t j) {
+        succ[j].push_back(i);
+        ++indeg[i];
+      };
+      if (gate.sign || gate.diagonal) {
+        for (uint32_t m = qubits(gate); m; m &= m - 1) {
+          const unsigned q = (unsigned)__builtin_ctz(m);
+          if (last_mix[q] >= 0) after((uint32_t)last_mix[q]);
+          since[q].push_back(i);
+        }
+      } else {
+        for (uint32_t j : since[gate.q]) after(j);
+        if (since[gate.q].empty() && last_mix[gate.q] >= 0) after((uint32_t)last_mix[gate.q]);
+        since[gate.q].clear();
+        last_mix[gate.q] = (long)i;
+      }
+      if (!indeg[i]) ready.push_back(i);
+    }
+  }
+
+  bool runs_in(uint32_t i, uint32_t set) const { return gates[i].sign || (set >> gates[i].q & 1u); }
+
+  // How many one-qubit gates (at most `budget`) could run within the set.
+  unsigned closure(uint32_t set, unsigned budget) {
+    ++now;
+    stack.clear();
+    for (uint32_t i : ready)
+      if (runs_in(i, set)) stack.push_back(i);
+    unsigned got = 0;
+    while (!stack.empty() && got < budget) {
+      const uint32_t i = stack.back();
+      stack.pop_back();
+      got += gates[i].sign ? 0 : 1;
+      for (uint32_t j : succ[i]) {
+        if (stamp[j] != now) {
+          stamp[j] = now;
+          left[j] = indeg[j];
+        }
+        if (--left[j] == 0 && runs_in(j, set)) stack.push_back(j);
+      }
+    }
+    return got;
+  }
+
+  // `set` with up to `room` of the candidates added, each the one that lets the most gates run.
+  uint32_t grow(uint32_t set, uint32_t candidates, unsigned room, unsigned budget) {
+    unsigned have = closure(set, budget);
+    while (room) {
+      unsigned best = have;
+      uint32_t bit = 0;
+      for (uint32_t m = candidates & ~set; m; m &= m - 1) {
+        const uint32_t b = m & (0u - m);
+        const unsigned c = closure(set | b, budget);
+        if (c > best) {
+          best = c;
+          bit = b;
+        }
+      }
+      if (!bit) break;
+      set |= bit;
+      have = best;
+      --room;
+    }
+    return set;
+  }
+
+  void take(size_t k) {  // runs ready[k]
+    const uint32_t i = ready[k];
+    ready[k] = ready.back();
+    ready.pop_back();
+    for (uint32_t j : succ[i])
+      if (--indeg[j] == 0) ready.push_back(j);
+  }
+};
+
+using cd = std::complex<double>;
+
+// One macro: what can run of the gates on the group's qubits q[], or of any signs.
+sweep_macro make_macro(planner& p, const unsigned (&q)[SWEEP_GROUP], bool any_signs) {
+  sweep_macro mac{};
+  for (int32_t& s : mac.slot) s = -1;
+  uint32_t group = 0;
+  for (unsigned qubit : q) group |= 1u << qubit;
+  auto bit_of = [&](unsigned qubit) {
+    unsigned b = 0;
+    while (q[b] != qubit) ++b;
+    return b;
+  };
+  // signs: those on the group's qubits, then any others whose distance has a term (they cost nothing)
+  for (int round = 0; round < 2; ++round)
+    for (size_t k = 0; k < p.ready.size();) {
+      const sweep_gate& g = p.gates[p.ready[k]];
+      if (!g.sign || (round == 0 && !(g.mask & group) && !any_signs)) {
+        ++k;
+        continue;
+      }
+      const unsigned lo = (unsigned)__builtin_ctz(g.mask), hi = 31u - (unsigned)__builtin_clz(g.mask);
+      uint32_t t = 0;
+      while (t < mac.num_terms && mac.d[t] != hi - lo) ++t;
+      if (t == mac.num_terms) {
+        if (round == 1 || t == (uint32_t)SWEEP_MAX_TERMS) {
+          ++k;
+          continue;
+        }
+        mac.d[mac.num_terms++] = hi - lo;
+      }
+      mac.A[t] ^= 1u << lo;
+      p.take(k);
+    }
+  // phases of the group's qubits: one product per qubit, one with a parameter among them
+  cd phase[SWEEP_GROUP][2];
+  for (auto& f : phase) f[0] = f[1] = 1.0;
+  for (size_t k = 0; k < p.ready.size();) {
+    const sweep_gate& g = p.gates[p.ready[k]];
+    if (g.sign || !g.diagonal || !(group >> g.q & 1u)) {
+      ++k;
+      continue;
+    }
+    const unsigned b = bit_of(g.q);
+    if (g.param >= 0) {
+      if (mac.slot[b] >= 0) {
+        ++k;
+        continue;
+      }
+      mac.slot[b] = g.param;
+      mac.weight[b][0] = g.d[1];
+      mac.weight[b][1] = g.d[7];
+      mac.phase_grads |= 1u << b;
+    }
+    phase[b][0] *= cd(g.u[0], g.u[1]);
+    phase[b][1] *= cd(g.u[6], g.u[7]);
+    mac.phases = 1;
+    p.take(k);
+  }
+  // mixing gates, one per qubit (running one makes the qubit's next diagonal gates ready, not its
+  // next mixing gate, unless nothing lies between: the mask keeps to one)
+  uint32_t mixed = 0;
+  for (size_t k = 0; k < p.ready.size();) {
+    const sweep_gate& g = p.gates[p.ready[k]];
+    if (g.sign || g.diagonal || !(group & ~mixed & 1u << g.q)) {
+      ++k;
+      continue;
+    }
+    const unsigned b = bit_of(g.q);
+    const double* u = g.u;
+    std::copy(u, u + 8, mac.matrix[b]);
+    mac.mix[b] = u[1] == 0.0 && u[3] == 0.0 && u[5] == 0.0 && u[7] == 0.0   ? SWEEP_MIX_REAL
+                 : u[1] == 0.0 && u[2] == 0.0 && u[4] == 0.0 && u[7] == 0.0 ? SWEEP_MIX_X
+                                                                            : SWEEP_MIX_GENERAL;
+    if (g.param >= 0) {
+      mac.slot[SWEEP_GROUP + b] = g.param;
+      const bool y_form = g.d[3] == 0.0 && g.d[5] == 0.0;  // D = [[0, a], [b, 0]], else [[0, i a], [i b, 0]]
+      mac.form[b] = y_form ? SWEEP_FORM_Y : SWEEP_FORM_X;
+      mac.mix_weight[b][0] = y_form ? g.d[2] : g.d[3];
+      mac.mix_weight[b][1] = y_form ? g.d[4] : g.d[5];
+    }
+    mixed |= 1u << g.q;
+    p.take(k);
+    k = 0;  // (take reorders the list)
+  }
+  for (int32_t s : mac.slot) mac.any_grads |= s >= 0 ? 1u : 0u;
+  // the terms' parity over the group's own bits: into the table where there is one
+  for (uint32_t m = 0; m < (1u << SWEEP_GROUP); ++m) {
+    uint32_t xe = 0;
+    cd f = 1.0;
+    for (unsigned b = 0; b < (unsigned)SWEEP_GROUP; ++b) {
+      xe |= ((m >> b) & 1u) << q[b];
+      f *= phase[b][(m >> b) & 1u];
+    }
+    uint32_t odd = 0;
+    for (uint32_t t = 0; t < mac.num_terms; ++t) odd += (uint32_t)__builtin_popcount(xe & (xe >> mac.d[t]) & mac.A[t]);
+    if (odd & 1u) {
+      if (mac.phases) f = -f;
+      else mac.uniform |= 1u << m;
+    }
+    mac.phase[m][0] = f.real();
+    mac.phase[m][1] = f.imag();
+  }
+  return mac;
+}
+
+}  // namespace
+
+int plan_sweep(const std::vector<sweep_gate>& gates, unsigned n, unsigned num_local, unsigned line_bits,
+               const std::function<int(const void* program, size_t bytes)>& emit) {
+  planner p(gates, n);
+  const uint32_t all = n >= 32 ? ~0u : (1u << n) - 1u;
+  const uint32_t line = (1u << line_bits) - 1u;
+  constexpr unsigned BLOCK_BUDGET = 256;  // gates the greedy choice of local qubits looks ahead
+  // A segment goes on to another macro where it runs this many gates: a macro takes the time of about
+  // two exchanges through LDS whatever it runs (24 qubits, 12 layers: 151 reverse macros in 58
+  // segments; 178 in 56 with macros of any size).
+  constexpr unsigned CHAIN_GATES = 4;
+  std::vector<sweep_segment> segments;
+  std::vector<sweep_macro> macros;
+  std::vector<char> program;
+  while (!p.ready.empty()) {
+    // local qubits: the line's, the greedy ones, then the lowest others
+    uint32_t local = p.grow(line, all, num_local - line_bits, BLOCK_BUDGET);
+    for (unsigned q = 0; (unsigned)__builtin_popcount(local) < num_local; ++q) local |= 1u << q;
+    sweep_header h{};
+    unsigned rank[32] = {}, r = 0;
+    for (uint32_t m = local; m; m &= m - 1) {
+      const unsigned q = (unsigned)__builtin_ctz(m);
+      rank[q] = r;
+      h.pos[r++] = (uint8_t)q;
+    }
+    segments.clear();
+    macros.clear();
+    while (!p.ready.empty()) {
+      uint32_t group = p.grow(0, local, SWEEP_GROUP, 4 * SWEEP_GROUP * SWEEP_MAX_MACROS);
+      // without a gate for these qubits the block ends (signs wait for a block that needs them), or
+      // only signs are left
+      const bool only_signs = group == 0;
+      if (only_signs && p.closure(all, 1) != 0) break;
+      // filled up with the highest local qubits: lanes then cover whole lines
+      for (unsigned q = n; q-- > 0 && (unsigned)__builtin_popcount(group) < (unsigned)SWEEP_GROUP;)
+        if (local >> q & 1u) group |= 1u << q;
+      sweep_segment s{};
+      unsigned q[SWEEP_GROUP], k = 0;
+      uint32_t bits = 0;
+      for (uint32_t m = group; m; m &= m - 1) {
+        q[k] = (unsigned)__builtin_ctz(m);
+        s.group[k] = (uint8_t)rank[q[k]];
+        s.qubits[k] = (uint8_t)q[k];
+        bits |= 1u << rank[q[k]];
+        ++k;
+      }
+      s.first_macro = (uint16_t)macros.size();
+      do {
+        macros.push_back(make_macro(p, q, only_signs));
+        ++s.num_macros;
+      } while (s.num_macros < SWEEP_MAX_MACROS && !p.ready.empty() && (only_signs || p.closure(group, CHAIN_GATES) >= CHAIN_GATES));
+      if (!(bits & line)) s.flags = (uint8_t)(SWEEP_STORES | (segments.empty() ? SWEEP_LOADS : 0));
+      segments.push_back(s);
+    }
+    for (size_t k = 0; k + 1 < segments.size(); ++k) segments[k].flags &= (uint8_t)~SWEEP_STORES;
+    h.num_segments = (uint32_t)segments.size();
+    h.num_macros = (uint32_t)macros.size();
+    h.macros_at = (uint32_t)(sizeof(sweep_header) + segments.size() * sizeof(sweep_segment));
+    const size_t bytes = h.macros_at + macros.size() * sizeof(sweep_macro);
+    program.assign((bytes + 63) & ~(size_t)63, 0);
+    std::memcpy(program.data(), &h, sizeof(h));
+    std::memcpy(program.data() + sizeof(h), segments.data(), segments.size() * sizeof(sweep_segment));
+    std::memcpy(program.data() + h.macros_at, macros.data(), macros.size() * sizeof(sweep_macro));
+    if (int st = emit(program.data(), program.size())) return st;
+  }
+  return 0;
+}
+
+}  // namespace brk

@@ -133,6 +133,52 @@ def access(request):
         brk.tune("nt_min_bytes", old)
 
 
+def one_qubit_ansatz(n, rng, layers, long_range):
+    """every one-qubit kind, with parameters and without (angles of 0 among them), Z and CZ at any distance
+    (more distances than a macro holds, repeated pairs), qubits without gates"""
+    ops = []
+    for layer in range(layers):
+        for q in range(n - 1 if layer % 2 else n):
+            kind = ("RX", "RY", "RZ", "EX", "EY", "EZ", "U1")[int(rng.integers(7))]
+            ops.append((kind, (q,), (), (0.0 if rng.integers(8) == 0 else float(rng.uniform(-3, 3)),)))
+        for _ in range(n if long_range else 0):
+            a, b = (int(x) for x in rng.choice(n, 2, replace=False))
+            ops.append(("Z", (a,), (b,), ()) if rng.integers(2) else ("Z", (a, b), (), ()))
+        for q in range(0 if long_range else n - 1):
+            ops.append(("Z", (q, q + 1), (), ()))
+        for _ in range(3):
+            q = int(rng.integers(n))
+            ops.append((("H", (q,), (), ()), ("X", (q,), (), ()), ("Y", (q,), (), ()), ("Z", (q,), (), ()),
+                        ("U3", (q,), (), tuple(float(x) for x in rng.uniform(-3, 3, 3))),
+                        ("U2", (q,), (), tuple(float(x) for x in rng.uniform(-3, 3, 2))),
+                        ("PHASE", (q,), (), (0.0, 1.0)))[int(rng.integers(7))])
+    return ops
+
+
+@pytest.mark.parametrize("dtype", [brk.C128, brk.C64])
+@pytest.mark.parametrize("n,layers,long_range", [(12, 1, False), (12, 5, True), (13, 4, False), (16, 6, True),
+                                                 (18, 3, False)])
+def test_merged_sweeps_match_chain_sweep(n, layers, long_range, dtype, access):
+    """Circuits of one-qubit gates, Z and CZ (the merged sweeps) against the per-run passes (tuning
+    adjoint_blocks = 0), from a state that is not a basis state; the bars of the test below."""
+    rng = np.random.default_rng(60 + n + layers)
+    ops = one_qubit_ansatz(n, rng, layers, long_range)
+    J, h = rng.uniform(-1, 1, n - 1), rng.uniform(-1, 1, n)
+    psi0 = rng.normal(size=1 << n) + 1j * rng.normal(size=1 << n)
+    psi0 /= np.linalg.norm(psi0)
+    note(f"gpu adjoint merged vs chain n={n} layers={layers} long={long_range} dtype={dtype} ({access})")
+    e1, g1, back1 = adjoint(n, ops, J, h, dtype, psi0)
+    brk.tune("adjoint_blocks", 0)
+    try:
+        e0, g0, _ = adjoint(n, ops, J, h, dtype, psi0)
+    finally:
+        brk.tune("adjoint_blocks", 1)
+    tol = 1e-12 if dtype == brk.C128 else 2e-5
+    assert abs(e1 - e0) < tol
+    assert np.max(np.abs(g1 - g0)) < tol
+    assert np.max(np.abs(back1 - psi0)) < (1e-12 if dtype == brk.C128 else 1e-5)
+
+
 @pytest.mark.parametrize("n,dtype", [(14, brk.C128), (13, brk.C64)])
 def test_blocked_sweep_matches_chain_sweep(n, dtype, access):
     """The blocked reverse sweep (default) against the per-run passes (tuning adjoint_blocks = 0)."""
