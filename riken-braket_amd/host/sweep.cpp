@@ -18,27 +18,40 @@ namespace {
 struct planner {
   const std::vector<sweep_gate>& gates;
   unsigned n;
-  std::vector<std::vector<uint32_t>> succ;
+  struct edge {
+    uint32_t to;
+    int32_t next;
+  };
+  std::vector<edge> edges;    // what depends on a gate: lists through the edges
+  std::vector<int32_t> succ;  // first edge of each gate, -1: none
   std::vector<uint32_t> indeg;
   std::vector<uint32_t> ready;  // runnable gates, any order
   std::vector<uint32_t> stamp, left;
   uint32_t now = 0;
-  std::vector<uint32_t> stack;
+  std::vector<uint32_t> stack, base;
+  std::vector<std::vector<uint32_t>> waiting;  // per qubit
 
+  template <typename F>
+  void for_successors(uint32_t i, F f) const {
+    for (int32_t e = succ[i]; e >= 0; e = edges[(size_t)e].next) f(edges[(size_t)e].to);
+  }
   uint32_t qubits(const sweep_gate& g) const { return g.sign ? g.mask : 1u << g.q; }
 
   planner(const std::vector<sweep_gate>& g, unsigned num_qubits) : gates(g), n(num_qubits) {
     const uint32_t count = (uint32_t)gates.size();
-    succ.assign(count, {});
+    succ.assign(count, -1);
+    edges.reserve(4 * (size_t)count);
     indeg.assign(count, 0);
     stamp.assign(count, 0);
     left.assign(count, 0);
+    waiting.assign(32, {});
     std::vector<long> last_mix(n, -1);
     std::vector<std::vector<uint32_t>> since(n);  // diagonal gates on a qubit since its last mixing gate
     for (uint32_t i = 0; i < count; ++i) {
       const sweep_gate& gate = gates[i];
       auto after = [&](uint32_t j) {
-        succ[j].push_back(i);
+        edges.push_back({i, succ[j]});
+        succ[j] = (int32_t)edges.size() - 1;
         ++indeg[i];
       };
       if (gate.sign || gate.diagonal) {
@@ -70,45 +83,89 @@ struct planner {
       const uint32_t i = stack.back();
       stack.pop_back();
       got += gates[i].sign ? 0 : 1;
-      for (uint32_t j : succ[i]) {
+      for_successors(i, [&](uint32_t j) {
         if (stamp[j] != now) {
           stamp[j] = now;
           left[j] = indeg[j];
         }
         if (--left[j] == 0 && runs_in(j, set)) stack.push_back(j);
-      }
+      });
     }
     return got;
   }
 
-  // `set` with up to `room` of the candidates added, each the one that lets the most gates run.
+  // `set` with up to `room` of the candidates added, each the one that lets the most gates (at most
+  // `budget`) run.  What runs within the set is simulated once; a candidate then only follows what it
+  // adds, from the gates that wait for it.
   uint32_t grow(uint32_t set, uint32_t candidates, unsigned room, unsigned budget) {
-    unsigned have = closure(set, budget);
-    while (room) {
-      unsigned best = have;
-      uint32_t bit = 0;
+    base = indeg;
+    for (auto& w : waiting) w.clear();
+    stack = ready;
+    run(set);
+    while (room--) {
+      unsigned best = 0;
+      unsigned qubit = 0;
       for (uint32_t m = candidates & ~set; m; m &= m - 1) {
-        const uint32_t b = m & (0u - m);
-        const unsigned c = closure(set | b, budget);
+        const unsigned q = (unsigned)__builtin_ctz(m);
+        if (waiting[q].empty()) continue;
+        const unsigned c = gain(set | 1u << q, q, budget);
         if (c > best) {
           best = c;
-          bit = b;
+          qubit = q;
         }
       }
-      if (!bit) break;
-      set |= bit;
-      have = best;
-      --room;
+      if (!best) break;
+      set |= 1u << qubit;
+      stack.swap(waiting[qubit]);
+      waiting[qubit].clear();
+      run(set);
     }
     return set;
+  }
+
+  // Runs the gates on the stack and what they make ready within the set, on `base`; the others wait.
+  void run(uint32_t set) {
+    while (!stack.empty()) {
+      const uint32_t i = stack.back();
+      stack.pop_back();
+      if (!runs_in(i, set)) {
+        waiting[gates[i].q].push_back(i);
+        continue;
+      }
+      for_successors(i, [&](uint32_t j) {
+        if (--base[j] == 0) stack.push_back(j);
+      });
+    }
+  }
+  // How many one-qubit gates (at most `budget`) more run once qubit q is in the set.
+  unsigned gain(uint32_t set, unsigned q, unsigned budget) {
+    ++now;
+    stack = waiting[q];
+    unsigned got = 0;
+    while (!stack.empty() && got < budget) {
+      const uint32_t i = stack.back();
+      stack.pop_back();
+      if (!runs_in(i, set)) continue;
+      got += gates[i].sign ? 0 : 1;
+      for_successors(i, [&](uint32_t j) {
+        if (stamp[j] != now) {
+          stamp[j] = now;
+          left[j] = base[j];
+        }
+        if (--left[j] == 0) stack.push_back(j);
+      });
+    }
+    stack.clear();
+    return got;
   }
 
   void take(size_t k) {  // runs ready[k]
     const uint32_t i = ready[k];
     ready[k] = ready.back();
     ready.pop_back();
-    for (uint32_t j : succ[i])
+    for_successors(i, [&](uint32_t j) {
       if (--indeg[j] == 0) ready.push_back(j);
+    });
   }
 };
 
@@ -225,7 +282,6 @@ int plan_sweep(const std::vector<sweep_gate>& gates, unsigned n, unsigned num_lo
   planner p(gates, n);
   const uint32_t all = n >= 32 ? ~0u : (1u << n) - 1u;
   const uint32_t line = (1u << line_bits) - 1u;
-  constexpr unsigned BLOCK_BUDGET = 256;  // gates the greedy choice of local qubits looks ahead
   // A segment goes on to another macro where it runs this many gates: a macro takes the time of about
   // two exchanges through LDS whatever it runs (24 qubits, 12 layers: 151 reverse macros in 58
   // segments; 178 in 56 with macros of any size).
@@ -235,7 +291,7 @@ int plan_sweep(const std::vector<sweep_gate>& gates, unsigned n, unsigned num_lo
   std::vector<char> program;
   while (!p.ready.empty()) {
     // local qubits: the line's, the greedy ones, then the lowest others
-    uint32_t local = p.grow(line, all, num_local - line_bits, BLOCK_BUDGET);
+    uint32_t local = p.grow(line, all, num_local - line_bits, ~0u);
     for (unsigned q = 0; (unsigned)__builtin_popcount(local) < num_local; ++q) local |= 1u << q;
     sweep_header h{};
     unsigned rank[32] = {}, r = 0;
