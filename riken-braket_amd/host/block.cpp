@@ -15,15 +15,17 @@
 //    a chunk; the local set is filled up with the lowest remaining qubits;
 //  * launches, which run: only the bits that a gate flips need to be local --
 //    control bits and the parity bits of diagonal gates (RZ, CZ, ...) outside
-//    the chunk are the same for all its amplitudes -- so a launch takes the
-//    gates of about two steps (the 32-qubit circuit of 208 ops: 12 launches
-//    for 27 steps; 20 qubits with 10 layers of RZ and CNOT: 12 for 41).
+//    the chunk are the same for all its amplitudes -- and moves may run out of
+//    order (launch_builder), so a launch takes the gates of two to four steps
+//    (20 qubits with 10 layers of RZ and CNOT: 9 for 41).
 // A group of one op runs on the plain kernels.
 #include <hip/hip_runtime_api.h>
 
 #include <algorithm>
 #include <cstring>
+#include <iterator>
 #include <new>
+#include <utility>
 #include <vector>
 
 #include "brk_block.hpp"
@@ -429,51 +431,101 @@ static int physical_op(const brk_circuit::op& o, permutation& perm, brk_circuit:
                               m->params.data(), d);
 }
 
-// Collects consecutive ops into launches and hands each over as soon as it is complete.
+// Collects ops into launches and hands each over as soon as it is complete.  A launch takes the ops
+// in order, and passes over one that does not fit for later ones where that changes no bit of the
+// result: a move (X, CNOT, SWAP) only renames the indices that a gate acts on, so it may pass, or be
+// passed by, any gate that mixes none of the qubits they share (two qubits' H, say, may not change
+// places: their roundings differ).  Launches for 200 gates, in order and so: 29 qubits 11-13 and 9-11,
+// 20 qubits 9 and 7, 18 qubits 7-8 and 5-7; 20 qubits with 10 layers of RZ and CNOT 12 and 9.
 // plain(op) / block(args) return a status.
 template <typename Plain, typename Block>
 struct launch_builder {
+  // Ops passed over at most; a launch of the above circuits takes 20 to 40.
+  static constexpr size_t LOOKAHEAD = 2 * BLOCK_MAX_OPS;
+  struct entry {
+    brk_circuit::op op;
+    gate_desc desc;
+  };
   chunk_shape shape;
   unsigned line_bits;
   Plain plain;
   Block block;
+  // the launch in the making
+  gate_desc descs[BLOCK_MAX_OPS];
+  unsigned count = 0;
   uint64_t mixing = 0;
   size_t room = 0;
-  std::vector<gate_desc> descs;
-  brk_circuit::op single;  // the first op of the group
+  brk_circuit::op first;
+  // the ops passed over: what they flip, and all that they touch; whether one of them rounds
+  std::vector<entry> rest;
+  uint64_t rest_mixing = 0, rest_qubits = 0;
+  bool rest_rounds = false;
+  std::vector<entry> pending;  // (empty but within add and flush)
   block_program prog;
   block_args args{};
 
   launch_builder(unsigned n, int dtype, Plain p, Block b)
       : shape(n, dtype), line_bits(block_run_qubits(dtype)), plain(p), block(b) {}
-  int add(const brk_circuit::op& m, const gate_desc& d) {
-    if (!shape.enabled() || !shape.fits(mixing_bits(d))) {
+  int add(brk_circuit::op&& m, const gate_desc& d) {
+    if (!shape.enabled() || !shape.fits(mixing_bits(d))) {  // too wide for a chunk
       if (int st = flush()) return st;
       return plain(m);
     }
-    if (descs.size() == (size_t)BLOCK_MAX_OPS || room + block_op_room(d) > BLOCK_ARG_ROOM ||
-        !shape.fits(mixing | mixing_bits(d)))
-      if (int st = flush()) return st;
-    if (descs.empty()) single = m;
-    mixing |= mixing_bits(d);
-    room += block_op_room(d);
-    descs.push_back(d);
-    return BRK_OK;
+    return place(std::move(m), d) ? emit() : BRK_OK;
   }
   int flush() {
-    int st = BRK_OK;
-    if (descs.size() == 1) {
-      st = plain(single);
-    } else if (!descs.empty()) {
-      make_block_program(descs.data(), (unsigned)descs.size(), shape.n, mixing, shape.num_local(), line_bits, &prog);
-      make_passes(prog, line_bits);
-      pack(prog, &args);
-      st = block(args);
+    while (count)
+      if (int st = emit()) return st;
+    return BRK_OK;
+  }
+
+ private:
+  // Whether the launch is complete with this op.
+  bool place(brk_circuit::op&& op, const gate_desc& d) {
+    const uint64_t m = mixing_bits(d);
+    const bool rounds = d.mode != BLOCK_SWAP;
+    const bool in_order = !(rest_mixing & d.qubits) && !(m & rest_qubits) && !(rounds && rest_rounds);
+    if (in_order && shape.fits(mixing | m) && room + block_op_room(d) <= BLOCK_ARG_ROOM) {
+      if (!count) first = std::move(op);
+      mixing |= m;
+      room += block_op_room(d);
+      descs[count++] = d;
+      return count == (unsigned)BLOCK_MAX_OPS;
     }
-    mixing = 0;
-    room = 0;
-    descs.clear();
-    return st;
+    rest_mixing |= m;
+    rest_qubits |= d.qubits;
+    rest_rounds |= rounds;
+    rest.push_back({std::move(op), d});
+    // (nothing passes a gate that rounds once every qubit is touched)
+    return rest.size() == LOOKAHEAD || (rest_rounds && rest_qubits == (1ull << shape.n) - 1ull);
+  }
+  int launch() {
+    if (count == 1) return plain(first);
+    make_block_program(descs, count, shape.n, mixing, shape.num_local(), line_bits, &prog);
+    make_passes(prog, line_bits);
+    pack(prog, &args);
+    return block(args);
+  }
+  // Runs the launch, and puts the ops passed over in the next ones; the last of these stays open.
+  int emit() {
+    size_t next = 0;
+    bool complete = true;
+    while (complete) {
+      if (int st = launch()) return st;
+      rest.insert(rest.end(), std::make_move_iterator(pending.begin() + next),
+                  std::make_move_iterator(pending.end()));
+      pending.swap(rest);
+      rest.clear();
+      count = 0;
+      mixing = rest_mixing = rest_qubits = 0;
+      room = 0;
+      rest_rounds = false;
+      complete = false;
+      for (next = 0; next < pending.size() && !complete; ++next)
+        complete = place(std::move(pending[next].op), pending[next].desc);
+    }
+    pending.clear();
+    return BRK_OK;
   }
 };
 
@@ -520,7 +572,7 @@ static int build_plan(const brk_circuit* circuit, int dtype, const unsigned* per
     if (!s.num_ops) s.first_op = i;
     ++s.num_ops;
     qubits |= d.qubits;
-    if (int st = b.add(m, d)) return st;
+    if (int st = b.add(std::move(m), d)) return st;
   }
   close_step();
   if (int st = b.flush()) return st;
@@ -546,7 +598,7 @@ int run_in_blocks(const brk_circuit* circuit, void* first, int dtype, permutatio
     gate_desc d;
     brk_circuit::op m;
     if (int st = physical_op(o, perm, &m, &d)) return st;
-    if (int st = b.add(m, d)) return st;
+    if (int st = b.add(std::move(m), d)) return st;
   }
   return b.flush();
 }

@@ -103,6 +103,34 @@ def test_run_equals_gate_by_gate_bitwise(n, dtype, seed, access):
         assert same_bits(want, x)
 
 
+@pytest.mark.parametrize("n,dtype,moves", [(14, brk.C128, 0.5), (15, brk.C64, 0.8), (18, brk.C128, 0.8),
+                                           (20, brk.C64, 0.97), (22, brk.C128, 0.97)])
+def test_moves_out_of_order_bitwise(n, dtype, moves):
+    """Moves that pass, or are passed by, gates that a launch leaves for later (and long runs of moves that
+    no launch takes together): the bits of the op-by-op run, and the same final permutation."""
+    note(f"gpu moves out of order n={n} dtype={dtype} moves={moves}")
+    rng = np.random.default_rng(n)
+    ops = []
+    for _ in range(500):
+        q = [int(x) for x in rng.permutation(n)[:4]]
+        if rng.random() < moves:
+            ops.append([("X", (q[0],), (), ()), ("X", (q[0],), (q[1],), ()), ("X", (q[0],), (q[1], q[2]), ()),
+                        ("SWAP", (q[0], q[1]), (), ()), ("LOCAL_SWAP", (q[0], q[1]), (), ())][rng.integers(5)])
+        else:
+            ops.append([("H", (q[0],), (), ()), ("RX", (q[0],), (q[1],), (0.3,)), ("RZ", (q[0],), (), (0.7,)),
+                        ("Z", (q[0],), (q[1],), ())][rng.integers(4)])
+    s = D.random_state(n, rng)
+    s[rng.random(s.size) < 0.3] = 0.0
+    c = brk.Circuit(n, ops)
+    a, b = DeviceState.from_host(s, dtype), DeviceState.from_host(s, dtype)
+    final, _ = c.run_timed(a.ptr, dtype)
+    assert c.run(b.ptr, dtype) == final
+    want, got = a.download(), b.download()
+    a.free()
+    b.free()
+    assert same_bits(want, got)
+
+
 def test_dense_low_qubit_blocks(oracle):
     """Many gates on the line qubits and their neighbours: long blocks, every pair mode."""
     n = 18
