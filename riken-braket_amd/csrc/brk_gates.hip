@@ -628,8 +628,8 @@ __global__ __launch_bounds__(BLOCK_THREADS, BLOCK_WAVES_PER_SIMD) void k_block(c
   constexpr int L = BLOCK_THREAD_BITS + GB;
   __shared__ cpx<R> lds[PER * BLOCK_THREADS];
   const block_view v((cbytes)__builtin_amdgcn_kernarg_segment_ptr() + sizeof(s));
-  // XCD-contiguous chunk order: consecutive chunks (neighbouring runs of memory) on one XCD
-  const uint64_t chunk = chunk_base(xcd_tile(blockIdx.x, gridDim.x, 1), v, L);
+  // consecutive chunks (neighbouring runs of memory) on one XCD
+  const uint64_t chunk = chunk_base(xcd_chunk(blockIdx.x, gridDim.x), v, L);
   const uint32_t t = threadIdx.x;
   const uint32_t npasses = v.h->num_passes;
   if (!(v.passes[0].flags & BLOCK_PASS_LOADS)) {

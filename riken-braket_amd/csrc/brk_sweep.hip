@@ -213,7 +213,7 @@ void k_sweep(cpx<R>* __restrict__ psi, cpx<R>* __restrict__ lam, const void* pro
   const csegment segments = (csegment)(prog + sizeof(sweep_header));
   const cmacro macros = (cmacro)(prog + h->macros_at);
   const uint32_t t = threadIdx.x;
-  const uint32_t chunk_number = (uint32_t)xcd_tile(blockIdx.x, gridDim.x, 1);  // XCD-contiguous chunk order
+  const uint32_t chunk_number = (uint32_t)xcd_chunk(blockIdx.x, gridDim.x);
   uint32_t chunk = chunk_number;  // (amplitude indices are 32-bit: SWEEP_MAX_QUBITS)
 #pragma unroll
   for (int r = 0; r < L; ++r) {
