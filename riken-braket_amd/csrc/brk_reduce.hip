@@ -2,10 +2,11 @@
 // values, Pauli-string expectation values and the open-chain Ising energy,
 // plus H|psi> for that Hamiltonian.
 //
-// Every reduction runs on a fixed grid of RED_BLOCKS blocks with a
-// grid-stride loop, so the assignment of amplitudes to threads, the in-block
-// tree and the host-side sum over the block partials (in block order) are the
-// same on every call: results are bit-reproducible.  Partial sums are kept in
+// Every reduction runs on a fixed grid of RED_BLOCKS blocks, so the assignment
+// of amplitudes to threads, the in-block tree and the host-side sum over the
+// block partials (in block order) are the same on every call: results are
+// bit-reproducible.  The blocks write their partials straight to pinned host
+// memory (24 KB at most): a copy back costs about 10 us more per call.  Partial sums are kept in
 // double whatever the element type (the reference accumulates per-thread
 // partials and then std::accumulate's them, inner_product.hpp:43-55; spin
 // values use long double, spin_expectation_value.hpp:31-64).
@@ -19,9 +20,36 @@
 
 namespace brk {
 
-// Grid-stride loops load RED_UNROLL strides ahead before adding them in stride order (the
-// same sums, more loads in flight per thread).
+// The items 0 .. n - 1 of a reduction, n a power of two: block b takes the tiles b, b + RED_BLOCKS, ...
+// of RED_UNROLL * RED_THREADS consecutive items, a tile's loads all in flight before its first add.
+// Bound: HBM reads.  A 4 GiB state's spin value (two amplitudes an item): 0.67-0.73 ms, 5.9-6.4 TB/s
+// by qubit; with the unrolled items a whole grid apart, the tiles' rows in RED_UNROLL places at a
+// time, 0.75-0.88 ms; one item a time that way 0.69-0.74.  (65536 blocks of one tile each: 0.66-0.68,
+// but 1.5 MB of partials.)
 constexpr int RED_UNROLL = 4;
+
+template <typename Load, typename Add>
+__device__ __forceinline__ void for_tiles(uint64_t n, Load load, Add add) {
+  constexpr uint64_t TILE = (uint64_t)RED_UNROLL * RED_THREADS;
+  for (uint64_t t = (uint64_t)blockIdx.x * TILE; t < n; t += (uint64_t)RED_BLOCKS * TILE) {
+    if (t + TILE <= n) {
+      decltype(load(t)) x[RED_UNROLL];
+#pragma unroll
+      for (int u = 0; u < RED_UNROLL; ++u) x[u] = load(t + (uint64_t)(u * RED_THREADS) + threadIdx.x);
+#pragma unroll
+      for (int u = 0; u < RED_UNROLL; ++u) add(x[u]);
+    } else {
+      for (uint64_t i = t + threadIdx.x; i < n; i += RED_THREADS) add(load(i));
+    }
+  }
+}
+
+// Two amplitudes of an item.
+template <typename R1, typename R2>
+struct amp_pair {
+  cpx<R1> x;
+  cpx<R2> y;
+};
 
 template <int NV>
 struct dvec {
@@ -57,46 +85,26 @@ template <typename R1, typename R2>
 __global__ __launch_bounds__(RED_THREADS) void k_inner(const cpx<R1>* __restrict__ a, const cpx<R2>* __restrict__ b,
                                                       uint64_t size, double* partial) {
   dvec<2> acc{{0.0, 0.0}};
-  const uint64_t stride = (uint64_t)RED_BLOCKS * RED_THREADS;
-  auto add = [&](cpx<R1> x, cpx<R2> y) {
-    const double xr = x.re, xi = x.im, yr = y.re, yi = y.im;
-    // conj(y) * x
-    acc.v[0] += yr * xr + yi * xi;
-    acc.v[1] += yr * xi - yi * xr;
-  };
-  uint64_t i = (uint64_t)blockIdx.x * RED_THREADS + threadIdx.x;
-  for (; i + (RED_UNROLL - 1) * stride < size; i += RED_UNROLL * stride) {
-    cpx<R1> x[RED_UNROLL];
-    cpx<R2> y[RED_UNROLL];
-#pragma unroll
-    for (int u = 0; u < RED_UNROLL; ++u) {
-      x[u] = a[i + u * stride];
-      y[u] = b[i + u * stride];
-    }
-#pragma unroll
-    for (int u = 0; u < RED_UNROLL; ++u) add(x[u], y[u]);
-  }
-  for (; i < size; i += stride) add(a[i], b[i]);
+  for_tiles(
+      size, [&](uint64_t i) { return amp_pair<R1, R2>{a[i], b[i]}; },
+      [&](const amp_pair<R1, R2>& p) {
+        const double xr = p.x.re, xi = p.x.im, yr = p.y.re, yi = p.y.im;
+        // conj(y) * x
+        acc.v[0] += yr * xr + yi * xi;
+        acc.v[1] += yr * xi - yi * xr;
+      });
   block_store<2>(acc, partial);
 }
 
 template <typename R>
 __global__ __launch_bounds__(RED_THREADS) void k_norm(const cpx<R>* __restrict__ a, uint64_t size, double* partial) {
   dvec<1> acc{{0.0}};
-  const uint64_t stride = (uint64_t)RED_BLOCKS * RED_THREADS;
-  auto add = [&](cpx<R> x) {
-    const double xr = x.re, xi = x.im;
-    acc.v[0] += xr * xr + xi * xi;
-  };
-  uint64_t i = (uint64_t)blockIdx.x * RED_THREADS + threadIdx.x;
-  for (; i + (RED_UNROLL - 1) * stride < size; i += RED_UNROLL * stride) {
-    cpx<R> x[RED_UNROLL];
-#pragma unroll
-    for (int u = 0; u < RED_UNROLL; ++u) x[u] = a[i + u * stride];
-#pragma unroll
-    for (int u = 0; u < RED_UNROLL; ++u) add(x[u]);
-  }
-  for (; i < size; i += stride) add(a[i]);
+  for_tiles(
+      size, [&](uint64_t i) { return a[i]; },
+      [&](const cpx<R>& x) {
+        const double xr = x.re, xi = x.im;
+        acc.v[0] += xr * xr + xi * xi;
+      });
   block_store<1>(acc, partial);
 }
 
@@ -105,16 +113,18 @@ template <typename R>
 __global__ __launch_bounds__(RED_THREADS) void k_spin(const cpx<R>* __restrict__ a, uint64_t npairs, uint64_t lower,
                                                      uint64_t qmask, double* partial) {
   dvec<3> acc{{0.0, 0.0, 0.0}};
-  const uint64_t stride = (uint64_t)RED_BLOCKS * RED_THREADS;
-  for (uint64_t g = (uint64_t)blockIdx.x * RED_THREADS + threadIdx.x; g < npairs; g += stride) {
-    const uint64_t i0 = ((g & ~lower) << 1) | (g & lower);
-    cpx<R> x0 = a[i0];
-    cpx<R> x1 = a[i0 | qmask];
-    const double r0 = x0.re, m0 = x0.im, r1 = x1.re, m1 = x1.im;
-    acc.v[0] += r0 * r1 + m0 * m1;
-    acc.v[1] += r0 * m1 - m0 * r1;
-    acc.v[2] += (r0 * r0 + m0 * m0) - (r1 * r1 + m1 * m1);
-  }
+  for_tiles(
+      npairs,
+      [&](uint64_t g) {
+        const uint64_t i0 = ((g & ~lower) << 1) | (g & lower);
+        return amp_pair<R, R>{a[i0], a[i0 | qmask]};
+      },
+      [&](const amp_pair<R, R>& p) {
+        const double r0 = p.x.re, m0 = p.x.im, r1 = p.y.re, m1 = p.y.im;
+        acc.v[0] += r0 * r1 + m0 * m1;
+        acc.v[1] += r0 * m1 - m0 * r1;
+        acc.v[2] += (r0 * r0 + m0 * m0) - (r1 * r1 + m1 * m1);
+      });
   block_store<3>(acc, partial);
 }
 
@@ -122,21 +132,24 @@ __global__ __launch_bounds__(RED_THREADS) void k_spin(const cpx<R>* __restrict__
 template <typename R>
 __global__ __launch_bounds__(RED_THREADS) void k_pauli(const cpx<R>* __restrict__ a, uint64_t size, uint64_t flip,
                                                       uint64_t sign, double* partial) {
+  struct item {
+    cpx<R> x, y;
+    bool odd;
+  };
   dvec<2> acc{{0.0, 0.0}};
-  const uint64_t stride = (uint64_t)RED_BLOCKS * RED_THREADS;
-  for (uint64_t i = (uint64_t)blockIdx.x * RED_THREADS + threadIdx.x; i < size; i += stride) {
-    cpx<R> x = a[i];
-    cpx<R> y = a[i ^ flip];
-    const double xr = x.re, xi = x.im, yr = y.re, yi = y.im;
-    double re = xr * yr + xi * yi;
-    double im = xr * yi - xi * yr;
-    if (__popcll(i & sign) & 1) {
-      re = -re;
-      im = -im;
-    }
-    acc.v[0] += re;
-    acc.v[1] += im;
-  }
+  for_tiles(
+      size, [&](uint64_t i) { return item{a[i], a[i ^ flip], (__popcll(i & sign) & 1) != 0}; },
+      [&](const item& p) {
+        const double xr = p.x.re, xi = p.x.im, yr = p.y.re, yi = p.y.im;
+        double re = xr * yr + xi * yi;
+        double im = xr * yi - xi * yr;
+        if (p.odd) {
+          re = -re;
+          im = -im;
+        }
+        acc.v[0] += re;
+        acc.v[1] += im;
+      });
   block_store<2>(acc, partial);
 }
 
@@ -325,28 +338,16 @@ template <typename R>
 __global__ __launch_bounds__(RED_THREADS) void k_zero_one(const cpx<R>* __restrict__ a, uint64_t npairs, uint64_t lower,
                                                          uint64_t qmask, double* partial) {
   dvec<2> acc{{0.0, 0.0}};
-  const uint64_t stride = (uint64_t)RED_BLOCKS * RED_THREADS;
-  auto add = [&](cpx<R> x0, cpx<R> x1) {
-    acc.v[0] += (double)x0.re * x0.re + (double)x0.im * x0.im;
-    acc.v[1] += (double)x1.re * x1.re + (double)x1.im * x1.im;
-  };
-  auto first = [&](uint64_t g) { return ((g & ~lower) << 1) | (g & lower); };
-  uint64_t g = (uint64_t)blockIdx.x * RED_THREADS + threadIdx.x;
-  for (; g + (RED_UNROLL - 1) * stride < npairs; g += RED_UNROLL * stride) {
-    cpx<R> x0[RED_UNROLL], x1[RED_UNROLL];
-#pragma unroll
-    for (int u = 0; u < RED_UNROLL; ++u) {
-      const uint64_t i0 = first(g + u * stride);
-      x0[u] = a[i0];
-      x1[u] = a[i0 | qmask];
-    }
-#pragma unroll
-    for (int u = 0; u < RED_UNROLL; ++u) add(x0[u], x1[u]);
-  }
-  for (; g < npairs; g += stride) {
-    const uint64_t i0 = first(g);
-    add(a[i0], a[i0 | qmask]);
-  }
+  for_tiles(
+      npairs,
+      [&](uint64_t g) {
+        const uint64_t i0 = ((g & ~lower) << 1) | (g & lower);
+        return amp_pair<R, R>{a[i0], a[i0 | qmask]};
+      },
+      [&](const amp_pair<R, R>& p) {
+        acc.v[0] += (double)p.x.re * p.x.re + (double)p.x.im * p.x.im;
+        acc.v[1] += (double)p.y.re * p.y.re + (double)p.y.im * p.y.im;
+      });
   block_store<2>(acc, partial);
 }
 
@@ -597,19 +598,16 @@ template <int NV, typename Launch>
 static int run_reduction(void* stream, Launch launch, double* out) {
   reduce_scratch* sc;
   if (int st = get_reduce_scratch(&sc)) return st;
-  // the device's scratch is ours from the launch until the partials are read back
+  // the device's scratch is ours from the launch until the partials are read
   std::lock_guard<std::mutex> hold(sc->busy);
   hipStream_t s = as_stream(stream);
-  launch(sc->device, s);
+  launch(sc->partials, s);
   if (int st = check_launch("reduction")) return st;
-  const hipError_t copied =
-      hipMemcpyAsync(sc->host, sc->device, sizeof(double) * RED_BLOCKS * NV, hipMemcpyDeviceToHost, s);
   const hipError_t synced = hipStreamSynchronize(s);
-  if (copied != hipSuccess) return fail(BRK_ERR_HIP, "reduction read-back: %s", hipGetErrorString(copied));
   if (synced != hipSuccess) return fail(BRK_ERR_HIP, "reduction: %s", hipGetErrorString(synced));
   for (int v = 0; v < NV; ++v) out[v] = 0.0;
   for (int b = 0; b < RED_BLOCKS; ++b)
-    for (int v = 0; v < NV; ++v) out[v] += sc->host[b * NV + v];
+    for (int v = 0; v < NV; ++v) out[v] += sc->partials[b * NV + v];
   return BRK_OK;
 }
 
@@ -817,17 +815,14 @@ static int ising_energy(const void* first, uint64_t size, const ising_args& args
   int status = BRK_OK;
   for (size_t k = 0; !status && k < passes.size(); ++k) {
     hipLaunchKernelGGL(k_ising<R>, dim3(grid), dim3(ISING_THREADS), 0, s, (const cpx<R>*)first, size, nchunks,
-                       passes[k], sc->device + k * grid);
+                       passes[k], sc->partials + k * grid);
     status = check_launch("Ising energy");
   }
-  const hipError_t copied =
-      status ? hipSuccess : hipMemcpyAsync(sc->host, sc->device, sizeof(double) * values, hipMemcpyDeviceToHost, s);
   const hipError_t synced = hipStreamSynchronize(s);
   if (status) return status;
-  if (copied != hipSuccess) return fail(BRK_ERR_HIP, "Ising read-back: %s", hipGetErrorString(copied));
   if (synced != hipSuccess) return fail(BRK_ERR_HIP, "Ising energy: %s", hipGetErrorString(synced));
   double total = 0.0;
-  for (size_t k = 0; k < values; ++k) total += sc->host[k];
+  for (size_t k = 0; k < values; ++k) total += sc->partials[k];
   *result = total;
   return BRK_OK;
 }

@@ -133,15 +133,10 @@ int get_reduce_scratch(reduce_scratch** out) {
   if ((int)g_scratch.size() <= dev) g_scratch.resize(dev + 1);
   if (!g_scratch[dev]) g_scratch[dev] = std::make_unique<reduce_scratch>();
   reduce_scratch& s = *g_scratch[dev];
-  if (s.device == nullptr) {
-    size_t bytes = sizeof(double) * RED_BLOCKS * RED_MAX_VALUES;
-    if (hipMalloc(&s.device, bytes) != hipSuccess) {
-      s.device = nullptr;
-      return fail(BRK_ERR_OUT_OF_MEMORY, "cannot allocate %zu bytes of reduction scratch", bytes);
-    }
-    if (hipHostMalloc(&s.host, bytes, hipHostMallocDefault) != hipSuccess) {
-      (void)hipFree(s.device);
-      s.device = nullptr;
+  if (s.partials == nullptr) {
+    const size_t bytes = sizeof(double) * RED_BLOCKS * RED_MAX_VALUES;
+    if (hipHostMalloc(&s.partials, bytes, hipHostMallocDefault) != hipSuccess) {
+      s.partials = nullptr;
       return fail(BRK_ERR_OUT_OF_MEMORY, "cannot allocate pinned reduction scratch");
     }
   }

@@ -126,3 +126,29 @@ def test_fill_hash_matches_numpy_twin():
     got = st.download()
     st.free()
     assert np.array_equal(got, D.hash_state_values(99, np.arange(4096), 0.5))
+
+
+@pytest.mark.parametrize("n,dtype", [(1, brk.C128), (9, brk.C64), (10, brk.C128), (11, brk.C128), (12, brk.C64),
+                                     (20, brk.C128), (21, brk.C128)])
+def test_reduction_tiles(oracle, n, dtype):
+    """Tiles of 1024 items on 1024 blocks: a part of one tile, one tile, some of the blocks, a tile each
+    (2^20 items) and two; against FP64 numpy sums.  At most 2^21 products of at most 1 / 2^n each."""
+    note(f"gpu reduction tiles n={n} dtype={dtype}")
+    rng = np.random.default_rng(n)
+    s, r = D.random_state(n, rng), D.random_state(n, rng)
+    if dtype == brk.C64:
+        s, r = (x.astype(np.complex64).astype(np.complex128) for x in (s, r))
+    a, b = DeviceState.from_host(s, dtype), DeviceState.from_host(r, dtype)
+    assert abs(brk.norm2(a.ptr, a.size, dtype) - np.vdot(s, s).real) < 1e-12
+    assert abs(brk.inner_product(a.ptr, dtype, b.ptr, dtype, a.size) - oracle.inner_product(s, r)) < 1e-12
+    for q in sorted({0, n // 2, n - 1}):
+        p = s.reshape(-1, 2, 1 << q)
+        up, down = p[:, 0], p[:, 1]
+        zero, one = np.sum(np.abs(up) ** 2), np.sum(np.abs(down) ** 2)
+        x = np.sum(np.conj(up) * down)
+        spin = brk.spin_expectation_value(a.ptr, a.size, dtype, q)
+        assert np.max(np.abs(np.array(spin) - [x.real, x.imag, 0.5 * (zero - one)])) < 1e-12
+        assert np.max(np.abs(np.array(brk.zero_one_probabilities(a.ptr, a.size, dtype, q)) - [zero, one])) < 1e-12
+        assert abs(brk.expectation_pauli_string(a.ptr, a.size, dtype, "X", [q]) - 2 * x.real) < 1e-12
+    a.free()
+    b.free()
