@@ -128,6 +128,26 @@ def test_generate_events_sparse_states(oracle):
     st.free()
 
 
+@pytest.mark.parametrize("n,dtype", [(2, brk.C64), (6, brk.C128), (7, brk.C128), (9, brk.C64), (11, brk.C128),
+                                     (11, brk.C64), (12, brk.C128), (15, brk.C64)])
+def test_generate_events_norms_by_wave(oracle, n, dtype):
+    """A wave's norms through LDS: parts of one wave, one wave, several, and 1, 2, 4 and 8 norms a lane; a
+    third of the amplitudes zero, targets at 0 and just below 1."""
+    note(f"gpu events by wave n={n} dtype={dtype}")
+    rng = np.random.default_rng(300 + n)
+    s = D.random_state(n, rng)
+    s[rng.random(s.size) < 0.33] = 0.0
+    s /= np.linalg.norm(s)
+    if dtype == brk.C64:
+        s = s.astype(np.complex64).astype(np.complex128)
+    c = canonical_draws(oracle, n, 2000) + [0.0, float(np.nextafter(1.0, 0.0))]
+    st = DeviceState.from_host(s, dtype)
+    gpu = brk.generate_events(st.ptr, st.size, dtype, c)
+    check_events(s, c, gpu, oracle.generate_events(s, c))
+    assert all(s[e] != 0.0 for e in gpu)
+    st.free()
+
+
 def test_generate_events_large(oracle):
     n = 26
     note(f"gpu events n={n} (1 GiB state, 20000 events)")
