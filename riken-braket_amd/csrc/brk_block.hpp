@@ -78,7 +78,7 @@ static_assert(sizeof(block_op) == 40, "read as five 64-bit words");
 // are group bits.  Gates that only move amplitudes (X, CNOT, SWAP, local swaps) on any
 // local bits come after them (num_moves ops): the segment writes its amplitudes to the
 // indices they move to.  A single pass applies one gate to the chunk in LDS with a
-// strided loop.
+// strided loop.  The program's ops lie in the order of its passes.
 enum block_pass_kind { BLOCK_PASS_SEGMENT = 0, BLOCK_PASS_SINGLE = 1 };
 enum block_pass_flags {
   BLOCK_PASS_LOADS = 1,  // the first pass: its groups come straight from the state
@@ -89,7 +89,7 @@ struct block_pass {
   uint8_t kind, num_ops, num_moves, flags;
   uint8_t group[4];   // ascending local bits of the group (L - 9 of them)
   uint8_t qubits[4];  // ... and the physical qubits they are
-  uint16_t first_op, pad;
+  uint32_t pad;
 };
 
 struct block_header {

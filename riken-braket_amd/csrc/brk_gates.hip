@@ -314,12 +314,6 @@ __device__ __forceinline__ block_gate decode(const op_words& r, const double (&u
   for (int k = 0; k < 8; ++k) g.u[k] = u[k];
   return g;
 }
-__device__ __forceinline__ block_gate load_gate(const block_view& v, uint32_t o) {
-  const op_words r = load_op(v, o);
-  double u[8];
-  load_coefs(v, r.coef(), u);
-  return decode(r, u);
-}
 // Whether the chunk with outer bits `base` satisfies the gate's conditions outside it.
 __device__ __forceinline__ bool acts_on(const block_gate& g, uint64_t base) {
   return (base & g.outer_cond) == g.outer_cond;
@@ -534,8 +528,8 @@ __device__ __forceinline__ void segment_rename_any(cpx<R> (&x)[PER], uint32_t fl
   }
 }
 
-// A diagonal gate without conditions in the chunk whose parity bits in the chunk are the group bits
-// ZG (over the group index): each member's coefficient is fixed at compile time.
+// A diagonal gate without conditions in the chunk whose parity bits in the group are ZG (over the
+// group index): which coefficient each member takes is fixed at compile time.
 template <int ZG, typename R, int PER>
 __device__ __forceinline__ void group_diag(cpx<R> (&x)[PER], cpx<R> c0, cpx<R> c1) {
   if constexpr (ZG < PER) {
@@ -561,18 +555,24 @@ __device__ __forceinline__ void segment_gate(cpx<R> (&x)[PER], uint32_t base, co
   if (op.kind == BLOCK_KIND_DIAG) {
     cpx<R> c0, c1;
     chunk_diag(op, chunk, c0, c1);
-    if ((op.group_cond | op.thread_cond | op.thread_zmask) == 0) {  // the common case
+    // parity bits in the thread's part only choose the thread's two coefficients (selecting them per
+    // member took 0.9 us a gate where this takes 0.56)
+    cpx<R> k0 = c0, k1 = c1;
+    if (op.thread_zmask != 0) {
+      const bool swapped = (__popc(base & op.thread_zmask) & 1) != 0;
+      k0 = csel(swapped, c1, c0);
+      k1 = csel(swapped, c0, c1);
+    }
+    if ((op.group_cond | op.thread_cond) == 0) {  // the common case
       switch (op.group_zmask) {
-        case 0: group_diag<0>(x, c0, c1); return;
-        case 1: group_diag<1>(x, c0, c1); return;
-        case 2: group_diag<2>(x, c0, c1); return;
-        case 4: group_diag<4>(x, c0, c1); return;
-        case 8: group_diag<8>(x, c0, c1); return;
+        case 0: group_diag<0>(x, k0, k1); return;
+        case 1: group_diag<1>(x, k0, k1); return;
+        case 2: group_diag<2>(x, k0, k1); return;
+        case 4: group_diag<4>(x, k0, k1); return;
+        case 8: group_diag<8>(x, k0, k1); return;
         default: break;
       }
     }
-    const bool swapped = (__popc(base & op.thread_zmask) & 1) != 0;
-    const cpx<R> k0 = csel(swapped, c1, c0), k1 = csel(swapped, c0, c1);
 #pragma unroll
     for (int m = 0; m < PER; ++m) {
       if ((m & op.group_cond) != op.group_cond) continue;  // uniform
@@ -617,13 +617,14 @@ __device__ __forceinline__ uint32_t move_linear(uint32_t j, const block_gate& op
 // the chunk in LDS.  The first and the last segment load from and store to the state
 // where their lanes cover whole lines, so a block of two segments exchanges its
 // amplitudes through LDS once.  The program is the launch's second argument, read where
-// the kernel arguments lie.  In a segment the descriptions of the next two gates are on
-// their way while a gate runs: they are scalar loads of about 0.1 us each, which a chunk
-// that has its CU to itself would otherwise wait for.
+// the kernel arguments lie.  The description of the next gate or move, across segments too, is on its
+// way while one runs: it is a scalar load of about 0.1 us, which a chunk that has its CU to itself
+// would otherwise wait for (20 qubits, where a move took 0.2 us: with the diagonal gates' paths in
+// segment_gate 338 -> 296 us, 12 qubits 175 -> 138).
 // Bound: the HBM round trip of the chunks (about 2.9 ms of a 29-qubit c128 state's 17.2 GB) plus what
-// the two workgroups of a CU do not hide of it in instructions: 4.0 ms a launch of 16 gates (4.3 TB/s)
-// on that state (4.4 ms with 64-bit indices and every move applied to every amplitude's index; 3.8 ms a
-// launch of 8 gates with every qubit local and an LDS round trip per pass).  Waves of
+// the two workgroups of a CU do not hide of it in instructions: 4.7 ms a launch of 21 gates on that
+// state, 0.22 a gate (0.28 with 64-bit indices and every move applied to every amplitude's index; 0.48
+// with every qubit local and an LDS round trip per pass).  Waves of
 // 16 amplitudes per lane (256 threads) run large states 1-2 % faster and small ones 15 % slower;
 // 1024 threads, which do not fit twice on a CU, half as fast.
 template <typename R, bool NT, int PER, typename I>
@@ -643,19 +644,25 @@ __global__ __launch_bounds__(BLOCK_THREADS, BLOCK_WAVES_PER_SIMD) void k_block(c
       lds[block_slot(t + BLOCK_THREADS * k)] = load_amp<NT>(s + (low | high_offset<I>(k, v)));
     __syncthreads();
   }
+  // the ops lie in the order of the passes: `cur` is always on its way
+  const uint32_t last = v.h->num_ops - 1;
+  uint32_t o = 0;
+  op_words cur = load_op(v, 0);
   for (uint32_t pi = 0; pi < npasses; ++pi) {
     const cpass pass = v.passes + pi;
-    const uint32_t first = pass->first_op;
     if (pass->kind == BLOCK_PASS_SINGLE) {
-      const block_gate op = load_gate(v, first);
+      const op_words next = load_op(v, min(++o, last));
+      double u[8];
+      load_coefs(v, cur.coef(), u);
+      const block_gate op = decode(cur, u);
+      cur = next;
       if (!acts_on(op, chunk)) continue;
       single_pass<R, PER>(lds, op, chunk, t);
       __syncthreads();
       continue;
     }
     const uint32_t num_ops = pass->num_ops, num_moves = pass->num_moves, flags = pass->flags;
-    const uint32_t last = first + (num_ops ? num_ops - 1 : 0);
-    op_words cur = load_op(v, first);
+    const uint32_t gates_end = o + num_ops, moves_end = gates_end + num_moves;
     uint32_t base = t, bit[GB + 1];
 #pragma unroll
     for (int i = 0; i < GB; ++i) {
@@ -684,8 +691,8 @@ __global__ __launch_bounds__(BLOCK_THREADS, BLOCK_WAVES_PER_SIMD) void k_block(c
 #pragma unroll
       for (int m = 0; m < PER; ++m) x[m] = lds[slot[m]];
     }
-    for (uint32_t o = 0; o < num_ops; ++o) {
-      const op_words next = load_op(v, min(first + o + 1, last));
+    while (o < gates_end) {
+      const op_words next = load_op(v, min(++o, last));
       double u[8];
       load_coefs(v, cur.coef(), u);
       const block_gate op = decode(cur, u);
@@ -697,9 +704,11 @@ __global__ __launch_bounds__(BLOCK_THREADS, BLOCK_WAVES_PER_SIMD) void k_block(c
     const bool linear = (flags & BLOCK_PASS_LINEAR) != 0;
     uint32_t j[PER];
     if (linear) {
-      for (uint32_t o = first + num_ops; o < first + num_ops + num_moves; ++o) {
+      while (o < moves_end) {
+        const op_words next = load_op(v, min(++o, last));
         const double none[8] = {};
-        const block_gate op = decode(load_op(v, o), none);
+        const block_gate op = decode(cur, none);
+        cur = next;
         if (!acts_on(op, chunk)) continue;
         base = move_linear(base, op, true);
 #pragma unroll
@@ -712,9 +721,11 @@ __global__ __launch_bounds__(BLOCK_THREADS, BLOCK_WAVES_PER_SIMD) void k_block(c
 #pragma unroll
       for (int m = 0; m < (1 << i); ++m) j[m | 1 << i] = j[m] ^ bit[i];
     if (!linear) {
-      for (uint32_t o = first + num_ops; o < first + num_ops + num_moves; ++o) {
+      while (o < moves_end) {
+        const op_words next = load_op(v, min(++o, last));
         const double none[8] = {};
-        const block_gate op = decode(load_op(v, o), none);
+        const block_gate op = decode(cur, none);
+        cur = next;
         if (!acts_on(op, chunk)) continue;
         const uint32_t flip = op.flip;
         if ((flip & op.cond) == 0) {  // X

@@ -98,7 +98,6 @@ static void make_passes(block_program& prog, unsigned line_bits) {
     block_pass& p = prog.passes[prog.h.num_passes++];
     p = block_pass{};
     p.kind = (uint8_t)kind;
-    p.first_op = (uint16_t)placed;
     return p;
   };
   auto close = [&]() {
