@@ -14,7 +14,7 @@ amplitudes (64 GiB) resident in HBM.  A step is one pass of the circuit.
                qubit then 10 layers of RZ on each qubit and a CNOT brick (315
                gates) -- run by the CPU oracle (ket's algorithm, -Ofast -fopenmp
                like bra's nompi-release build, all host cores): gate loop only,
-               1 warm-up, median of 5; the GPU's per-gate and gate-block times
+               1 warm-up, median of 5; the GPU's gate-by-gate and gate-block times
                for the same circuit beside it.  cpu_baseline_30q: the oracle on
                the benchmark circuit's generator at 30 qubits (bounded sample)
   fused_c64  = the precision form on the same circuit: greedy fusion into dense
@@ -22,7 +22,7 @@ amplitudes (64 GiB) resident in HBM.  A step is one pass of the circuit.
                state, FP32 MFMA GEMMs; circuit time, speedup over the complex128
                per-gate path and infidelity 1 - |<psi_c128|psi_c64>|^2 (FP64)
   batch_c64  = the batching form: 4096 ansatz circuits of 10..20 qubits in one
-               graph-captured persistent launch; circuits/s, p50/p99 latency
+               captured graph, a launch per stage level; circuits/s, p50/p99 latency
   adjoint_c128 = the differentiation form: adjoint gradient of a 24-qubit,
                576-parameter ansatz; gradients/s, max error vs parameter shift over
                all 576 parameters and vs central differences on a sample
@@ -137,8 +137,9 @@ def _host_description():
 def cpu_baseline_20q(stream, runs=5):
     """The reference's CPU case on the host: 20 qubits, H wall + 10 RZ / CNOT-brick layers (315
     gates), the CPU oracle built like bra's nompi-release (-Ofast -fopenmp), all host cores.
-    Gate loop only, 1 warm-up, median of `runs`.  The same circuit on the GPU (per-gate and
-    gate blocks, median of `runs` after a warm-up) goes beside it."""
+    Gate loop only, 1 warm-up, median of `runs`.  The same circuit on the GPU (gate by
+    gate, the kernels' times between events, and in gate blocks, median of `runs` after a warm-up) goes
+    beside it."""
     import numpy as np
 
     import brk
@@ -171,17 +172,18 @@ def cpu_baseline_20q(stream, runs=5):
     st = DeviceState(n)
     gpu = {"per_gate": [], "blocks": []}
     for k in range(runs + 1):
-        for key, run in (("per_gate", lambda: circuit.run(st.ptr, stream=stream)),
-                         ("blocks", lambda: plan.run(st.ptr, stream))):
-            brk.set_basis_state(st.ptr, st.size, brk.C128, 0, stream)
-            hip.synchronize(stream)
-            e0, e1 = hip.Event(), hip.Event()
-            e0.record(stream)
-            run()
-            e1.record(stream)
-            e1.synchronize()
-            if k:
-                gpu[key].append(e0.elapsed_ms(e1))
+        brk.set_basis_state(st.ptr, st.size, brk.C128, 0, stream)
+        per_gate = sum(circuit.run_timed(st.ptr, stream=stream)[1])
+        brk.set_basis_state(st.ptr, st.size, brk.C128, 0, stream)
+        hip.synchronize(stream)
+        e0, e1 = hip.Event(), hip.Event()
+        e0.record(stream)
+        plan.run(st.ptr, stream)
+        e1.record(stream)
+        e1.synchronize()
+        if k:
+            gpu["per_gate"].append(per_gate)
+            gpu["blocks"].append(e0.elapsed_ms(e1))
     got = st.download()
     st.free()
     err = float(np.max(np.abs(got - s)))
@@ -457,7 +459,7 @@ def plain_energy(n, ops, J, h, stream):
 
 def batch_leg(args, stream):
     """Batching form: 4096 hardware-efficient-ansatz circuits of 10..20 qubits (8 layers),
-    complex64 states, one graph-captured persistent launch per batch; FP64 energies."""
+    complex64 states, one captured graph per batch; FP64 energies."""
     import numpy as np
 
     import brk

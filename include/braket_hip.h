@@ -455,8 +455,9 @@ int brk_block_plan_step(const brk_block_plan* plan, unsigned i, unsigned* first_
                         unsigned* num_local, unsigned* local_qubits);
 int brk_block_plan_final_permutation(const brk_block_plan* plan, unsigned* permutation);
 /* Runs the plan on a state of 2^num_qubits amplitudes of the plan's dtype.
-   Consecutive steps share a launch where the bits their gates flip fit in one
-   chunk (control bits and diagonal gates may lie outside it).  The block
+   Steps share a launch where the bits their gates flip fit in one chunk
+   (control bits and diagonal gates may lie outside it, and X, CNOT and SWAP run
+   before or after gates they commute with bit for bit).  The block
    programs travel in the launches' arguments: nothing is uploaded or kept on
    the device. */
 int brk_block_plan_run(brk_block_plan* plan, void* first, void* stream);

@@ -1,4 +1,4 @@
-// Batching form: one persistent launch runs a list of small circuits and
+// Batching form: a launch per stage level runs a list of small circuits and
 // writes the FP64 Ising energy of each (ancestor in the reference: bra's
 // CIRCUITS mode, which advances several states one after another,
 // bra/src/bra.cpp:315-336, bra/src/interpreter.cpp:411-419).
@@ -226,8 +226,8 @@ __device__ void gate_pass(const chunk_ctx& c, cu32 w, uint32_t tid) {
 }
 
 // The X terms of NP local positions p[]: each thread holds the 2^NP amplitudes of a group, as a gate
-// pass does, so the chunk is read once for up to four terms (one read a term: 16 qubits' last stage
-// spent as long on its X terms as on its gates).  FP64 products and sums.
+// pass does, so the chunk is read once for up to four terms (24 circuits of 13..19 qubits 0.27 ms, with
+// one read a term 0.30; 1024 circuits of 10..20 qubits 5.3 and 5.4 ms).  FP64 products and sums.
 template <int NP>
 __device__ double measure_pass(const chunk_ctx& c, const uint32_t (&p)[4], const double (&h2)[4], uint32_t tid) {
   uint32_t boff[1 << NP];

@@ -18,8 +18,8 @@
 // before.  Stages run level by level: one launch runs stage k of every circuit
 // (of a round, see host/batch.cpp) as a queue of items, each a few chunks of one
 // circuit's stage, so that a few large circuits fill the device too (24 circuits
-// of 13..19 qubits: 0.30 ms; one workgroup per circuit and all chunks: 7.4 ms.
-// 1024 of 10..20 qubits: 5.4 against 16.9 ms, the time of one 20-qubit circuit).
+// of 13..19 qubits: 0.27 ms; one workgroup per circuit and all chunks: 7.4 ms.
+// 1024 of 10..20 qubits: 5.2 against 16.9 ms, the time of one 20-qubit circuit).
 #pragma once
 
 #include <cstdint>
