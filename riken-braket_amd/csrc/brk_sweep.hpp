@@ -57,8 +57,8 @@ struct sweep_segment {
   uint8_t group[4];   // ascending local bits
   uint8_t qubits[4];  // ... and the physical qubits they are
   uint8_t flags, num_macros;
-  uint16_t first_macro;
-  uint32_t pad;
+  uint16_t pad;
+  uint32_t first_macro;  // (a block takes as many macros as its gates need)
 };
 struct sweep_header {
   uint32_t num_segments;  // they follow the header

@@ -348,3 +348,39 @@ def test_op_wider_than_a_block_uses_the_run_sweep():
     tm[k] -= math.pi / 2
     ref = 0.5 * (plain_energy(n, W.with_parameters(ops, tp), J, h) - plain_energy(n, W.with_parameters(ops, tm), J, h))
     assert abs(g1[k] - ref) < 1e-11
+
+
+@pytest.mark.parametrize("dtype", [brk.C128, brk.C64])
+def test_long_circuit_on_one_qubit(dtype):
+    """66 000 parameters, RY and RX in turn on the highest of 12 qubits: one sweep block would hold more than
+    2^16 macros.  Against the adjoint method on the qubit's own 2-vector.  Every gate rounds with a relative
+    error of a few units of its type at random, in both directions of the sweep: 2 N of them add up to
+    4 sqrt(2 N) units of E's scale, 8 times that is the bar."""
+    n, count = 12, 66000
+    rng = np.random.default_rng(77)
+    theta = rng.uniform(-3, 3, count)
+    ops = [("RX" if k % 2 else "RY", (n - 1,), (), (float(theta[k]),)) for k in range(count)]
+    J, h = rng.uniform(-1, 1, n - 1), rng.uniform(-1, 1, n)
+    note(f"gpu adjoint: {count} gates on one qubit, dtype={dtype}")
+    e, g, back = adjoint(n, ops, J, h, dtype)
+    X, Y, Z = np.array([[0, 1], [1, 0]]), np.array([[0, -1j], [1j, 0]]), np.diag([1.0, -1.0])
+    G = [X if k % 2 else Y for k in range(count)]
+    U = [math.cos(t / 2) * np.eye(2) - 1j * math.sin(t / 2) * G[k] for k, t in enumerate(theta)]
+    psi = np.array([1.0, 0.0], dtype=complex)
+    for u in U:
+        psi = u @ psi
+    # the others stay |0>: their Z are 1, their X average 0
+    lam = (np.sum(J[:-1]) * np.eye(2) + J[-1] * Z + h[-1] * X) @ psi
+    want = np.empty(count)
+    want_e = np.vdot(psi, lam).real
+    for k in range(count - 1, -1, -1):
+        want[k] = 2 * np.vdot(lam, -0.5j * (G[k] @ psi)).real
+        psi, lam = U[k].conj().T @ psi, U[k].conj().T @ lam
+    unit = 2.0 ** (-53 if dtype == brk.C128 else -24)
+    tol = 32 * math.sqrt(2 * count) * unit * (np.sum(np.abs(J)) + np.sum(np.abs(h)))
+    note(f"gpu adjoint: energy off {abs(e - want_e):.2e}, gradient {np.max(np.abs(g - want)):.2e}, bar {tol:.2e}")
+    assert abs(e - want_e) < tol
+    assert np.max(np.abs(g - want)) < tol
+    start = np.zeros(1 << n, dtype=complex)
+    start[0] = 1.0
+    assert np.max(np.abs(back - start)) < tol
