@@ -43,6 +43,10 @@ struct gate_desc {
 int describe_physical_op(int code, const unsigned* targets, unsigned num_targets, const unsigned* controls,
                          unsigned num_controls, const double* params, gate_desc* out);
 
+// The share of the state that the gate's plain kernel reads and writes: a condition bit above the line
+// boundary halves it.
+double plain_share(const gate_desc& d, int dtype);
+
 // What a block's kernel does for a gate: the described mode, with a 2x2 matrix told apart by the
 // exact zeros of its coefficients (the forms of pair_math).
 enum block_kind {

@@ -1769,6 +1769,17 @@ int describe_physical_op(int code, const unsigned* t, unsigned nt, const unsigne
   return BRK_OK;
 }
 
+// (by the plans of the entry points below)
+double plain_share(const gate_desc& d, int dtype) {
+  const bool swap = (d.cond & d.flip) != 0, one_target = (d.flip & (d.flip - 1ull)) == 0;
+  const bool lane = (swap || one_target) && (d.flip & ((1ull << lane_target_bits(dtype)) - 1ull)) != 0;
+  const unsigned threshold = lane ? LANE_BITS : line_bits(dtype);
+  // a SWAP's own condition counts where both its qubits are inserted
+  const uint64_t tested = lane ? d.cond & ~d.flip : d.cond;
+  const int halvings = __builtin_popcountll(tested >> threshold);
+  return std::ldexp(1.0, -halvings);
+}
+
 }  // namespace brk
 
 using namespace brk;

@@ -18,7 +18,7 @@
 //    the chunk are the same for all its amplitudes -- and moves may run out of
 //    order (launch_builder), so a launch takes the gates of two to four steps
 //    (20 qubits with 10 layers of RZ and CNOT: 9 for 41).
-// A group of one op runs on the plain kernels.
+// A group of one op, or of ops that act on a small part of the state, runs on the plain kernels.
 #include <hip/hip_runtime_api.h>
 
 #include <algorithm>
@@ -446,6 +446,8 @@ struct launch_builder {
     gate_desc desc;
   };
   chunk_shape shape;
+  int dtype;
+  double state_bytes;
   unsigned line_bits;
   Plain plain;
   Block block;
@@ -454,7 +456,8 @@ struct launch_builder {
   unsigned count = 0;
   uint64_t mixing = 0;
   size_t room = 0;
-  brk_circuit::op first;
+  double plain_bytes = 0.0;  // what the ops' plain kernels move, as state (plain_is_faster)
+  std::vector<brk_circuit::op> ops;  // for their plain kernels: all of them while those are faster
   // the ops passed over: what they flip, and all that they touch; whether one of them rounds
   std::vector<entry> rest;
   uint64_t rest_mixing = 0, rest_qubits = 0;
@@ -464,7 +467,10 @@ struct launch_builder {
   block_args args{};
 
   launch_builder(unsigned n, int dtype, Plain p, Block b)
-      : shape(n, dtype), line_bits(block_run_qubits(dtype)), plain(p), block(b) {}
+      : shape(n, dtype), dtype(dtype), state_bytes((dtype == BRK_C128 ? 16.0 : 8.0) * (double)(1ull << n)),
+        line_bits(block_run_qubits(dtype)), plain(p), block(b) {
+    ops.reserve(BLOCK_MAX_OPS);
+  }
   int add(brk_circuit::op&& m, const gate_desc& d) {
     if (!shape.enabled() || !shape.fits(mixing_bits(d))) {  // too wide for a chunk
       if (int st = flush()) return st;
@@ -485,9 +491,10 @@ struct launch_builder {
     const bool rounds = d.mode != BLOCK_SWAP;
     const bool in_order = !(rest_mixing & d.qubits) && !(m & rest_qubits) && !(rounds && rest_rounds);
     if (in_order && shape.fits(mixing | m) && room + block_op_room(d) <= BLOCK_ARG_ROOM) {
-      if (!count) first = std::move(op);
       mixing |= m;
       room += block_op_room(d);
+      plain_bytes += std::max(plain_share(d, dtype) * state_bytes + 6e6, 12e6);
+      if (!count || plain_is_faster()) ops.push_back(std::move(op));  // (it stays slower once it is)
       descs[count++] = d;
       return count == (unsigned)BLOCK_MAX_OPS;
     }
@@ -498,8 +505,24 @@ struct launch_builder {
     // (nothing passes a gate that rounds once every qubit is touched)
     return rest.size() == LOOKAHEAD || (rest_rounds && rest_qubits == (1ull << shape.n) - 1ull);
   }
+  // A launch moves the whole state whatever its gates act on; their plain kernels move what they act on,
+  // but no less than what passes in a kernel's 3 us (12 MB of the state), and 6 MB more each for their
+  // start and end.  The line is where both take the same time: complex64 plain kernels move a state 10 %
+  // slower than a launch does (2 GiB: 735 and 690 us), complex128 ones 4 % faster (4 GiB: 1360 and 1420).
+  // 28 qubits complex128, launch against plain kernels: two Z with 10 controls 1.38 ms and 17 us, two X
+  // with 4 controls 1.43 and 0.18 ms, two CNOT 1.42 and 1.36, H and CZ 1.45 and 1.69, four CZ 1.38 and
+  // 1.34; 22 qubits: two CZ 22 and 11 us, four 23 and 27; up to 20 qubits a launch is always the faster.
+  // Over 946 circuits of 2 to 8 such gates (10 to 28 qubits, both types) the choice is at most 3 % slower
+  // than the other one.
+  bool plain_is_faster() const {
+    return plain_bytes < (dtype == BRK_C128 ? 1.08 : 0.90) * state_bytes;
+  }
   int launch() {
-    if (count == 1) return plain(first);
+    if (count == 1 || plain_is_faster()) {
+      for (const brk_circuit::op& op : ops)
+        if (int st = plain(op)) return st;
+      return BRK_OK;
+    }
     make_block_program(descs, count, shape.n, mixing, shape.num_local(), line_bits, &prog);
     make_passes(prog, line_bits);
     pack(prog, &args);
@@ -516,8 +539,10 @@ struct launch_builder {
       pending.swap(rest);
       rest.clear();
       count = 0;
+      ops.clear();
       mixing = rest_mixing = rest_qubits = 0;
       room = 0;
+      plain_bytes = 0.0;
       rest_rounds = false;
       complete = false;
       for (next = 0; next < pending.size() && !complete; ++next)

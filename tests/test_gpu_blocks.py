@@ -193,3 +193,27 @@ def test_block_order_run_matches_plain(oracle, n, dtype, seed):
         ref = s.copy()
         run_ops(oracle, ref, ops)
         assert np.max(np.abs(blocked - ref)) < 1e-12
+
+
+@pytest.mark.parametrize("n,dtype,seed", [(22, brk.C128, 61), (23, brk.C64, 62), (24, brk.C128, 63)])
+def test_many_controls_gate_by_gate_bitwise(n, dtype, seed):
+    """Gates with up to 9 controls among others, on states where two or three of them are cheaper as plain
+    kernels than as a launch: the bits of brk_circuit_run_timed (a plain kernel per op)."""
+    note(f"gpu blocks: many controls n={n} dtype={dtype} seed={seed}")
+    rng = np.random.default_rng(seed)
+    ops = []
+    for _ in range(12):
+        ops += random_ops(n, int(rng.integers(1, 4)), int(rng.integers(1 << 30)), max_controls=9, local_swaps=1)
+        q = [int(x) for x in rng.permutation(n)[:7]]
+        ops += [("Z", (q[0],), tuple(q[1:]), ()), ("X", (q[0],), tuple(q[1:5]), ()),
+                ("X", (q[1],), (q[0], q[2], q[3]), ())]
+    s = D.random_state(n, rng)
+    s[rng.random(s.size) < 0.3] = 0.0
+    c = brk.Circuit(n, ops)
+    a, b = DeviceState.from_host(s, dtype), DeviceState.from_host(s, dtype)
+    final, _ = c.run_timed(a.ptr, dtype)
+    assert c.run(b.ptr, dtype) == final
+    want, got = a.download(), b.download()
+    a.free()
+    b.free()
+    assert same_bits(want, got)
