@@ -40,3 +40,13 @@ def test_every_gate_runs_once(check, kind, gates, n, num_local):
     assert got["status"] == 0 and got["blocks"] >= 1
     assert (got["wrong"], got["missed"], got["twice"]) == (0, 0, 0)
     assert code == 0
+
+
+@pytest.mark.parametrize("kind,gates,n,num_local", [("chain", 100000, 12, 12), ("phases", 60000, 20, 11),
+                                                    ("layers", 300000, 12, 12)])
+def test_planning_time_grows_with_the_circuit(check, kind, gates, n, num_local):
+    """About 2 us a gate (0.1-0.2 s here), however long the circuit: planning that looks at all gates left for
+    every macro or segment takes 8 s or more for the first and the second."""
+    code, got = check(kind, gates, n, num_local)
+    assert code == 0
+    assert got["seconds"] < 1.5
