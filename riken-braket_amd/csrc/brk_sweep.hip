@@ -246,10 +246,11 @@ void k_sweep(cpx<R>* __restrict__ psi, cpx<R>* __restrict__ lam, const void* pro
     }
     __syncthreads();
   }
+  uint32_t first_macro = 0;  // of the segment (counted: with a number to load 24 qubits took 9.54 ms, now 9.49)
   for (uint32_t si = 0; si < num_segments; ++si) {
     const csegment seg = segments + si;
     const uint32_t flags = seg->flags, num_macros = seg->num_macros;
-    const cmacro first = macros + seg->first_macro;
+    const cmacro first = macros + first_macro;
     uint32_t base = t, dep[GROUP], q[SWEEP_GROUP];
     dep[0] = 0;
 #pragma unroll
@@ -284,7 +285,7 @@ void k_sweep(cpx<R>* __restrict__ psi, cpx<R>* __restrict__ lam, const void* pro
     }
     for (uint32_t mi = 0; mi < num_macros; ++mi) {
       const cmacro mac = first + mi;
-      fetch(seg->first_macro + mi + 1);
+      fetch(first_macro + mi + 1);
       double value[8] = {};
       apply_diagonal<R, BOTH>(x, y, mac, low, q, value);
       mix<0, R, BOTH>(x, y, mac, value);
@@ -329,6 +330,7 @@ void k_sweep(cpx<R>* __restrict__ psi, cpx<R>* __restrict__ lam, const void* pro
         }
       }
     }
+    first_macro += num_macros;
     if (seen == 1u) __builtin_amdgcn_s_sleep(0);  // (keeps the fetches)
     if (flags & SWEEP_STORES) return;
   }

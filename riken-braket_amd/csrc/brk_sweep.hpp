@@ -56,9 +56,9 @@ enum sweep_flags {
 struct sweep_segment {
   uint8_t group[4];   // ascending local bits
   uint8_t qubits[4];  // ... and the physical qubits they are
-  uint8_t flags, num_macros;
-  uint16_t pad;
-  uint32_t first_macro;  // (a block takes as many macros as its gates need)
+  uint8_t flags, num_macros;  // its macros follow those of the segments before it
+  uint16_t pad16;
+  uint32_t pad;
 };
 struct sweep_header {
   uint32_t num_segments;  // they follow the header

@@ -373,7 +373,6 @@ int plan_sweep(const std::vector<sweep_gate>& gates, unsigned n, unsigned num_lo
         bits |= 1u << rank[q[k]];
         ++k;
       }
-      s.first_macro = (uint32_t)macros.size();
       do {
         macros.push_back(make_macro(p, q, only_signs));
         ++s.num_macros;

@@ -83,9 +83,10 @@ int main(int argc, char** argv) {
     for (uint32_t s = 0; s < h.num_segments; ++s) {
       sweep_segment seg;
       std::memcpy(&seg, p + sizeof(h) + s * sizeof(seg), sizeof(seg));
-      if (seg.first_macro != next || seg.first_macro + seg.num_macros > h.num_macros) ++wrong;
+      const size_t first = next;
       next += seg.num_macros;
-      for (size_t m = seg.first_macro; m < (size_t)seg.first_macro + seg.num_macros && m < h.num_macros; ++m) {
+      if (seg.num_macros == 0 || next > h.num_macros) ++wrong;
+      for (size_t m = first; m < next && m < h.num_macros; ++m) {
         sweep_macro mac;
         std::memcpy(&mac, p + h.macros_at + m * sizeof(mac), sizeof(mac));
         for (int32_t slot : mac.slot)
