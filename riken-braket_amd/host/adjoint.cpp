@@ -528,8 +528,12 @@ static int sweep_gradient(const std::vector<sweep_gate>& forward_gates, const st
   const unsigned L = dtype == BRK_C128 ? SWEEP_REVERSE_LOCAL_C128 : SWEEP_REVERSE_LOCAL_C64;
   const uint64_t chunks = size >> L;
   // one leased buffer: nparams x chunks partials, the nparams gradients, the energy's partials, then
-  // the programs, which go up from pinned memory
-  const size_t nsums = std::max(1u, nparams), room = 2 * sweep_program_bound(forward_gates.size());
+  // the programs, which go up from pinned memory.  That holds both sweeps' programs, of a long circuit as
+  // many blocks as fit in SWEEP_STAGING: once it is full, it is used again after the blocks in it have run.
+  constexpr size_t SWEEP_STAGING = 4u << 20;
+  static_assert(SWEEP_STAGING >= 4 * SWEEP_BLOCK_BYTES, "planning goes on while blocks run");
+  const size_t nsums = std::max(1u, nparams);
+  const size_t room = std::min(2 * sweep_program_bound(forward_gates.size()), SWEEP_STAGING);
   const size_t doubles = (size_t)nparams * chunks + nsums + 2 * INNER_BLOCKS;
   partials_lease lease;
   if (int s = get_partials(doubles + room / sizeof(double) + 8, room, st, lease)) return s;
@@ -540,7 +544,11 @@ static int sweep_gradient(const std::vector<sweep_gate>& forward_gates, const st
   size_t used = 0;
   auto run = [&](const std::vector<sweep_gate>& gates, unsigned num_local, void* second) {
     return plan_sweep(gates, n, num_local, line_bits, [&](const void* program, size_t bytes) -> int {
-      if (used + bytes > room) return fail(BRK_ERR_INVALID_ARGUMENT, "sweep programs outgrow their buffer");
+      if (used + bytes > room) {
+        if (bytes > room) return fail(BRK_ERR_INVALID_ARGUMENT, "a sweep program outgrows its buffer");
+        if (hipStreamSynchronize(st) != hipSuccess) return fail(BRK_ERR_HIP, "hipStreamSynchronize failed");
+        used = 0;
+      }
       std::memcpy(lease.pinned + used, program, bytes);
       if (hipMemcpyAsync(device + used, lease.pinned + used, bytes, hipMemcpyHostToDevice, st) != hipSuccess)
         return fail(BRK_ERR_HIP, "uploading the sweep programs failed");

@@ -338,12 +338,13 @@ int plan_sweep(const std::vector<sweep_gate>& gates, unsigned n, unsigned num_lo
   // two exchanges through LDS whatever it runs (24 qubits, 12 layers: 151 reverse macros in 58
   // segments; 178 in 56 with macros of any size).
   constexpr unsigned CHAIN_GATES = 4;
+  constexpr unsigned BLOCK_GATES = 2 * SWEEP_GROUP * SWEEP_BLOCK_MACROS;  // a full block's macros run no more
   std::vector<sweep_segment> segments;
   std::vector<sweep_macro> macros;
   std::vector<char> program;
   while (p.remaining) {
     // local qubits: the line's, the greedy ones, then the lowest others
-    uint32_t local = p.grow(line, all, num_local - line_bits, ~0u);
+    uint32_t local = p.grow(line, all, num_local - line_bits, BLOCK_GATES);
     for (unsigned q = 0; (unsigned)__builtin_popcount(local) < num_local; ++q) local |= 1u << q;
     sweep_header h{};
     unsigned rank[32] = {}, r = 0;
@@ -354,7 +355,7 @@ int plan_sweep(const std::vector<sweep_gate>& gates, unsigned n, unsigned num_lo
     }
     segments.clear();
     macros.clear();
-    while (p.remaining) {
+    while (p.remaining && macros.size() + SWEEP_MAX_MACROS <= SWEEP_BLOCK_MACROS) {
       uint32_t group = p.grow(0, local, SWEEP_GROUP, 4 * SWEEP_GROUP * SWEEP_MAX_MACROS);
       // without a gate for these qubits the block ends (signs wait for a block that needs them), or
       // only signs are left

@@ -29,6 +29,12 @@ struct sweep_gate {
 int plan_sweep(const std::vector<sweep_gate>& gates, unsigned n, unsigned num_local, unsigned line_bits,
                const std::function<int(const void* program, size_t bytes)>& emit);
 
+// A block ends at this many macros (ordinary ones hold below 100; every macro runs a gate at least), so
+// that its program has a size that does not depend on the circuit's.
+constexpr size_t SWEEP_BLOCK_MACROS = 1024;
+constexpr size_t SWEEP_BLOCK_BYTES =
+    sizeof(sweep_header) + SWEEP_BLOCK_MACROS * (sizeof(sweep_macro) + sizeof(sweep_segment)) + 64;
+
 // Bytes the programs of a plan of this many gates take at most: a macro and a segment for every
 // gate, and a block's header and padding (every block runs at least one gate).
 inline size_t sweep_program_bound(size_t gates) {

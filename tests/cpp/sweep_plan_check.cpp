@@ -95,6 +95,7 @@ int main(int argc, char** argv) {
     }
     if (next != h.num_macros) ++wrong;
     if (h.macros_at + (size_t)h.num_macros * sizeof(sweep_macro) > bytes || bytes % 64 != 0) ++wrong;
+    if (bytes > SWEEP_BLOCK_BYTES) ++wrong;
     ++blocks;
     largest = std::max(largest, (size_t)h.num_macros);
     bytes_in_all += bytes;

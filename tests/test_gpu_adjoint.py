@@ -352,8 +352,8 @@ def test_op_wider_than_a_block_uses_the_run_sweep():
 
 @pytest.mark.parametrize("dtype", [brk.C128, brk.C64])
 def test_long_circuit_on_one_qubit(dtype):
-    """66 000 parameters, RY and RX in turn on the highest of 12 qubits: one sweep block would hold more than
-    2^16 macros.  Against the adjoint method on the qubit's own 2-vector.  Every gate rounds with a relative
+    """66 000 parameters, RY and RX in turn on the highest of 12 qubits: more than 2^16 macros,
+    and programs beyond what the upload buffer holds at a time.  Against the adjoint method on the qubit's own 2-vector.  Every gate rounds with a relative
     error of a few units of its type at random, in both directions of the sweep: 2 N of them add up to
     4 sqrt(2 N) units of E's scale, 8 times that is the bar."""
     n, count = 12, 66000

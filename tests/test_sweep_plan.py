@@ -35,7 +35,7 @@ def check(tmp_path_factory):
                                                     ("layers", 300000, 12, 12), ("layers", 576, 24, 11),
                                                     ("phases", 3000, 14, 11)])
 def test_every_gate_runs_once(check, kind, gates, n, num_local):
-    """Also where a block takes more than 2^16 macros: a segment finds its macros by their number."""
+    """Also in circuits of more than 2^16 macros, and in blocks of a bounded size."""
     code, got = check(kind, gates, n, num_local)
     assert got["status"] == 0 and got["blocks"] >= 1
     assert (got["wrong"], got["missed"], got["twice"]) == (0, 0, 0)
