@@ -15,6 +15,7 @@
 #include "brk_block.hpp"
 
 #include <algorithm>
+#include <cmath>
 #include <complex>
 #include <vector>
 
@@ -824,7 +825,8 @@ static int make_ising_args(unsigned nq, const double* J, const double* h, ising_
   return BRK_OK;
 }
 
-// <H> in passes of k_ising (terms with h = 0 are left out).
+// <H> in passes of k_ising (terms with h = 0 are left out).  A field that is not finite multiplies its
+// qubit's whole <X>, after the passes: over parts of the sum it gives 0 * inf and inf - inf.
 template <typename R>
 static int ising_energy(const void* first, uint64_t size, const ising_args& args, double* result, void* stream) {
   constexpr unsigned L = ising_shape<R>::L, line = sizeof(R) == 8 ? 3 : 4;  // qubits of a 128-byte line
@@ -847,7 +849,7 @@ static int ising_energy(const void* first, uint64_t size, const ising_args& args
     for (unsigned q = 0; r < L; ++q) {
       if (!(local >> q & 1ull)) continue;
       p.pos[r] = q;
-      if (q >= next && q < end && args.h[q] != 0.0) {
+      if (q >= next && q < end && args.h[q] != 0.0 && std::isfinite(2.0 * args.h[q])) {
         p.measure |= 1u << r;
         p.h2[r] = 2.0 * args.h[q];  // <X_q> = 2 sum Re conj(a0) a1
       }
@@ -860,7 +862,7 @@ static int ising_energy(const void* first, uint64_t size, const ising_args& args
   if (int st = get_reduce_scratch(&sc)) return st;
   const size_t values = passes.size() * grid;
   if (values > (size_t)RED_BLOCKS * RED_MAX_VALUES) return fail(BRK_ERR_INVALID_ARGUMENT, "too many Ising passes");
-  std::lock_guard<std::mutex> hold(sc->busy);
+  std::unique_lock<std::mutex> hold(sc->busy);
   hipStream_t s = as_stream(stream);
   int status = BRK_OK;
   for (size_t k = 0; !status && k < passes.size(); ++k) {
@@ -873,6 +875,13 @@ static int ising_energy(const void* first, uint64_t size, const ising_args& args
   if (synced != hipSuccess) return fail(BRK_ERR_HIP, "Ising energy: %s", hipGetErrorString(synced));
   double total = 0.0;
   for (size_t k = 0; k < values; ++k) total += sc->partials[k];
+  hold.unlock();
+  for (unsigned q = 0; q < n; ++q) {
+    if (std::isfinite(2.0 * args.h[q])) continue;
+    double raw[3];
+    if (int st = spin_raw(first, size, sizeof(R) == 8 ? BRK_C128 : BRK_C64, q, raw, stream)) return st;
+    total += 2.0 * args.h[q] * raw[0];
+  }
   *result = total;
   return BRK_OK;
 }

@@ -152,3 +152,32 @@ def test_reduction_tiles(oracle, n, dtype):
         assert abs(brk.expectation_pauli_string(a.ptr, a.size, dtype, "X", [q]) - 2 * x.real) < 1e-12
     a.free()
     b.free()
+
+
+@pytest.mark.parametrize("n,dtype", [(3, brk.C128), (9, brk.C64), (14, brk.C128), (16, brk.C64)])
+def test_ising_fields_that_are_not_finite(n, dtype):
+    """A field multiplies its qubit's whole <X>: an infinite one gives the infinity of that sign beside finite
+    terms (also where the state is smaller than a chunk, and where parts of the sum differ in sign), two of
+    opposite results give no number, and so does one that is no number."""
+    note(f"gpu ising with infinite fields n={n} dtype={dtype}")
+    rng = np.random.default_rng(90 + n)
+    host = D.random_state(n, rng).astype(np.complex128 if dtype == brk.C128 else np.complex64)
+    st = DeviceState.from_host(host, dtype)
+    J, h = rng.uniform(-1, 1, n - 1), rng.uniform(-1, 1, n)
+    signs = []
+    for q in (0, n // 2, n - 1):
+        x = brk.spin_expectation_value(st.ptr, st.size, dtype, q)[0]
+        assert x != 0.0
+        signs.append((q, np.sign(x)))
+        for value in (np.inf, -np.inf, 1.7e308):  # (the last: finite, its double is not)
+            g = h.copy()
+            g[q] = value
+            assert brk.expectation_ising(st.ptr, st.size, dtype, J, g) == np.copysign(np.inf, value) * np.sign(x)
+        g = h.copy()
+        g[q] = np.nan
+        assert np.isnan(brk.expectation_ising(st.ptr, st.size, dtype, J, g))
+    g = h.copy()
+    (a, sa), (b, sb) = signs[:2]
+    g[a], g[b] = np.inf * sa, -np.inf * sb
+    assert np.isnan(brk.expectation_ising(st.ptr, st.size, dtype, J, g))
+    st.free()
