@@ -407,27 +407,23 @@ std::vector<size_t> block_order(const std::vector<brk_circuit::op>& ops, unsigne
   return order;
 }
 
-static brk_circuit::op map_op(const brk_circuit::op& o, const permutation& perm) {
-  brk_circuit::op m = o;
-  for (auto& q : m.targets) q = perm.perm[q];
-  for (auto& q : m.controls) q = perm.perm[q];
-  return m;
+// Op o of the circuit at physical qubits (m's lists are used again); advances the map over it.
+static void place_op(const brk_circuit::op& o, permutation& perm, brk_circuit::op* m) {
+  *m = o;
+  if (o.code == BRK_OP_LOCAL_SWAP) {  // given at physical qubits; the map changes for the ops after it
+    perm.permutate(perm.inverse[o.targets[0]], perm.inverse[o.targets[1]]);
+    return;
+  }
+  for (auto& q : m->targets) q = perm.perm[q];
+  for (auto& q : m->controls) q = perm.perm[q];
 }
 
-// Describes op i of the circuit at physical qubits and advances the map over it.
-static int physical_op(const brk_circuit::op& o, permutation& perm, brk_circuit::op* m, gate_desc* d) {
-  if (o.code == BRK_OP_LOCAL_SWAP) {
-    // the data of a local swap is a SWAP gate on its two physical qubits
-    // (swap_permutated_local_qubits.hpp:64-77); the map changes for the ops after it
-    *m = o;
-    if (int st = describe_physical_op(BRK_OP_SWAP, o.targets.data(), 2, nullptr, 0, nullptr, d)) return st;
-    perm.permutate(perm.inverse[o.targets[0]], perm.inverse[o.targets[1]]);
-    return BRK_OK;
-  }
-  *m = map_op(o, perm);
-  return describe_physical_op(m->code, m->targets.data(), (unsigned)m->targets.size(),
-                              m->controls.empty() ? nullptr : m->controls.data(), (unsigned)m->controls.size(),
-                              m->params.data(), d);
+// The description of an op at physical qubits: the data of a local swap is a SWAP gate on its two qubits
+// (swap_permutated_local_qubits.hpp:64-77).
+static int describe_op(const brk_circuit::op& m, gate_desc* d) {
+  return describe_physical_op(m.code == BRK_OP_LOCAL_SWAP ? (int)BRK_OP_SWAP : m.code, m.targets.data(),
+                              (unsigned)m.targets.size(), m.controls.empty() ? nullptr : m.controls.data(),
+                              (unsigned)m.controls.size(), m.params.data(), d);
 }
 
 // Collects ops into launches and hands each over as soon as it is complete.  A launch takes the ops
@@ -468,9 +464,7 @@ struct launch_builder {
 
   launch_builder(unsigned n, int dtype, Plain p, Block b)
       : shape(n, dtype), dtype(dtype), state_bytes((dtype == BRK_C128 ? 16.0 : 8.0) * (double)(1ull << n)),
-        line_bits(block_run_qubits(dtype)), plain(p), block(b) {
-    ops.reserve(BLOCK_MAX_OPS);
-  }
+        line_bits(block_run_qubits(dtype)), plain(p), block(b) {}
   int add(brk_circuit::op&& m, const gate_desc& d) {
     if (!shape.enabled() || !shape.fits(mixing_bits(d))) {  // too wide for a chunk
       if (int st = flush()) return st;
@@ -588,10 +582,11 @@ static int build_plan(const brk_circuit* circuit, int dtype, const unsigned* per
     return BRK_OK;
   };
   launch_builder<decltype(plain), decltype(block)> b(n, dtype, plain, block);
+  brk_circuit::op m;
   for (unsigned i = 0; i < circuit->ops.size(); ++i) {
     gate_desc d;
-    brk_circuit::op m;
-    if (int st = physical_op(circuit->ops[i], perm, &m, &d)) return st;
+    place_op(circuit->ops[i], perm, &m);
+    if (int st = describe_op(m, &d)) return st;
     if (!shape.enabled() || s.num_ops == (unsigned)BLOCK_MAX_OPS || !shape.fits(qubits | d.qubits)) close_step();
     if (!s.num_ops) s.first_op = i;
     ++s.num_ops;
@@ -617,12 +612,20 @@ int run_in_blocks(const brk_circuit* circuit, void* first, int dtype, permutatio
   const uint64_t size = 1ull << circuit->num_qubits;
   auto plain = [&](const brk_circuit::op& m) { return apply_physical_op(m, first, size, dtype, stream); };
   auto block = [&](const block_args& a) { return launch_block(a, first, size, dtype, stream); };
+  brk_circuit::op m;
+  if (circuit->ops.size() <= 1 || !chunk_shape(circuit->num_qubits, dtype).enabled()) {  // nothing to collect
+    for (const auto& o : circuit->ops) {
+      place_op(o, perm, &m);
+      if (int st = plain(m)) return st;
+    }
+    return BRK_OK;
+  }
   launch_builder<decltype(plain), decltype(block)> b(circuit->num_qubits, dtype, plain, block);
   for (const auto& o : circuit->ops) {
     gate_desc d;
-    brk_circuit::op m;
-    if (int st = physical_op(o, perm, &m, &d)) return st;
-    if (int st = b.add(std::move(m), d)) return st;
+    place_op(o, perm, &m);
+    if (int st = describe_op(m, &d)) return st;
+    if (int st = b.add(std::move(m), d)) return st;  // (takes the op only where it keeps it)
   }
   return b.flush();
 }
