@@ -224,7 +224,7 @@ struct partials_slot {
   std::mutex busy;
   double* ptr = nullptr;
   size_t doubles = 0;
-  char* pinned = nullptr;  // staging of the sweeps' programs
+  char* pinned = nullptr;  // the sweeps' results and the staging of their programs
   size_t pinned_bytes = 0;
 };
 static std::mutex g_partials_mutex;
@@ -527,20 +527,21 @@ static int sweep_gradient(const std::vector<sweep_gate>& forward_gates, const st
   const unsigned line_bits = dtype == BRK_C128 ? 3 : 4;  // one 128-byte line
   const unsigned L = dtype == BRK_C128 ? SWEEP_REVERSE_LOCAL_C128 : SWEEP_REVERSE_LOCAL_C64;
   const uint64_t chunks = size >> L;
-  // one leased buffer: nparams x chunks partials, the nparams gradients, the energy's partials, then
-  // the programs, which go up from pinned memory.  That holds both sweeps' programs, of a long circuit as
-  // many blocks as fit in SWEEP_STAGING: once it is full, it is used again after the blocks in it have run.
+  // one leased buffer: nparams x chunks partials, then the programs.  In pinned memory: the nparams gradients
+  // and the energy's partials, which the kernels write there (copies back took 10 us more a call), then the
+  // programs on their way up.  There is room for both sweeps' programs, of a long circuit for as many blocks
+  // as fit in SWEEP_STAGING: once it is full, it is used again after the blocks in it have run.
   constexpr size_t SWEEP_STAGING = 4u << 20;
   static_assert(SWEEP_STAGING >= 4 * SWEEP_BLOCK_BYTES, "planning goes on while blocks run");
-  const size_t nsums = std::max(1u, nparams);
   const size_t room = std::min(2 * sweep_program_bound(forward_gates.size()), SWEEP_STAGING);
-  const size_t doubles = (size_t)nparams * chunks + nsums + 2 * INNER_BLOCKS;
+  const size_t doubles = (size_t)nparams * chunks, results = nparams + 2 * INNER_BLOCKS;
   partials_lease lease;
-  if (int s = get_partials(doubles + room / sizeof(double) + 8, room, st, lease)) return s;
-  double* partials = lease.ptr;
-  double* sums = partials + (size_t)nparams * chunks;
-  double* energy_partials = sums + nsums;
-  char* device = reinterpret_cast<char*>(((uintptr_t)(energy_partials + 2 * INNER_BLOCKS) + 63) & ~(uintptr_t)63);
+  if (int s = get_partials(doubles + room / sizeof(double) + 8, results * sizeof(double) + room, st, lease)) return s;
+  double* const partials = lease.ptr;
+  char* const device = reinterpret_cast<char*>(((uintptr_t)(partials + doubles) + 63) & ~(uintptr_t)63);
+  double* const sums = reinterpret_cast<double*>(lease.pinned);
+  double* const energy_partials = sums + nparams;
+  char* const staging = reinterpret_cast<char*>(sums + results);
   size_t used = 0;
   auto run = [&](const std::vector<sweep_gate>& gates, unsigned num_local, void* second) {
     return plan_sweep(gates, n, num_local, line_bits, [&](const void* program, size_t bytes) -> int {
@@ -549,8 +550,8 @@ static int sweep_gradient(const std::vector<sweep_gate>& forward_gates, const st
         if (hipStreamSynchronize(st) != hipSuccess) return fail(BRK_ERR_HIP, "hipStreamSynchronize failed");
         used = 0;
       }
-      std::memcpy(lease.pinned + used, program, bytes);
-      if (hipMemcpyAsync(device + used, lease.pinned + used, bytes, hipMemcpyHostToDevice, st) != hipSuccess)
+      std::memcpy(staging + used, program, bytes);
+      if (hipMemcpyAsync(device + used, staging + used, bytes, hipMemcpyHostToDevice, st) != hipSuccess)
         return fail(BRK_ERR_HIP, "uploading the sweep programs failed");
       const int status = launch_sweep(device + used, num_local, psi, second, size, dtype, partials, stream);
       used += bytes;
@@ -562,14 +563,11 @@ static int sweep_gradient(const std::vector<sweep_gate>& forward_gates, const st
   if (!status) status = launch_inner_partials(lam, psi, size, dtype, energy_partials, stream);
   if (!status) status = run(reverse_gates, L, lam);
   if (!status) status = sum_gradient_partials(partials, nparams, chunks, 2.0, sums, stream);
-  std::vector<double> host(nsums + 2 * INNER_BLOCKS);
-  if (!status && hipMemcpyAsync(host.data(), sums, host.size() * sizeof(double), hipMemcpyDeviceToHost, st) != hipSuccess)
-    status = fail(BRK_ERR_HIP, "copying the gradient failed");
   if (hipStreamSynchronize(st) != hipSuccess && !status) status = fail(BRK_ERR_HIP, "hipStreamSynchronize failed");
   if (status) return status;
-  std::copy(host.begin(), host.begin() + nparams, gradient);
+  std::copy(sums, sums + nparams, gradient);
   double e = 0.0;
-  for (int b = 0; b < INNER_BLOCKS; ++b) e += host[nsums + 2 * b];
+  for (int b = 0; b < INNER_BLOCKS; ++b) e += energy_partials[2 * b];
   *energy = e;
   return BRK_OK;
 }
