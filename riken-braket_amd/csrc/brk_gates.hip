@@ -635,6 +635,7 @@ __global__ __launch_bounds__(BLOCK_THREADS, BLOCK_WAVES_PER_SIMD) void k_block(c
   constexpr int GB = PER == 1 ? 0 : PER == 2 ? 1 : PER == 4 ? 2 : PER == 8 ? 3 : 4;
   constexpr int L = BLOCK_THREAD_BITS + GB;
   __shared__ cpx<R> lds[PER * BLOCK_THREADS];
+  static_assert(sizeof(s) % alignof(block_args) == 0, "the program follows the pointer");
   const block_view v((cbytes)__builtin_amdgcn_kernarg_segment_ptr() + sizeof(s));
   // consecutive chunks (neighbouring runs of memory) on one XCD
   const uint64_t chunk = chunk_base(xcd_chunk(blockIdx.x, gridDim.x), v, L);

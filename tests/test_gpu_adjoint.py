@@ -384,3 +384,25 @@ def test_long_circuit_on_one_qubit(dtype):
     start = np.zeros(1 << n, dtype=complex)
     start[0] = 1.0
     assert np.max(np.abs(back - start)) < tol
+
+
+@pytest.mark.parametrize("n,dtype", [(20, brk.C64), (21, brk.C64), (19, brk.C128), (20, brk.C128)])
+def test_merged_sweeps_on_many_chunks(n, dtype, access):
+    """256 chunks and more, forward and reverse (another order of the chunks over the chip than below), with
+    sign terms at every distance, against the per-run passes; the bars of the tests above."""
+    rng = np.random.default_rng(160 + n)
+    ops = one_qubit_ansatz(n, rng, 3, True)
+    J, h = rng.uniform(-1, 1, n - 1), rng.uniform(-1, 1, n)
+    psi0 = rng.normal(size=1 << n) + 1j * rng.normal(size=1 << n)
+    psi0 /= np.linalg.norm(psi0)
+    note(f"gpu adjoint merged vs chain, many chunks: n={n} dtype={dtype} ({access})")
+    e1, g1, back1 = adjoint(n, ops, J, h, dtype, psi0)
+    brk.tune("adjoint_blocks", 0)
+    try:
+        e0, g0, _ = adjoint(n, ops, J, h, dtype, psi0)
+    finally:
+        brk.tune("adjoint_blocks", 1)
+    tol = 1e-12 if dtype == brk.C128 else 2e-5
+    assert abs(e1 - e0) < tol
+    assert np.max(np.abs(g1 - g0)) < tol
+    assert np.max(np.abs(back1 - psi0)) < (1e-12 if dtype == brk.C128 else 1e-5)

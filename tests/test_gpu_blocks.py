@@ -5,6 +5,7 @@ block applies each gate with the same IEEE operation sequence -- and, for
 complex<double>, within 1e-12 of the CPU oracle.  Circuits mix every op kind
 with controls, multi-target strings, local swaps and a non-identity starting
 permutation."""
+import ctypes as C
 import sys
 
 import numpy as np
@@ -12,6 +13,7 @@ import pytest
 
 import brk
 import dense as D
+import hip
 from devstate import DeviceState
 from oracle_circuits import run_ops
 from randops import random_ops
@@ -217,3 +219,153 @@ def test_many_controls_gate_by_gate_bitwise(n, dtype, seed):
     a.free()
     b.free()
     assert same_bits(want, got)
+
+
+# brk_circuit_run itself runs in gate blocks: what follows compares with brk_circuit_run_timed, which launches
+# a plain kernel for every op.
+def gate_by_gate(n, ops, dtype, runs, perm0=None, seed=0):
+    """The final state of the ops on plain kernels, and of every run (circuit, pointer) -> permutation."""
+    rng = np.random.default_rng(seed)
+    s = D.random_state(n, rng)
+    c = brk.Circuit(n, ops)
+    a = DeviceState.from_host(s, dtype)
+    final, _ = c.run_timed(a.ptr, dtype, perm0)
+    want = a.download()
+    for run in runs:
+        a.upload(s)
+        assert run(c, a.ptr) == final
+        yield want, a.download()
+    a.free()
+
+
+@pytest.mark.parametrize("n,dtype,seed", [(3, brk.C128, 1), (9, brk.C128, 2), (12, brk.C128, 3), (13, brk.C128, 4),
+                                          (16, brk.C128, 5), (20, brk.C128, 6), (9, brk.C64, 10), (12, brk.C64, 7),
+                                          (14, brk.C64, 8), (20, brk.C64, 9), (23, brk.C64, 11)])
+def test_blocked_equals_gate_by_gate_bitwise(n, dtype, seed, access):
+    note(f"gpu blocked vs gate by gate n={n} dtype={dtype} seed={seed} ({access})")
+    ops = random_ops(n, 160, seed, local_swaps=3 if n >= 4 else 0)
+    perm0 = [int(q) for q in np.random.default_rng(seed).permutation(n)]
+    for want, got in gate_by_gate(n, ops, dtype, [lambda c, p: c.run_blocked(p, dtype, perm0)], perm0, seed):
+        assert same_bits(want, got)
+
+
+@pytest.mark.parametrize("dtype", [brk.C128, brk.C64])
+def test_dense_low_qubits_gate_by_gate_bitwise(dtype):
+    """Many gates on the line qubits and their neighbours: long blocks, every pair mode."""
+    n = 18
+    note(f"gpu blocks vs gate by gate: low-qubit circuit dtype={dtype}")
+    ops = random_ops(n, 400, 11, qubit_pool=range(10))
+    runs = [lambda c, p: c.run(p, dtype), lambda c, p: c.run_blocked(p, dtype)]
+    for want, got in gate_by_gate(n, ops, dtype, runs, None, 11):
+        assert same_bits(want, got)
+
+
+@pytest.mark.parametrize("dtype", [brk.C128, brk.C64])
+def test_large_state_gate_by_gate_bitwise(dtype):
+    """26 qubits, a plan run twice and the circuit run twice against two runs of plain kernels."""
+    n = 26
+    note(f"gpu blocks vs gate by gate: n={n} dtype={dtype}")
+    c = brk.Circuit(n, random_ops(n, 60, 12, max_controls=1))
+    plan = brk.BlockPlan(c, dtype)
+    got = []
+    for run in (lambda p: c.run_timed(p, dtype), plan.run, lambda p: c.run(p, dtype)):
+        st = DeviceState(n, dtype)
+        brk.fill_modular(st.ptr, st.size, dtype, (1e-4, 3e-4), (7, 3, 101, 11, 5, 97))
+        run(st.ptr)
+        run(st.ptr)
+        brk.call("brk_stream_synchronize", None)
+        got.append(st.download())
+        st.free()
+    assert same_bits(got[0], got[1]) and same_bits(got[0], got[2])
+
+
+def hip_runtime():
+    """The HIP runtime that the engine loaded, for the calls that its C ABI does not wrap."""
+    with open("/proc/self/maps") as f:
+        paths = {line.split()[-1] for line in f if "libamdhip64.so" in line}
+    (path,) = paths
+    return C.CDLL(path)
+
+
+@pytest.mark.parametrize("n,dtype", [(12, brk.C128), (14, brk.C64), (23, brk.C128)])
+def test_captured_runs_replay(n, dtype):
+    """A plan's run and a circuit's run captured in a graph: nothing of them lies in memory that a replay
+    could find changed.  Several replays, each from a new state after other runs, bit for bit the plain
+    kernels' result (23 qubits: launches and plain kernels)."""
+    note(f"gpu blocks captured n={n} dtype={dtype}")
+    brk.load()
+    runtime = hip_runtime()
+
+    def call(name, *args):
+        assert getattr(runtime, name)(*args) == 0, name
+
+    rng = np.random.default_rng(n)
+    ops = random_ops(n, 80, 70 + n, max_controls=4, local_swaps=2)
+    ops += [("Z", (n - 1,), tuple(range(n - 8, n - 1)), ()), ("X", (n - 2,), tuple(range(n - 9, n - 2)), ())]
+    c = brk.Circuit(n, ops)
+    plan = brk.BlockPlan(c, dtype)
+    st, other = DeviceState(n, dtype), DeviceState(n, dtype)
+    stream = C.c_void_p(hip.create_stream())
+    graphs = []
+    for run in (plan.run, lambda p, s: c.run(p, dtype, None, s)):
+        graph, executable = C.c_void_p(), C.c_void_p()
+        call("hipStreamBeginCapture", stream, 0)
+        run(st.ptr, stream.value)
+        call("hipStreamEndCapture", stream, C.byref(graph))
+        call("hipGraphInstantiate", C.byref(executable), graph, None, None, C.c_size_t(0))
+        call("hipGraphDestroy", graph)
+        graphs.append(executable)
+    del plan
+    for k in range(4):
+        s = D.random_state(n, rng)
+        other.upload(s)
+        c.run_timed(other.ptr, dtype)
+        want = other.download()
+        for executable in graphs:
+            st.upload(s)
+            brk.call("brk_stream_synchronize", None)
+            call("hipGraphLaunch", executable, stream)
+            hip.synchronize(stream.value)
+            assert same_bits(want, st.download()), k
+            c.run(other.ptr, dtype)  # other runs between the replays
+            brk.call("brk_stream_synchronize", None)
+    for executable in graphs:
+        call("hipGraphExecDestroy", executable)
+    call("hipStreamDestroy", stream)
+    st.free()
+    other.free()
+
+
+@pytest.mark.slow
+def test_33_qubits_gate_by_gate_bitwise():
+    """More than 2^32 amplitudes (64-bit indices in the blocks): gates, controls, moves and a local swap on the
+    highest qubits, in gate blocks against plain kernels, every amplitude."""
+    n = 33
+    if hip.mem_info()[0] < 140 << 30:
+        pytest.skip("needs 140 GiB of free device memory")
+    note(f"gpu blocks: n={n} complex64")
+    ops = [("H", (32,), (), ()), ("X", (0,), (32,), ()), ("RZ", (32,), (), (0.7,)), ("X", (32,), (5,), ()),
+           ("U3", (31,), (), (0.3, 0.9, -0.4)), ("H", (4,), (32,), ()), ("Z", (32,), (31,), ()),
+           ("SWAP", (32, 3), (), ()), ("RX", (3,), (32,), (1.1,)), ("LOCAL_SWAP", (32, 2), (), ()),
+           ("RY", (32,), (), (0.2,)), ("ESWAP", (32, 30), (), (0.6,)), ("X", (32,), (30, 31), ()),
+           ("EZ", (32, 7), (), (0.5,)), ("H", (20,), (), ()), ("X", (20,), (32,), ()), ("U1", (32,), (20,), (0.8,)),
+           ("EX", (32, 8), (), (0.4,)), ("Y", (32,), (), ()), ("H", (32,), (), ())]
+    c = brk.Circuit(n, ops)
+    a, b = DeviceState(n, brk.C64), DeviceState(n, brk.C64)
+    try:
+        for st in (a, b):
+            brk.fill_hash(st.ptr, st.size, brk.C64, 33, 2.0 ** -16)
+        final, _ = c.run_timed(a.ptr, brk.C64)
+        assert c.run(b.ptr, brk.C64) == final
+        brk.call("brk_stream_synchronize", None)
+        part = 1 << 30  # bytes a time
+        x, y = np.empty(part // 8, dtype=np.uint64), np.empty(part // 8, dtype=np.uint64)
+        for at in range(0, a.nbytes, part):
+            if at % (8 * part) == 0:
+                note(f"gpu blocks: n={n}, GiB {at // part} of {a.nbytes // part}")
+            brk.call("brk_memcpy_dtoh", x.ctypes.data, a.ptr + at, part, None)
+            brk.call("brk_memcpy_dtoh", y.ctypes.data, b.ptr + at, part, None)
+            assert np.array_equal(x, y), at
+    finally:
+        a.free()
+        b.free()

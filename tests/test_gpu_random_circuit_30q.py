@@ -142,3 +142,20 @@ def test_fused_c64_vs_oracle(reference, width):
     finally:
         src.free()
         st.free()
+
+
+def test_blocks_bit_identical_to_gate_by_gate(per_gate):
+    """brk_circuit_run and its gate blocks against one plain kernel per op (brk_circuit_run_timed)."""
+    blocks, perm = per_gate
+    st = DeviceState(N)
+    try:
+        brk.fill_hash(st.ptr, st.size, brk.C128, FILL_SEED, SCALE)
+        note("30q: gate by gate")
+        perm_g, _ = brk.Circuit(N, _ops()).run_timed(st.ptr)
+        assert perm_g == perm
+        for start in range(0, st.size, CHUNK):
+            a = _download_range(blocks, start, CHUNK)
+            b = _download_range(st, start, CHUNK)
+            assert np.array_equal(a.view(np.uint64), b.view(np.uint64)), start
+    finally:
+        st.free()
