@@ -159,7 +159,6 @@ struct chunk_ctx {
   const uint32_t* thi;
   uint32_t cbase;  // global index bits of the chunk
   uint32_t L;
-  cstage S;
 };
 
 __device__ __forceinline__ uint32_t global_index(const chunk_ctx& c, uint32_t j) {
@@ -354,7 +353,7 @@ __global__ __launch_bounds__(BATCH_THREADS, BATCH_WAVES_PER_SIMD) void k_batch(b
     const uint32_t csize = 1u << L;
     const uint32_t end_chunk = items[k].first_chunk + items[k].num_chunks;
     for (uint32_t cidx = items[k].first_chunk; cidx < end_chunk; ++cidx) {
-      const chunk_ctx c{chunk, tlo, thi, deposit(cidx, chunk_mask), L, S};
+      const chunk_ctx c{chunk, tlo, thi, deposit(cidx, chunk_mask), L};
       if (flags & BS_INIT) {
         for (uint32_t j = tid; j < csize; j += BATCH_THREADS)
           chunk[lpad(j)] = f2{global_index(c, j) == 0 ? 1.0f : 0.0f, 0.0f};

@@ -65,7 +65,7 @@ enum block_kind {
 // the bits of `inserted` (the pair bit and the cond bits), then the cond bits set.
 struct block_op {
   uint8_t kind, pair_bit;
-  uint8_t group_flip, group_pair;   // register segments: flip and pair bit over the group index
+  uint8_t group_flip, pad8;         // register segments: flip over the group index
   uint8_t group_zmask, group_cond;  // register segments: the masks' parts over the group index
                                     // (zmask, a pair gate's sign; cond),
   uint16_t coef;                    // first of its coefficients (none for H, SWAP, NEGATE)

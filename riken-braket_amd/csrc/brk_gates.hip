@@ -275,8 +275,8 @@ struct op_words {
   __device__ __forceinline__ uint32_t coef() const { return (uint32_t)(w[0] >> 48); }
 };
 struct block_gate {
-  uint32_t kind, pair_bit, group_flip, group_pair, group_zmask, group_cond;
-  uint32_t flip, cond, sign, zmask, inserted, thread_cond, thread_zmask;
+  uint32_t kind, pair_bit, group_flip, group_zmask, group_cond;
+  uint32_t flip, cond, sign, inserted, thread_cond, thread_zmask;
   uint64_t outer_cond, outer_zmask;
   double u[8];
 };
@@ -298,13 +298,11 @@ __device__ __forceinline__ block_gate decode(const op_words& r, const double (&u
   g.kind = byte(r.w[0], 0);
   g.pair_bit = byte(r.w[0], 1);
   g.group_flip = byte(r.w[0], 2);
-  g.group_pair = byte(r.w[0], 3);
   g.group_zmask = byte(r.w[0], 4);
   g.group_cond = byte(r.w[0], 5);
   g.flip = half(r.w[1], 0);
   g.cond = half(r.w[1], 1);
   g.sign = half(r.w[1], 2);
-  g.zmask = half(r.w[1], 3);
   g.inserted = half(r.w[2], 0);
   g.thread_cond = half(r.w[2], 1);
   g.thread_zmask = half(r.w[2], 2);
@@ -381,8 +379,7 @@ __device__ __forceinline__ void kind_math(const double (&u)[8], uint32_t sign, u
     y0 = cadd(cmul(m00, x0), cmul(m01, x1));
     y1 = cadd(cmul(m10, x0), cmul(m11, x1));
   } else {
-    constexpr int MODE = KIND == BLOCK_KIND_H ? MODE_H : KIND == BLOCK_KIND_SWAP ? MODE_SWAP
-                         : KIND == BLOCK_KIND_ESWAP ? MODE_ESWAP : MODE_MATRIX;
+    constexpr int MODE = KIND == BLOCK_KIND_H ? MODE_H : KIND == BLOCK_KIND_ESWAP ? MODE_ESWAP : MODE_MATRIX;
     pair_math<R, MODE>(u, sign, j0, x0, x1, y0, y1);
   }
 }
@@ -392,7 +389,6 @@ template <typename F>
 __device__ __forceinline__ void with_pair_kind(const block_gate& op, F f) {
   switch (op.kind != BLOCK_KIND_ESWAP && op.sign != 0 ? (uint32_t)BLOCK_KIND_SIGNED : op.kind) {
     case BLOCK_KIND_H: f(std::integral_constant<int, BLOCK_KIND_H>()); break;
-    case BLOCK_KIND_SWAP: f(std::integral_constant<int, BLOCK_KIND_SWAP>()); break;
     case BLOCK_KIND_ESWAP: f(std::integral_constant<int, BLOCK_KIND_ESWAP>()); break;
     case BLOCK_KIND_REAL: f(std::integral_constant<int, BLOCK_KIND_REAL>()); break;
     case BLOCK_KIND_X: f(std::integral_constant<int, BLOCK_KIND_X>()); break;
@@ -404,38 +400,24 @@ __device__ __forceinline__ void with_pair_kind(const block_gate& op, F f) {
 // LDS slot of local index j: an XOR swizzle, so that groups over low bits spread over all banks.
 __device__ __forceinline__ uint32_t block_slot(uint32_t j) { return j ^ ((j >> 3) & 7u) ^ ((j >> 6) & 7u); }
 
-// One gate over the whole chunk: a strided loop over exactly the local indices it changes.
+// One pair gate over the whole chunk (diagonal gates and moves are in segments): a strided loop over exactly
+// the local indices it changes.
 template <typename R, int PER>
-__device__ __forceinline__ void single_pass(cpx<R>* lds, const block_gate& op, uint64_t base, uint32_t t) {
+__device__ __forceinline__ void single_pass(cpx<R>* lds, const block_gate& op, uint32_t t) {
   constexpr uint32_t CAP = PER * BLOCK_THREADS;
   const uint32_t inserted = op.inserted, set = op.cond;
   const uint32_t items = CAP >> __popc(inserted);
-  if (op.kind == BLOCK_KIND_NEGATE) {  // the visited indices are exactly the cond subspace
+  const uint32_t flip = op.flip;
+  with_pair_kind(op, [&](auto kind) {
     for (uint32_t v = t; v < items; v += BLOCK_THREADS) {
-      const uint32_t j = block_slot(op_index(v, inserted, set));
-      lds[j] = cneg(lds[j]);
+      const uint32_t j0 = op_index(v, inserted, set), j1 = j0 ^ flip;
+      const cpx<R> x0 = lds[block_slot(j0)], x1 = lds[block_slot(j1)];
+      cpx<R> y0, y1;
+      kind_math<R, kind>(op.u, op.sign, j0, x0, x1, y0, y1);
+      lds[block_slot(j0)] = y0;
+      lds[block_slot(j1)] = y1;
     }
-  } else if (op.kind == BLOCK_KIND_DIAG) {
-    cpx<R> c0, c1;
-    chunk_diag(op, base, c0, c1);
-    const uint32_t zmask = op.zmask;
-    for (uint32_t v = t; v < items; v += BLOCK_THREADS) {
-      const uint32_t j = op_index(v, inserted, set);
-      lds[block_slot(j)] = cmul(lds[block_slot(j)], csel((__popc(j & zmask) & 1) != 0, c1, c0));
-    }
-  } else {
-    const uint32_t flip = op.flip;
-    with_pair_kind(op, [&](auto kind) {
-      for (uint32_t v = t; v < items; v += BLOCK_THREADS) {
-        const uint32_t j0 = op_index(v, inserted, set), j1 = j0 ^ flip;
-        const cpx<R> x0 = lds[block_slot(j0)], x1 = lds[block_slot(j1)];
-        cpx<R> y0, y1;
-        kind_math<R, kind>(op.u, op.sign, j0, x0, x1, y0, y1);
-        lds[block_slot(j0)] = y0;
-        lds[block_slot(j1)] = y1;
-      }
-    });
-  }
+  });
 }
 
 // A pair gate of a segment on pairs (m, m | F) whose group conditions hold.  A sign mask lies in
@@ -654,14 +636,14 @@ __global__ __launch_bounds__(BLOCK_THREADS, BLOCK_WAVES_PER_SIMD) void k_block(c
   op_words cur = load_op(v, 0);
   for (uint32_t pi = 0; pi < npasses; ++pi) {
     const cpass pass = v.passes + pi;
-    if (pass->kind == BLOCK_PASS_SINGLE) {
+    if (__builtin_expect(pass->kind == BLOCK_PASS_SINGLE, 0)) {  // (rare: its code out of the way, 1 % at 20 qubits)
       const op_words next = load_op(v, min(++o, last));
       double u[8];
       load_coefs(v, cur.coef(), u);
       const block_gate op = decode(cur, u);
       cur = next;
       if (!acts_on(op, chunk)) continue;
-      single_pass<R, PER>(lds, op, chunk, t);
+      single_pass<R, PER>(lds, op, t);
       __syncthreads();
       continue;
     }

@@ -125,7 +125,6 @@ static void make_passes(block_program& prog, unsigned line_bits) {
       for (unsigned g = 0; g < k; ++g) {
         const uint32_t bit = 1u << p.group[g];
         if (!diagonal && (o.flip & bit)) o.group_flip |= (uint8_t)(1u << g);
-        if (!diagonal && p.group[g] == o.pair_bit) o.group_pair = (uint8_t)(1u << g);
         if ((diagonal ? o.zmask : o.sign) & bit) o.group_zmask |= (uint8_t)(1u << g);
         if (o.cond & bit) o.group_cond |= (uint8_t)(1u << g);
       }
