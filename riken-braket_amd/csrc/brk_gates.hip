@@ -1762,8 +1762,7 @@ double plain_share(const gate_desc& d, int dtype) {
   const unsigned threshold = lane ? LANE_BITS : line_bits(dtype);
   // a SWAP's own condition counts where both its qubits are inserted
   const uint64_t tested = lane ? d.cond & ~d.flip : d.cond;
-  const int halvings = __builtin_popcountll(tested >> threshold);
-  return std::ldexp(1.0, -halvings);
+  return 1.0 / (double)(1ull << __builtin_popcountll(tested >> threshold));
 }
 
 }  // namespace brk

@@ -486,8 +486,10 @@ struct launch_builder {
     if (in_order && shape.fits(mixing | m) && room + block_op_room(d) <= BLOCK_ARG_ROOM) {
       mixing |= m;
       room += block_op_room(d);
-      plain_bytes += std::max(plain_share(d, dtype) * state_bytes + 6e6, 12e6);
-      if (!count || plain_is_faster()) ops.push_back(std::move(op));  // (it stays slower once it is)
+      if (plain_is_faster()) {  // (slower once, it stays so, and the op is not needed any more)
+        plain_bytes += std::max(plain_share(d, dtype) * state_bytes + 6e6, 12e6);
+        if (!count || plain_is_faster()) ops.push_back(std::move(op));
+      }
       descs[count++] = d;
       return count == (unsigned)BLOCK_MAX_OPS;
     }
