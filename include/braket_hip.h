@@ -584,11 +584,16 @@ int brk_batch_stage(const brk_batch* batch, unsigned circuit, unsigned stage, un
 int brk_batch_stage_op(const brk_batch* batch, unsigned circuit, unsigned stage, unsigned k, int* kind,
                        uint64_t* qubit_mask, double* matrix);
 /* Runs every circuit; energies[i] receives circuit i's energy (host array of
-   num_circuits).  Ordered after the work already on `stream`; returns when done. */
+   num_circuits).  Ordered after the work already on `stream`; returns when done.
+   The same batch gives the same bits every time; a circuit of several stages
+   may round its FP64 sum differently in another batch, whose size decides how
+   many partial sums it is made of. */
 int brk_batch_run(brk_batch* batch, double* energies, void* stream);
 /* Same, with the device time of the graph launch and, per circuit (may be
-   NULL), the wall-clock times in ms when a workgroup took it from the queue
-   and when its energy was written, both relative to the first take. */
+   NULL), the wall-clock times in ms when a workgroup took its first stage from
+   the queue and when its energy was written, both relative to the first take.
+   The circuits advance a stage at a time together, so between the two lies
+   also the other circuits' work on the stages that this one shares. */
 int brk_batch_run_timed(brk_batch* batch, double* energies, double* elapsed_ms, double* circuit_start_ms,
                         double* circuit_end_ms, void* stream);
 

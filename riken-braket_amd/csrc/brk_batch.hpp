@@ -30,7 +30,7 @@ constexpr int BATCH_THREADS = 512;      // two workgroups per CU overlap each ot
 constexpr int BATCH_WG_PER_CU = 2;
 constexpr int BATCH_MAX_LOCAL = 13;     // 2^13 complex64 = 64 KiB of LDS per chunk
 constexpr int BATCH_PASSENGERS = 4;     // qubits 0..3 are always local: chunk rows are 128-byte runs
-constexpr int BATCH_MAX_QUBITS = 24;    // per circuit (one 2^n slot per workgroup for multi-stage circuits)
+constexpr int BATCH_MAX_QUBITS = 24;    // per circuit (one of several stages has a slot of 2^n amplitudes)
 constexpr int BATCH_MAX_GROUP = 4;      // local positions per gate instruction (16 amplitudes per thread)
 constexpr int BATCH_MAX_GROUP_OPS = 8;  // 2x2 gates per gate instruction
 constexpr int BATCH_CHUNK = 1 << BATCH_MAX_LOCAL;

@@ -131,9 +131,10 @@ __device__ __forceinline__ uint64_t xcd_tile(uint32_t b, uint32_t nblocks, int r
 // The same for the chunks of the gate blocks and sweeps, whose accesses are runs of 128 bytes apart:
 // an XCD takes 32 consecutive chunks (one per CU), and the 8 XCDs 256, so what the chip reads at a
 // time lies in runs of 32 KiB where consecutive chunks are neighbours in memory.  With an eighth of
-// the chunks per XCD the runs were 4 KiB each, in 8 places.  29 qubits (complex128), 11 launches of
-// gate blocks: 55.5 ms so, 56.0 with the eighths (55.4, 56.4 and 57.4 with 8, 128 and 512 chunks in
-// a row); another circuit there 25.9 and 26.6 (26.3, 26.4, 26.6); gradient of 24 qubits 9.67 and 9.78.
+// the chunks per XCD the runs were 4 KiB each, in 8 places.  A small gain, against the eighths: 29
+// qubits (complex128), 11 launches of gate blocks 56.0 -> 55.5 ms, another circuit there 26.6 -> 25.9,
+// gradient of 24 qubits 9.78 -> 9.67.  How many chunks in a row hardly matters: with 8, 128 and 512 the
+// first took 55.4, 56.4 and 57.4, the second 26.3, 26.4 and 26.6; 32 is within 0.2 % of the best in both.
 // Few chunks, or a number that is no multiple of 256, keep the contiguous eighths.
 __device__ __forceinline__ uint64_t xcd_chunk(uint32_t b, uint32_t nblocks) {
   if (nblocks & 255u) return xcd_tile(b, nblocks, 1);

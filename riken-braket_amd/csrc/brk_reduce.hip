@@ -2,10 +2,10 @@
 // values, Pauli-string expectation values and the open-chain Ising energy,
 // plus H|psi> for that Hamiltonian.
 //
-// Every reduction runs on a fixed grid of RED_BLOCKS blocks, so the assignment
-// of amplitudes to threads, the in-block tree and the host-side sum over the
-// block partials (in block order) are the same on every call: results are
-// bit-reproducible.  The blocks write their partials straight to pinned host
+// A reduction runs on a grid that its state's size fixes -- RED_BLOCKS blocks, the
+// Ising energy up to ISING_GRID a pass -- so the assignment of amplitudes to
+// threads, the in-block tree and the host-side sum over the block partials (in
+// block order) are the same on every call: results are bit-reproducible.  The blocks write their partials straight to pinned host
 // memory (24 KB at most): a copy back costs about 10 us more per call.  Partial sums are kept in
 // double whatever the element type (the reference accumulates per-thread
 // partials and then std::accumulate's them, inner_product.hpp:43-55; spin

@@ -1,7 +1,7 @@
 // Differentiation form, host side: the adjoint method for
 // E(theta) = <psi(theta)| H |psi(theta)> with the open-chain Ising H.
 //
-//   forward:  psi = U_N ... U_1 |psi0>        (plain per-gate kernels)
+//   forward:  psi = U_N ... U_1 |psi0>
 //             lam = H psi, E = <psi|lam>
 //   reverse:  for i = N..1:  dE/dtheta_i = 2 Re <lam| D_i |psi>,
 //             psi := U_i^dagger psi, lam := U_i^dagger lam,
@@ -9,21 +9,23 @@
 //   RX/RY/RZ(theta) = exp(-i theta G / 2):  D = -(i/2) G
 //   EX/EY/EZ(phi)   = exp(i phi G):         D = i G
 //   U1(lambda)      = diag(1, e^{i lambda}):  D = diag(0, i)
-// Default (tuning adjoint_blocks = 1): the forward pass runs in gate blocks,
-// and the reverse sweep in blocks of ops whose qubits fit in a chunk of 2^11
-// (complex<double>) or 2^12 (complex<float>) amplitudes: psi and lambda chunks
-// stay in LDS while the block's inverse ops are un-applied and its gradient
-// terms summed (k_adjoint_block), one HBM round trip of both states per block.
-// Within a block, register segments take runs of ops on at most L - 9 qubits
-// (every thread holds a group of psi and lambda amplitudes) with one LDS round
-// trip; RX / RY / RZ-type ops use the general formulas with their zero terms
-// left out.  Per-chunk gradient terms are summed on the device in a fixed order.
-// Otherwise: runs of consecutive single-qubit ops on the same qubit are swept
-// by one fused kernel (csrc/brk_adjoint.hip); runs of Z / CZ ops (diagonal,
-// self-inverse, mutually commuting) are one sign pass per state; other ops
-// are un-applied to both states with the plain kernels.  That forward pass
-// merges the same runs: a single-qubit run becomes one 2x2 product (FP64 on
-// the host), a Z / CZ run one sign pass.
+// Three routes:
+//  * merged sweeps (csrc/brk_sweep.hpp), for circuits of uncontrolled one-qubit ops, Z and CZ on 12 to 32
+//    qubits: both directions in blocks that merge what commutes, launched as they are planned
+//    (host/sweep.cpp);
+//  * adjoint blocks, for other circuits whose ops fit in a block, from 11 qubits (complex<double>) or 12
+//    (complex<float>): the forward pass in gate blocks, the reverse sweep in blocks of ops whose qubits fit
+//    in a chunk of 2^11 or 2^12 amplitudes: psi and lambda chunks stay in LDS while the block's inverse ops
+//    are un-applied and its gradient terms summed (k_adjoint_block), one HBM round trip of both states per
+//    block.  Within a block, register segments take runs of ops on at most L - 9 qubits (every thread holds
+//    a group of psi and lambda amplitudes) with one LDS round trip; RX / RY / RZ-type ops use the general
+//    formulas with their zero terms left out.  Per-chunk gradient terms are summed on the device in a fixed
+//    order;
+//  * otherwise, and for every circuit with tuning adjoint_blocks = 0, run by run: consecutive single-qubit
+//    ops on the same qubit are swept by one fused kernel (csrc/brk_adjoint.hip); runs of Z / CZ ops
+//    (diagonal, self-inverse, mutually commuting) are one sign pass per state; other ops are un-applied to
+//    both states with the plain kernels.  Its forward pass merges the same runs: a single-qubit run becomes
+//    one 2x2 product (FP64 on the host), a Z / CZ run one sign pass.
 #include "circuit.hpp"
 #include "brk_adjoint.hpp"
 #include "brk_block.hpp"
