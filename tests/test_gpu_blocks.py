@@ -279,25 +279,15 @@ def test_large_state_gate_by_gate_bitwise(dtype):
     assert same_bits(got[0], got[1]) and same_bits(got[0], got[2])
 
 
-def hip_runtime():
-    """The HIP runtime that the engine loaded, for the calls that its C ABI does not wrap."""
-    with open("/proc/self/maps") as f:
-        paths = {line.split()[-1] for line in f if "libamdhip64.so" in line}
-    (path,) = paths
-    return C.CDLL(path)
-
-
 @pytest.mark.parametrize("n,dtype", [(12, brk.C128), (14, brk.C64), (23, brk.C128)])
 def test_captured_runs_replay(n, dtype):
     """A plan's run and a circuit's run captured in a graph: nothing of them lies in memory that a replay
     could find changed.  Several replays, each from a new state after other runs, bit for bit the plain
     kernels' result (23 qubits: launches and plain kernels)."""
     note(f"gpu blocks captured n={n} dtype={dtype}")
-    brk.load()
-    runtime = hip_runtime()
 
-    def call(name, *args):
-        assert getattr(runtime, name)(*args) == 0, name
+    def call(name, *args):  # the HIP runtime that the engine is linked against (its C ABI wraps no graphs)
+        assert getattr(brk.load(), name)(*args) == 0, name
 
     rng = np.random.default_rng(n)
     ops = random_ops(n, 80, 70 + n, max_controls=4, local_swaps=2)
