@@ -606,7 +606,8 @@ __device__ __forceinline__ uint32_t move_linear(uint32_t j, const block_gate& op
 // way while one runs: it is a scalar load of about 0.1 us, which a chunk that has its CU to itself
 // would otherwise wait for (20 qubits, where a move took 0.2 us: with the diagonal gates' paths in
 // segment_gate 338 -> 296 us, 12 qubits 175 -> 138).
-// Bound: the HBM round trip of the chunks (about 2.9 ms of a 29-qubit c128 state's 17.2 GB) plus what
+// Bound: the HBM round trip of the chunks (2.9 to 4.1 ms of a 29-qubit c128 state's 17.2 GB, by the
+// qubits that are local; four fifths of the launches' time) plus what
 // the two workgroups of a CU do not hide of it in instructions: 4.7 ms a launch of 21 gates on that
 // state, 0.22 a gate (0.28 with 64-bit indices and every move applied to every amplitude's index; 0.48
 // with every qubit local and an LDS round trip per pass).  Waves of

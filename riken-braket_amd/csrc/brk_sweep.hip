@@ -195,8 +195,8 @@ __device__ __forceinline__ void apply_diagonal(cpx<R> (&x)[GROUP], cpx<R> (&y)[G
 }
 
 // Bound: FP64 instructions (VALU 57 % busy in the reverse sweep, 66 % forward).  24 qubits, 12 layers
-// of RY, RZ and CZ, c128: 8 reverse blocks of 0.81 ms and 8 forward blocks of 0.34 ms, against 21 of
-// 0.60 ms and 17 of 0.40 ms gate by gate; 9.6 against 20.1 ms per gradient.  Fetching the next
+// of RY, RZ and CZ, c128: 8 reverse blocks of 0.80 ms and 8 forward blocks of 0.33 ms, against 21 of
+// 0.60 ms and 17 of 0.40 ms gate by gate; 9.5 against 20.1 ms per gradient.  Fetching the next
 // macro's lines ahead: 15 qubits 55 -> 38 us a reverse block (few chunks: latency), 24 qubits no change.
 // One workgroup of 2^(L - 3) threads per chunk.  Two workgroups per CU (64 KiB of LDS each, plus the
 // gradient sums).  The gradient terms of a segment's macros are summed over rows of 16 lanes in
