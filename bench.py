@@ -22,7 +22,7 @@ amplitudes (64 GiB) resident in HBM.  A step is one pass of the circuit.
                state, FP32 MFMA GEMMs; circuit time, speedup over the complex128
                per-gate path and infidelity 1 - |<psi_c128|psi_c64>|^2 (FP64)
   batch_c64  = the batching form: 4096 ansatz circuits of 10..20 qubits in one
-               captured graph, a launch per stage level; circuits/s, p50/p99 latency
+               graph, a launch per stage level; circuits/s, p50/p99 latency
   adjoint_c128 = the differentiation form: adjoint gradient of a 24-qubit,
                576-parameter ansatz; gradients/s, max error vs parameter shift over
                all 576 parameters and vs central differences on a sample
@@ -459,7 +459,7 @@ def plain_energy(n, ops, J, h, stream):
 
 def batch_leg(args, stream):
     """Batching form: 4096 hardware-efficient-ansatz circuits of 10..20 qubits (8 layers),
-    complex64 states, one captured graph per batch; FP64 energies."""
+    complex64 states, one graph per batch; FP64 energies."""
     import numpy as np
 
     import brk
@@ -469,7 +469,7 @@ def batch_leg(args, stream):
     t0 = time.perf_counter()
     batch = brk.Batch(items)
     plan_s = time.perf_counter() - t0
-    energies = batch.run(stream)  # first run uploads the program and captures the graph
+    energies = batch.run(stream)  # first run uploads the program and makes the graph
     runs = []
     for _ in range(max(1, args.steps)):
         e, ms, start, end = batch.run_timed(stream)

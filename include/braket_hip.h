@@ -543,7 +543,7 @@ int brk_adjoint_ising_gradient(const brk_circuit* circuit, void* psi, void* work
 
 /* ------------------------------------------------------------------------ */
 /* Batching form: many small independent circuits in one persistent launch  */
-/* per stage, captured as one HIP graph and replayed.  Each circuit runs on  */
+/* per stage, made one HIP graph and replayed.  Each circuit runs on         */
 /* its own complex64 state from |0...0> and yields its FP64 open-chain      */
 /* Ising energy sum_i J_i <Z_i Z_i+1> + sum_i h_i <X_i>.  Reference: bra's  */
 /* CIRCUITS mode, which advances several states in turn                     */
@@ -569,7 +569,7 @@ enum {
    single-qubit ops (consecutive ones on one qubit are multiplied into one
    2x2 matrix in FP64) and BRK_OP_Z on any qubits (Z, CZ, CnZ); anything else
    is BRK_ERR_UNSUPPORTED.  Planning needs no device; the first run uploads
-   the program to the current device and captures the graph. */
+   the program to the current device and makes the graph. */
 int brk_batch_create(const brk_circuit* const* circuits, unsigned num_circuits, const double* const* J,
                      const double* const* h, brk_batch** out);
 int brk_batch_destroy(brk_batch* batch);

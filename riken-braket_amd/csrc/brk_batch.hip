@@ -494,16 +494,31 @@ __global__ __launch_bounds__(256) void k_batch_reset(batch_launch P, uint32_t* c
 
 }  // namespace
 
-int launch_batch_reset(const batch_launch& L, uint32_t* counters, uint32_t num_counters, void* stream) {
-  const uint32_t items = std::max(num_counters, L.num_circuits);
-  hipLaunchKernelGGL(k_batch_reset, dim3((items + 255) / 256), dim3(256), 0, as_stream(stream), L, counters,
-                     num_counters);
-  return check_launch("batch reset");
+static int add_kernel(void* graph, void** last, const void* kernel, unsigned grid, unsigned block, void** args) {
+  hipKernelNodeParams p{};
+  p.func = const_cast<void*>(kernel);
+  p.gridDim = dim3(grid);
+  p.blockDim = dim3(block);
+  p.kernelParams = args;
+  hipGraphNode_t node = nullptr;
+  auto* before = reinterpret_cast<hipGraphNode_t*>(last);
+  const hipError_t e = hipGraphAddKernelNode(&node, static_cast<hipGraph_t>(graph), before, *before ? 1 : 0, &p);
+  if (e != hipSuccess) return fail(BRK_ERR_HIP, "adding a batch launch failed: %s", hipGetErrorString(e));
+  *before = node;
+  return BRK_OK;
 }
 
-int launch_batch(const batch_launch& L, unsigned grid, void* stream) {
-  hipLaunchKernelGGL(k_batch, dim3(grid), dim3(BATCH_THREADS), 0, as_stream(stream), L);
-  return check_launch("batch");
+int add_batch_reset(void* graph, void** last, const batch_launch& L, uint32_t* counters, uint32_t num_counters) {
+  const uint32_t items = std::max(num_counters, L.num_circuits);
+  batch_launch launch = L;
+  void* args[] = {&launch, &counters, &num_counters};
+  return add_kernel(graph, last, (const void*)k_batch_reset, (items + 255) / 256, 256, args);
+}
+
+int add_batch(void* graph, void** last, const batch_launch& L, unsigned grid) {
+  batch_launch launch = L;
+  void* args[] = {&launch};
+  return add_kernel(graph, last, (const void*)k_batch, grid, BATCH_THREADS, args);
 }
 
 }  // namespace brk

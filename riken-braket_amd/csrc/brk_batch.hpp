@@ -125,9 +125,10 @@ struct batch_launch {
   uint64_t* t_end;         // ... and when its energy was written
 };
 
-// Enqueues the reset of `num_counters` queue heads and of every circuit's remaining partials, then
-// (launch_batch) one persistent launch over L.items, on `stream` (capturable: no memset nodes).
-int launch_batch_reset(const batch_launch& L, uint32_t* counters, uint32_t num_counters, void* stream);
-int launch_batch(const batch_launch& L, unsigned grid, void* stream);
+// Add a kernel to a graph (hipGraph_t), after the node `last` (hipGraphNode_t; null: none), which it then is:
+// the reset of `num_counters` queue heads and of every circuit's remaining partials, and (add_batch) one
+// persistent launch over L.items.
+int add_batch_reset(void* graph, void** last, const batch_launch& L, uint32_t* counters, uint32_t num_counters);
+int add_batch(void* graph, void** last, const batch_launch& L, unsigned grid);
 
 }  // namespace brk

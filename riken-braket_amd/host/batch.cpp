@@ -1,6 +1,6 @@
 // Batching form, host side: compiles a list of small circuits into the stage
 // programs of csrc/brk_batch.hpp, uploads them once, and runs the persistent
-// kernel as a captured HIP graph (a reset, then one launch per stage level).
+// kernel as a HIP graph made once (a reset, then one launch per stage level).
 //
 // Per circuit:
 //  1. ops -> planner ops: uncontrolled single-qubit ops become 2x2 gates
@@ -593,23 +593,22 @@ int ensure_device(brk_batch* b) {
   if (hipEventCreateWithFlags(&b->ev_in, hipEventDisableTiming) != hipSuccess ||
       hipEventCreate(&b->ev_begin) != hipSuccess || hipEventCreate(&b->ev_end) != hipSuccess)
     return brk::fail(BRK_ERR_HIP, "cannot create the batch events");
-  // graph: the reset and the launches, captured once and replayed
-  if (hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal) != hipSuccess)
-    return brk::fail(BRK_ERR_HIP, "hipStreamBeginCapture failed");
-  int launch_status = brk::launch_batch_reset(L, counters, (uint32_t)plan.launches.size(), b->stream);
+  // graph: the reset and the launches, made once and replayed.  Its nodes are added one by one: while one
+  // thread captured a stream, another's calls on the legacy stream (its own batch's upload) failed.
+  hipGraph_t graph = nullptr;
+  if (hipGraphCreate(&graph, 0) != hipSuccess) return brk::fail(BRK_ERR_HIP, "hipGraphCreate failed");
+  void* last = nullptr;
+  int launch_status = brk::add_batch_reset(graph, &last, L, counters, (uint32_t)plan.launches.size());
   for (size_t k = 0; !launch_status && k < plan.launches.size(); ++k) {
     L.items = items + plan.launches[k].first;
     L.num_items = (uint32_t)plan.launches[k].count;
     L.counter = counters + k;
-    launch_status = brk::launch_batch(L, std::min<unsigned>(workgroups, L.num_items), b->stream);
+    launch_status = brk::add_batch(graph, &last, L, std::min<unsigned>(workgroups, L.num_items));
   }
-  hipGraph_t graph = nullptr;
-  const hipError_t end = hipStreamEndCapture(b->stream, &graph);
   if (launch_status) {
-    if (graph) (void)hipGraphDestroy(graph);
+    (void)hipGraphDestroy(graph);
     return launch_status;
   }
-  if (end != hipSuccess || !graph) return brk::fail(BRK_ERR_HIP, "hipStreamEndCapture failed");
   const hipError_t inst = hipGraphInstantiate(&b->exec, graph, nullptr, nullptr, 0);
   (void)hipGraphDestroy(graph);
   if (inst != hipSuccess) {

@@ -2,12 +2,14 @@
 batch kernel (complex64 states, FP64 energies) against the FP64 plain per-gate
 path and the CPU oracle; determinism and graph replays."""
 import sys
+import threading
 
 import numpy as np
 import pytest
 
 import brk
 import circuits as W
+import hip
 from devstate import DeviceState
 from oracle_circuits import run_ops
 
@@ -181,3 +183,32 @@ def test_full_workload_sampled():
     for i in sorted(rng.choice(len(items), 24, replace=False)):
         n, ops, J, h = items[i]
         assert abs(e[i] - plain_energy(n, ops, J, h)) < E_TOL, (i, n)
+
+
+def test_new_batches_on_several_threads():
+    """Six threads make and run batches of their own at the same time, each on its own stream: no call fails, and
+    every energy has the bits that it has when the batches run one after the other."""
+    note("gpu batch: new batches on six threads")
+    alone, together = {}, {}
+
+    def work(t, out):
+        stream = hip.create_stream()
+        out[t] = []
+        for r in range(25):
+            items = W.batch_ansatz(num_circuits=4, min_qubits=5, max_qubits=15, layers=2, seed=100 * t + r)
+            try:
+                out[t].append(brk.Batch(items).run(stream))
+            except brk.BrkError as e:
+                out[t].append(str(e))
+
+    for t in range(6):
+        work(t, alone)
+    threads = [threading.Thread(target=work, args=(t, together)) for t in range(6)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    failed = [x for runs in together.values() for x in runs if isinstance(x, str)]
+    assert not failed, failed
+    for t in range(6):
+        assert all(np.array_equal(x, y) for x, y in zip(alone[t], together[t]))
