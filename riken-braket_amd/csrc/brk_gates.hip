@@ -427,30 +427,12 @@ __device__ __forceinline__ void segment_pairs(cpx<R> (&x)[PER], const block_gate
   if constexpr (F < PER) {
     const uint32_t cond = op.group_cond, sign = op.group_zmask;
     auto apply = [&](auto kind) {
-      // a pair's two results; ESWAP: pair_math's two forms, which pairs take which is uniform (it selects
-      // per amplitude)
-      auto pair = [&](int m, const double (&u)[8], cpx<R>& y0, cpx<R>& y1) {
-        if constexpr (kind == BLOCK_KIND_ESWAP) {
-          const cpx<R> e = {(R)u[0], (R)u[1]}, x0 = x[m], x1 = x[m | F];
-          const R c = (R)u[2], sn = (R)u[3];
-          if ((m & sign) != 0) {
-            y0 = {x0.re * c - x1.im * sn, x0.im * c + x1.re * sn};
-            y1 = {x1.re * c - x0.im * sn, x1.im * c + x0.re * sn};
-          } else {
-            y0 = cmul(x0, e);
-            y1 = cmul(x1, e);
-          }
-        } else {
-          kind_math<R, kind>(u, 0, 0, x[m], x[m | F], y0, y1);
-        }
-      };
-      // the common case: no selects (24 ESWAP in a row, 25 qubits complex128, took 1030 us with them, now 946)
-      if ((cond | op.thread_cond | (kind == BLOCK_KIND_ESWAP ? 0u : sign)) == 0) {
+      if ((cond | sign | op.thread_cond) == 0) {  // the common case: no branches, no selects
 #pragma unroll
         for (int m = 0; m < PER; ++m) {
           if ((m & F) != 0) continue;
           cpx<R> y0, y1;
-          pair(m, op.u, y0, y1);
+          kind_math<R, kind>(op.u, 0, 0, x[m], x[m | F], y0, y1);
           x[m] = y0;
           x[m | F] = y1;
         }
@@ -467,16 +449,45 @@ __device__ __forceinline__ void segment_pairs(cpx<R> (&x)[PER], const block_gate
           if ((__popc(m & sign) & 1) != 0)
             for (int k = 2; k < 6; ++k) u[k] = -u[k];
         }
-        pair(m, u, y0, y1);
+        kind_math<R, kind>(u, 0, 0, x[m], x[m | F], y0, y1);
         x[m] = csel(on, y0, x[m]);
         x[m | F] = csel(on, y1, x[m | F]);
+      }
+    };
+    // ESWAP: pair_math's two forms, which pairs take which is uniform (it selects per amplitude); without
+    // conditions no selects: 24 in a row, 25 qubits complex128, 1030 -> 990 us.  (In two loops 946, but other
+    // gates' code then ran up to 0.8 % slower; as a function of its own 887 and 1.5 %, at 128 registers.)
+    auto eswap = [&]() {
+      const cpx<R> e = {(R)op.u[0], (R)op.u[1]};
+      const R c = (R)op.u[2], sn = (R)op.u[3];
+      const bool everywhere = (cond | op.thread_cond) == 0;
+#pragma unroll
+      for (int m = 0; m < PER; ++m) {
+        if ((m & F) != 0) continue;
+        if ((m & cond) != cond) continue;  // uniform
+        const cpx<R> x0 = x[m], x1 = x[m | F];
+        cpx<R> y0, y1;
+        if ((m & sign) != 0) {
+          y0 = {x0.re * c - x1.im * sn, x0.im * c + x1.re * sn};
+          y1 = {x1.re * c - x0.im * sn, x1.im * c + x0.re * sn};
+        } else {
+          y0 = cmul(x0, e);
+          y1 = cmul(x1, e);
+        }
+        if (everywhere) {
+          x[m] = y0;
+          x[m | F] = y1;
+        } else {
+          x[m] = csel(on, y0, x0);
+          x[m | F] = csel(on, y1, x1);
+        }
       }
     };
     switch (op.kind) {  // (X, CNOT and SWAP are moves)
       case BLOCK_KIND_H: apply(std::integral_constant<int, BLOCK_KIND_H>()); break;
       case BLOCK_KIND_REAL: apply(std::integral_constant<int, BLOCK_KIND_REAL>()); break;
       case BLOCK_KIND_X: apply(std::integral_constant<int, BLOCK_KIND_X>()); break;
-      case BLOCK_KIND_ESWAP: apply(std::integral_constant<int, BLOCK_KIND_ESWAP>()); break;
+      case BLOCK_KIND_ESWAP: eswap(); break;
       default: apply(std::integral_constant<int, BLOCK_KIND_MATRIX>()); break;
     }
   }
